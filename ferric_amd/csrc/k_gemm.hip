@@ -44,9 +44,6 @@ __device__ __forceinline__ bf16x8 as_b8(u32x4 v) { return __builtin_bit_cast(bf1
 
 constexpr int kRowNormThreads = 256;  // the residual + RMSNorm kernel's thread count and mapping
 
-// Batches of more than 32 rows run as 32-row chunks (gridDim.z of them, one
-// split): every chunk streams the same weight tiles.
-//
 // NS >= 0 (one row): the row's residual + RMSNorm runs in the prologue of
 // every workgroup (RowNormArgs; NS split-K slabs folded, NJ 16-byte chunks
 // per thread), with the norm kernel's thread mapping and reduction order
@@ -59,7 +56,7 @@ constexpr int kRowNormThreads = 256;  // the residual + RMSNorm kernel's thread 
 // zero: they only produce the discarded output rows).
 template <int NT, int MT, int EPI, int WAVES, int UNROLL, int NS = -1, int NJ = 1>
 __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const uint16_t* __restrict__ xt,
-                                                         const uint16_t* __restrict__ w, uint32_t m_total,
+                                                         const uint16_t* __restrict__ w, uint32_t m,
                                                          uint32_t kb_count, uint32_t kb_split, uint32_t x_mtiles,
                                                          const uint16_t* residual, void* out, uint32_t ldo,
                                                          uint32_t* err, RowNormArgs na) {
@@ -68,26 +65,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const uint16_t* __rest
   static_assert(!kNorm || WAVES * 64 >= kRowNormThreads, "the norm's 256-thread mapping");
   __shared__ float red[WAVES][NT * MT * 256];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // A launch over several 32-row chunks (always one split) reads each weight
-  // slice once per chunk. Workgroups go to the 8 XCDs round-robin by
-  // dispatch order, so the order is arranged for the chunks of one slice to
-  // be dispatched back to back on one XCD: they run together there and the
-  // later ones find the weight tiles in that XCD's L2. Slices past the last
-  // multiple of 8 keep their chunks consecutive in dispatch order.
-  uint32_t slice = blockIdx.x, chunk = blockIdx.z;
-  if (gridDim.z > 1) {
-    const uint32_t S = gridDim.x, C = gridDim.z, S8 = S & ~7u;
-    const uint32_t b = blockIdx.x + S * blockIdx.z;
-    if (b < S8 * C) {
-      const uint32_t r = b >> 3;
-      chunk = r % C;
-      slice = (r / C) * 8 + (b & 7u);
-    } else {
-      const uint32_t t = b - S8 * C;
-      slice = S8 + t / C;
-      chunk = t % C;
-    }
-  }
+  const uint32_t slice = blockIdx.x;
   const uint32_t tile0 = slice * NT;
   const uint32_t split = blockIdx.y;
   const uint32_t s_lo = split * kb_split;
@@ -100,10 +78,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const uint16_t* __rest
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
     wp[nt] = reinterpret_cast<const u32x4*>(w) + ((uint64_t)(tile0 + nt) * kb_count + kb_lo) * 64 + lane;
-  const uint32_t row0 = chunk * 16 * MT;
-  const uint32_t m = min(m_total - row0, 16u * MT);
   const uint64_t xkb = (uint64_t)x_mtiles * 64;  // 16-byte units per k-block of the activation
-  const u32x4* xp = reinterpret_cast<const u32x4*>(xt) + (uint64_t)kb_lo * xkb + chunk * MT * 64 + lane;
+  const u32x4* xp = reinterpret_cast<const u32x4*>(xt) + (uint64_t)kb_lo * xkb + lane;
 
   f32x4 acc[NT][MT];
 #pragma unroll
@@ -334,7 +310,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const uint16_t* __rest
       if (row < m) {
         const uint32_t col = (tile0 / 2 + pair) * 16 + i;
         const uint32_t y = swiglu_bf16(round_bf16(g), round_bf16(u), bad);
-        reinterpret_cast<uint16_t*>(out)[act_offset_m(row0 + row, col, act_mtiles(m_total))] = (uint16_t)y;
+        reinterpret_cast<uint16_t*>(out)[act_offset(row, col)] = (uint16_t)y;
       }
     }
     if (bad) raise_error(err, ERR_NONFINITE);
@@ -348,7 +324,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(const uint16_t* __rest
       for (int wv = 1; wv < WAVES; ++wv) v += red[wv][idx];
       if (row >= m) continue;
       const uint64_t n = (uint64_t)(tile0 + nt) * 16 + i;
-      const uint64_t o = (uint64_t)(row0 + row) * ldo + n;
+      const uint64_t o = (uint64_t)row * ldo + n;
       if constexpr (EPI == FH_EPI_PARTIAL) {
         reinterpret_cast<float*>(out)[(uint64_t)split * kMaxRows * ldo + o] = v;
       } else if constexpr (EPI == FH_EPI_BF16) {
@@ -379,43 +355,12 @@ void launch_variant(const uint16_t* xt, const uint16_t* w, uint32_t m, uint32_t 
                        x_mtiles, residual, out, ldo, err, RowNormArgs{});
 }
 
-// 32 < m <= 256 (a speculative verify, a small prefill chunk): one split, the
-// rows in chunks of 64 (MT = 4, unroll 2) or 32 (MT = 2, unroll 4). The
-// 64-row chunk halves how often each weight tile is fetched; with 8 waves its
-// wave-partial buffer is 128 KiB of LDS (one workgroup per CU), so it is
-// taken there only when the launch fits in one round of the 256 CUs.
-// Measured at 160 rows (8B shapes, cold weights, us per launch):
-//   QKV 6144 x 4096    NT 4, 8 waves: 32-row 29.9, 64-row 38.1 (288 workgroups)
-//   O 4096 x 4096      NT 4, 8 waves: 32-row 28.3, 64-row 20.2
-//   down 4096 x 12288  NT 4, 8 waves: 32-row 78.5, 64-row 55.5
-//   gate/up 24576      64-row: NT 4 with 4 waves 94.2, NT 2 112.6 (32-row NT 2: 128.4)
-//   LM head 151936     NT 4, 4 waves: 32-row 788, 64-row 618
-// Also slower on every shape: unroll 1, 2-wave workgroups, 128-row chunks
-// (gate/up 96 against 106-147, down 56 against 58-95).
-template <int NT, int EPI, int WAVES>
-void launch_wide(const uint16_t* xt, const uint16_t* w, uint32_t m, uint32_t n, uint32_t k, const uint16_t* residual,
-                 void* out, uint32_t ldo, uint32_t* err, hipStream_t s) {
-  const uint32_t kb = k / 32;
-  const uint32_t x_mtiles = act_mtiles(m);
-  const uint32_t slices = n / (16 * NT);
-  if (WAVES == 8 && slices * ((m + 63) / 64) > 256) {
-    dim3 grid(slices, 1, (m + 31) / 32);
-    hipLaunchKernelGGL((gemm_kernel<NT, 2, EPI, WAVES, 4>), grid, dim3(WAVES * 64), 0, s, xt, w, m, kb, kb, x_mtiles,
-                       residual, out, ldo, err, RowNormArgs{});
-  } else {
-    dim3 grid(slices, 1, (m + 63) / 64);
-    hipLaunchKernelGGL((gemm_kernel<NT, 4, EPI, WAVES, 2>), grid, dim3(WAVES * 64), 0, s, xt, w, m, kb, kb, x_mtiles,
-                       residual, out, ldo, err, RowNormArgs{});
-  }
-}
-
 // 32 < m <= 256 rows, n % 128 == 0 (a speculative verify; the epilogues a
 // wide batch's projections use): the activation panel of each k-block is
 // staged in LDS once per workgroup and shared by its 4 waves; each wave
-// streams its own 2 weight tiles per k-block into a register ring. The
-// launches above read the activations once per 64 weight rows from L2 and
-// the weights once per row chunk; here each workgroup reads the activations
-// once per 128 weight rows and each weight tile once. Split-K across
+// streams its own 2 weight tiles per k-block into a register ring: each
+// workgroup reads the activations once per 128 weight rows and each weight
+// tile once. Split-K across
 // workgroups (FH_EPI_PARTIAL) fills the CUs for the narrow projections; the
 // consumer adds the slabs in split order.
 //
@@ -434,7 +379,7 @@ void launch_wide(const uint16_t* xt, const uint16_t* w, uint32_t m, uint32_t n, 
 // one k-block assumed complete once all later ones were) the fast panel
 // loads overtook the weight stream and MFMAs read weight registers and
 // panel tiles before they arrived. Measured at 160 rows, cold weights, us
-// per launch (against the 64/32-row launches above): gate/up 24576 x 4096
+// per launch (against the weight stream over 64/32-row chunks): gate/up 24576 x 4096
 // 55 (95), down 4096 x 12288 in 8 splits 28 (56), O 4096 x 4096 in 8 splits
 // 14 (20), QKV 6144 x 4096 in 5 splits 18 (30), LM head 151936 x 4096 306
 // (617). Weight rings of 4 and 8 k-blocks (gate/up 65, 56), 2 or 8 waves, 4
@@ -681,19 +626,6 @@ void launch_epi(const uint16_t* xt, const uint16_t* w, uint32_t m, uint32_t n, u
       return;
     }
   }
-  if constexpr (EPI != FH_EPI_PARTIAL) {
-    if (m > kMaxRows) {
-      if (n % 64 == 0 && n < 16384 && EPI != FH_EPI_SWIGLU)
-        launch_wide<4, EPI, 8>(xt, w, m, n, k, residual, out, ldo, err, s);
-      else if (n % 64 == 0)
-        launch_wide<4, EPI, 4>(xt, w, m, n, k, residual, out, ldo, err, s);
-      else if (n % 32 == 0)
-        launch_wide<2, EPI, 4>(xt, w, m, n, k, residual, out, ldo, err, s);
-      else if constexpr (EPI != FH_EPI_SWIGLU)
-        launch_wide<1, EPI, 4>(xt, w, m, n, k, residual, out, ldo, err, s);
-      return;
-    }
-  }
   const SmallVariant v = small_variant(EPI, m, n, k, splits);
 #define FH_VARIANT(NT_, WAVES_) launch_variant<NT_, EPI, WAVES_, 4>(xt, w, m, n, k, splits, residual, out, ldo, err, s)
   if (v.nt == 4) {
@@ -822,7 +754,9 @@ hipError_t launch_gemm(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_
                        uint32_t epilogue, uint32_t splits, const uint16_t* residual, void* out, uint32_t ldo,
                        uint32_t* err, hipStream_t s) {
   if (splits == 0) return hipErrorInvalidValue;
-  if (m > kMaxRows && (epilogue == FH_EPI_PARTIAL ? !gemm_partial_rows_ok(m, n) : splits != 1))
+  // Beyond kMaxRows rows only the panel kernel's epilogues and shapes run here.
+  if (m > kMaxRows && (m > kPanelRows || n % kPanelCols != 0 || epilogue == FH_EPI_BF16 || epilogue == FH_EPI_RESIDUAL ||
+                       (epilogue != FH_EPI_PARTIAL && splits != 1)))
     return hipErrorInvalidValue;
   switch (epilogue) {
     case FH_EPI_BF16: launch_epi<FH_EPI_BF16>(x_tiled, w_tiled, m, n, k, 1, residual, out, ldo, err, s); break;

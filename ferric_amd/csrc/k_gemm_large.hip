@@ -1,17 +1,14 @@
-// K1 projections for prefill and wide verify batches (m > 32 token rows):
-// bf16 MFMA (v_mfma_f32_16x16x32_bf16), FP32 accumulation, compute-bound.
+// K1 projections of prefill chunks (m > 256 token rows) whose 256 x 256
+// blocks fill the CUs, and the choice between this kernel and the ones with
+// smaller blocks (k_gemm_band.hip, k_gemm_mid.hip): bf16 MFMA
+// (v_mfma_f32_16x16x32_bf16), FP32 accumulation, compute-bound.
 //
 // Operands come from their tile orders (common.hpp): the weight in weight
 // tile order and the activation in activation tile order with act_mtiles(m)
 // row tiles, so every operand fetch of a wave is one contiguous 1 KiB in the
-// exact MFMA register layout. Two kernels:
-//  * gemm_large_xd_kernel (n % 256 == 0: every projection): 256 x 256
-//    blocks of 8 waves sharing each k-block's weight tiles through LDS,
-//    activation tiles loaded by each wave;
-//  * gemm_large_kernel (the LM head's 151936 rows): 128 x 128 blocks of 4
-//    waves loading operands straight into registers (each tile fetched by
-//    two waves; the second fetch hits the CU's cache).
-// Each wave accumulates its MFMA tiles over the whole k range.
+// exact MFMA register layout. A workgroup has 8 waves sharing each k-block's
+// weight tiles through LDS; activation tiles are loaded by each wave. Each
+// wave accumulates its MFMA tiles over the whole k range.
 //
 // Epilogues (same rounding points as the decode kernel, no split-K here):
 //   FH_EPI_BF16     out[m][n] = bf16(acc)
@@ -31,114 +28,8 @@ namespace {
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr uint32_t kStreamedRows = 256;
-constexpr int kNT = 4;  // n-tiles per wave
-constexpr int kMT = 4;  // m-tiles per wave
-constexpr int kBlockTiles = 2 * kNT;  // 16-row tiles per block side (128 rows)
-static_assert(kLargeBlockRows % (16 * 2 * kMT) == 0, "padded rows cover whole blocks");
 
 __device__ __forceinline__ bf16x8 b8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
-
-template <int EPI>
-__global__ __launch_bounds__(256) void gemm_large_kernel(const uint16_t* __restrict__ xt,
-                                                         const uint16_t* __restrict__ w, uint32_t m,
-                                                         uint32_t mtiles, uint32_t kb_count,
-                                                         const uint16_t* residual, void* out, uint32_t ldo,
-                                                         uint32_t out_mtiles, uint32_t* err) {
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t nt0 = blockIdx.x * kBlockTiles + (wave & 1) * kNT;  // first 16-row weight tile
-  const uint32_t mt0 = blockIdx.y * kBlockTiles + (wave >> 1) * kMT;  // first 16-row activation tile
-  if (mt0 * 16 >= m) return;  // this wave's rows are all padding
-
-  // Per k-block: weight tile (nb, kb) at (nb * kb_count + kb) KiB; activation
-  // tile (kb, mt) at (kb * mtiles + mt) KiB. Pointers are in 16-byte units.
-  const u32x4* wp = reinterpret_cast<const u32x4*>(w) + (uint64_t)nt0 * kb_count * 64 + lane;
-  const u32x4* xp = reinterpret_cast<const u32x4*>(xt) + (uint64_t)mt0 * 64 + lane;
-  const uint64_t w_tile_stride = (uint64_t)kb_count * 64;  // next n-tile
-  const uint64_t x_kb_stride = (uint64_t)mtiles * 64;      // next k-block
-
-  f32x4 acc[kNT][kMT];
-#pragma unroll
-  for (int i = 0; i < kNT; ++i)
-#pragma unroll
-    for (int j = 0; j < kMT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  u32x4 wa[kNT], xa[kMT], wb[kNT], xb[kMT];
-  auto load = [&](u32x4(&wv)[kNT], u32x4(&xv)[kMT], uint32_t kb) {
-#pragma unroll
-    for (int i = 0; i < kNT; ++i) wv[i] = wp[i * w_tile_stride + kb * 64];
-#pragma unroll
-    for (int j = 0; j < kMT; ++j) xv[j] = xp[kb * x_kb_stride + j * 64];
-  };
-  auto compute = [&](const u32x4(&wv)[kNT], const u32x4(&xv)[kMT]) {
-#pragma unroll
-    for (int i = 0; i < kNT; ++i)
-#pragma unroll
-      for (int j = 0; j < kMT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b8(wv[i]), b8(xv[j]), acc[i][j], 0, 0, 0);
-  };
-  load(wa, xa, 0);
-  for (uint32_t kb = 0; kb < kb_count; kb += 2) {
-    if (kb + 1 < kb_count) load(wb, xb, kb + 1);
-    __builtin_amdgcn_sched_barrier(0);
-    compute(wa, xa);
-    __builtin_amdgcn_sched_barrier(0);
-    if (kb + 1 < kb_count) {
-      if (kb + 2 < kb_count) load(wa, xa, kb + 2);
-      __builtin_amdgcn_sched_barrier(0);
-      compute(wb, xb);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-
-  // D layout: lane l, element e holds weight row n = 16 nt + 4 (l / 16) + e
-  // and activation row m = 16 mt + l % 16.
-  const uint32_t q = lane >> 4, c = lane & 15;
-  if constexpr (EPI == FH_EPI_SWIGLU) {
-    static_assert(kNT % 2 == 0, "gate/up tile pairs");
-    bool bad = false;
-#pragma unroll
-    for (int p = 0; p < kNT / 2; ++p) {
-      const uint32_t col = ((nt0 + 2 * p) / 2) * 16 + 4 * q;  // first of 4 output columns
-#pragma unroll
-      for (int j = 0; j < kMT; ++j) {
-        const uint32_t row = (mt0 + j) * 16 + c;
-        if (row >= m) continue;
-        uint32_t y[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          y[e] = swiglu_bf16(round_bf16(acc[2 * p][j][e]), round_bf16(acc[2 * p + 1][j][e]), bad);
-        uint2 v = make_uint2(y[0] | (y[1] << 16), y[2] | (y[3] << 16));
-        *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(out) + act_offset_m(row, col, out_mtiles)) = v;
-      }
-    }
-    if (bad) raise_error(err, ERR_NONFINITE);
-  } else {
-#pragma unroll
-    for (int i = 0; i < kNT; ++i) {
-      const uint32_t n = (nt0 + i) * 16 + 4 * q;
-#pragma unroll
-      for (int j = 0; j < kMT; ++j) {
-        const uint32_t row = (mt0 + j) * 16 + c;
-        if (row >= m) continue;
-        const uint64_t o = (uint64_t)row * ldo + n;
-        if constexpr (EPI == FH_EPI_F32) {
-          *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(out) + o) = acc[i][j];
-        } else if constexpr (EPI == FH_EPI_BF16) {
-          uint2 v = make_uint2(f32_to_bf16(acc[i][j][0]) | (f32_to_bf16(acc[i][j][1]) << 16),
-                               f32_to_bf16(acc[i][j][2]) | (f32_to_bf16(acc[i][j][3]) << 16));
-          *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(out) + o) = v;
-        } else {
-          const uint2 rv = *reinterpret_cast<const uint2*>(residual + o);
-          const float r0 = lo_bf16(rv.x), r1 = hi_bf16(rv.x), r2 = lo_bf16(rv.y), r3 = hi_bf16(rv.y);
-          uint2 v = make_uint2(f32_to_bf16((0.0f + acc[i][j][0]) + r0) | (f32_to_bf16((0.0f + acc[i][j][1]) + r1) << 16),
-                               f32_to_bf16((0.0f + acc[i][j][2]) + r2) | (f32_to_bf16((0.0f + acc[i][j][3]) + r3) << 16));
-          *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(out) + o) = v;
-        }
-      }
-    }
-  }
-}
 
 constexpr int kBigTiles = 16;  // 16-row tiles per block side (256 rows)
 
@@ -372,14 +263,39 @@ __global__ __launch_bounds__(512) void gemm_large_xd_kernel(const uint16_t* __re
   }
 }
 
+// Estimated microseconds of a launch of 256 x 256 blocks (fitted with
+// mid_cost, k_gemm_mid.hip): whole rounds of the 256 CUs, a k-block taking
+// longer the more CUs run, and what a block costs around its k loop.
+float block_cost(uint32_t m, uint32_t n, uint32_t k) {
+  const uint32_t blocks = n / (16 * kBigTiles) * ((m + 255) / 256);
+  const float kb_us = blocks < 100 ? 0.57f : blocks < 256 ? 0.66f : 0.73f;
+  return ((blocks + 255) / 256) * (12.5f + (k / 32) * kb_us);
+}
+
+// Which of the three kernels a projection of m rows runs.
+enum class LargeKernel { kMid, kBand, kBlock };
+
+LargeKernel pick_kernel(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, bool whole_heads) {
+  const float mid = gemm_mid_cost(m, n, k, whole_heads), band = gemm_band_cost(m, n, k, epilogue);
+  const bool block_ok = m > kPanelRows && n % (16 * kBigTiles) == 0;
+  const float block = block_ok ? block_cost(m, n, k) : -1.f;
+  if (block_ok && block <= mid && (band < 0.f || block <= band)) return LargeKernel::kBlock;
+  return band >= 0.f && band < mid ? LargeKernel::kBand : LargeKernel::kMid;
+}
+
 }  // namespace
 
 hipError_t launch_gemm_qkv_rope(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_t m, uint32_t n, uint32_t k,
                                 const QkvRopeArgs& qa, hipStream_t s) {
   const uint32_t mtiles = act_mtiles(m);
-  if (m <= kStreamedRows || n % (16 * kBigTiles) != 0 || k % 32 != 0 || mtiles % kBigTiles != 0 ||
+  if (m <= kPanelRows || n % (16 * kBigTiles) != 0 || k % 32 != 0 || mtiles % kBigTiles != 0 ||
       n != (qa.qh + 2 * qa.kvh) * 128)
     return hipErrorInvalidValue;
+  switch (pick_kernel(m, n, k, FH_EPI_BF16, true)) {
+    case LargeKernel::kMid: return launch_gemm_mid_qkv_rope(x_tiled, w_tiled, m, n, k, qa, s);
+    case LargeKernel::kBand: return launch_gemm_band_qkv_rope(x_tiled, w_tiled, m, n, k, qa, s);
+    case LargeKernel::kBlock: break;
+  }
   const dim3 grid(n / (16 * kBigTiles), mtiles / kBigTiles);
   hipLaunchKernelGGL((gemm_large_xd_kernel<kEpiQkvRope>), grid, dim3(512), 0, s, x_tiled, w_tiled, m, mtiles, k / 32,
                      (const uint16_t*)nullptr, (void*)nullptr, 0u, 0u, qa, (uint32_t*)nullptr);
@@ -389,50 +305,32 @@ hipError_t launch_gemm_qkv_rope(const uint16_t* x_tiled, const uint16_t* w_tiled
 hipError_t launch_gemm_large(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_t m, uint32_t n, uint32_t k,
                              uint32_t epilogue, const uint16_t* residual, void* out, uint32_t ldo, uint32_t* err,
                              hipStream_t s) {
-  // Up to kStreamedRows rows the weight-streaming kernel is faster: it runs
-  // 32-row chunks of the batch against the same weight tiles (a prefill
-  // chunk of 17..32 rows when row_capacity < 32, a speculative verify batch).
-  if (m <= kStreamedRows) return launch_gemm(x_tiled, w_tiled, m, n, k, epilogue, 1, residual, out, ldo, err, s);
-  if (n % (16 * kBlockTiles) != 0 || k % 32 != 0) return hipErrorInvalidValue;
-  const uint32_t mtiles = act_mtiles(m);
-  const uint32_t out_mtiles = epilogue == FH_EPI_SWIGLU ? act_mtiles(m) : 0u;
-  const uint32_t kb = k / 32;
-  if (n % (16 * kBigTiles) == 0 && mtiles % kBigTiles == 0) {
-    const dim3 grid(n / (16 * kBigTiles), mtiles / kBigTiles);
+  if (m <= kMaxRows) return launch_gemm(x_tiled, w_tiled, m, n, k, epilogue, 1, residual, out, ldo, err, s);
+  if (n % kPanelCols != 0 || k % 32 != 0) return hipErrorInvalidValue;
+  // Up to kPanelRows rows the SwiGLU and FP32 epilogues have the panel kernel.
+  if (m <= kPanelRows && (epilogue == FH_EPI_SWIGLU || epilogue == FH_EPI_F32))
+    return launch_gemm(x_tiled, w_tiled, m, n, k, epilogue, 1, residual, out, ldo, err, s);
+  switch (pick_kernel(m, n, k, epilogue, false)) {
+    case LargeKernel::kMid:
+      return launch_gemm_mid(x_tiled, w_tiled, m, n, k, epilogue, residual, out, ldo, err, s);
+    case LargeKernel::kBand:
+      return launch_gemm_band(x_tiled, w_tiled, m, n, k, epilogue, residual, out, ldo, err, s);
+    case LargeKernel::kBlock: break;
+  }
+  const uint32_t mtiles = act_mtiles(m), kb = k / 32;
+  const uint32_t out_mtiles = epilogue == FH_EPI_SWIGLU ? mtiles : 0u;
+  const dim3 grid(n / (16 * kBigTiles), mtiles / kBigTiles);
 #define FH_BIG(E)                                                                                           \
   hipLaunchKernelGGL((gemm_large_xd_kernel<E>), grid, dim3(512), 0, s, x_tiled, w_tiled, m, mtiles, kb, residual, \
                      out, ldo, out_mtiles, QkvRopeArgs{}, err)
-    switch (epilogue) {
-      case FH_EPI_BF16: FH_BIG(FH_EPI_BF16); break;
-      case FH_EPI_RESIDUAL: FH_BIG(FH_EPI_RESIDUAL); break;
-      case FH_EPI_SWIGLU: FH_BIG(FH_EPI_SWIGLU); break;
-      case FH_EPI_F32: FH_BIG(FH_EPI_F32); break;
-      default: return hipErrorInvalidValue;
-    }
-#undef FH_BIG
-    return hipGetLastError();
-  }
-  const dim3 grid(n / (16 * kBlockTiles), mtiles / kBlockTiles);
   switch (epilogue) {
-    case FH_EPI_BF16:
-      hipLaunchKernelGGL(gemm_large_kernel<FH_EPI_BF16>, grid, dim3(256), 0, s, x_tiled, w_tiled, m, mtiles, kb,
-                         residual, out, ldo, out_mtiles, err);
-      break;
-    case FH_EPI_RESIDUAL:
-      hipLaunchKernelGGL(gemm_large_kernel<FH_EPI_RESIDUAL>, grid, dim3(256), 0, s, x_tiled, w_tiled, m, mtiles, kb,
-                         residual, out, ldo, out_mtiles, err);
-      break;
-    case FH_EPI_SWIGLU:
-      hipLaunchKernelGGL(gemm_large_kernel<FH_EPI_SWIGLU>, grid, dim3(256), 0, s, x_tiled, w_tiled, m, mtiles, kb,
-                         residual, out, ldo, out_mtiles, err);
-      break;
-    case FH_EPI_F32:
-      hipLaunchKernelGGL(gemm_large_kernel<FH_EPI_F32>, grid, dim3(256), 0, s, x_tiled, w_tiled, m, mtiles, kb,
-                         residual, out, ldo, out_mtiles, err);
-      break;
-    default:
-      return hipErrorInvalidValue;
+    case FH_EPI_BF16: FH_BIG(FH_EPI_BF16); break;
+    case FH_EPI_RESIDUAL: FH_BIG(FH_EPI_RESIDUAL); break;
+    case FH_EPI_SWIGLU: FH_BIG(FH_EPI_SWIGLU); break;
+    case FH_EPI_F32: FH_BIG(FH_EPI_F32); break;
+    default: return hipErrorInvalidValue;
   }
+#undef FH_BIG
   return hipGetLastError();
 }
 

@@ -1,0 +1,379 @@
+// K1 projections of mid-sized batches (a prompt of some hundred rows, or a
+// narrow weight): too few 256 x 256 blocks for the 256 CUs, too many rows to
+// stream the weight once per row chunk. bf16 MFMA
+// (v_mfma_f32_32x32x16_bf16), FP32 accumulation.
+//
+// A workgroup owns a block of 32 TN weight rows x 32 TM activation rows and
+// its waves split k: wave w takes k-blocks w, w + WAVES, ... and accumulates
+// the whole block over them, so the k loop has no LDS traffic and no
+// barrier; every operand goes from its tile order (common.hpp) straight into
+// registers, D half-k-block stages deep. At the end the waves' partial blocks
+// are added in wave order through LDS, 32 activation rows at a time, where
+// the epilogue also gets its row-contiguous stores. The sum over k is a
+// reassociation of the serial order, as in the other projection kernels,
+// fixed by the launch shape.
+//
+// What bounds it: the operands, read from L2 (64 (TN + TM) KiB per k-block of
+// 32 and workgroup / 32): about 14.6 TB/s over all CUs on every block shape,
+// with and without the MFMAs and at 3 to 7 stages in flight, so the largest
+// block that still fills the CUs is the fastest (launch_gemm_mid picks it).
+// Measured against the 256 x 256-block kernel (us per launch, cold weights):
+//   777 rows: O 4096 x 4096 87 -> 39, down 4096 x 12288 225 -> 98, QKV 6144 x 4096 88 -> 63
+//   509 rows: O 1024 x 2048 47 -> 7.2, down 1024 x 3072 64 -> 9.5, gate/up 6144 x 1024 35 -> 12
+//   300 rows: O 4096 x 4096 85 -> 25
+//   48 rows: down 4096 x 12288 55 (the weight-streaming kernel over row chunks) -> 32
+//
+// A 32x32x16 operand (lane l: row l % 32, columns 8 (l / 32) .. + 7) is half
+// a k-block of two adjacent 16-row tiles: in-tile lanes l % 16 + 16 (l / 32)
+// (+ 32 for the second half) of tile (l / 16) % 2, so a load is four
+// contiguous 256-byte runs.
+#include <cmath>
+#include <type_traits>
+
+#include "common.hpp"
+#include "kernels.hpp"
+#include "../../include/ferric_hip.h"
+
+namespace fh {
+
+namespace {
+
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+__device__ __forceinline__ bf16x8 b8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
+
+// Calls f(std::integral_constant<int, I>) for I = B .. E - 1, unrolled at compile time.
+template <int B, int E, class F>
+__device__ __forceinline__ void mid_for(F&& f) {
+  if constexpr (B < E) {
+    f(std::integral_constant<int, B>{});
+    mid_for<B + 1, E>(f);
+  }
+}
+
+// The QKV projection with QK-norm, RoPE and the KV append in its epilogue
+// (TN = 4: a workgroup's columns are one head).
+constexpr int kMidEpiQkvRope = 16;
+constexpr int kMidQkPitch = 68;  // words per staged head row: 64 + 4 keeps rows 16-byte aligned, reads conflict-free
+
+template <int TN, int TM, int WAVES, int D, int OCC, int EPI>
+__global__ __launch_bounds__(WAVES * 64, OCC) void gemm_mid_kernel(const uint16_t* __restrict__ xt,
+                                                                   const uint16_t* __restrict__ w, uint32_t m,
+                                                                   uint32_t mtiles, uint32_t kb_count,
+                                                                   const uint16_t* residual, void* out, uint32_t ldo,
+                                                                   const QkvRopeArgs qa, uint32_t* err) {
+  constexpr int kN = 32 * TN, kPitch = kN + 4, kThreads = WAVES * 64;
+  constexpr size_t kRedBytes = sizeof(float) * WAVES * 32 * kPitch;
+  constexpr size_t kStageBytes = EPI == kMidEpiQkvRope ? 4ull * 32 * TM * kMidQkPitch : 0;
+  static_assert(EPI != kMidEpiQkvRope || (TN == 4 && 32 * TM <= kThreads), "one head per workgroup, a lane per row");
+  static_assert(kRedBytes >= kStageBytes, "the staged head rows reuse the reduction's LDS");
+  __shared__ __attribute__((aligned(16))) unsigned char lds_raw[kRedBytes];
+  auto& red = *reinterpret_cast<float(*)[WAVES][32][kPitch]>(lds_raw);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // Block order by XCD (workgroups go to the 8 XCDs round-robin): XCD j takes
+  // n-blocks j, j + 8, ... and walks all m-blocks of each, so a weight tile
+  // is fetched into one XCD's L2 only. N-blocks past the last multiple of 8
+  // keep their m-blocks consecutive in dispatch order.
+  const uint32_t NB = gridDim.x, MB = gridDim.y, N8 = NB & ~7u, b = blockIdx.x + NB * blockIdx.y;
+  uint32_t gx, gy;
+  if (b < N8 * MB) {
+    const uint32_t r = b >> 3;
+    gy = r % MB;
+    gx = (r / MB) * 8 + (b & 7u);
+  } else {
+    const uint32_t t = b - N8 * MB;
+    gx = N8 + t / MB;
+    gy = t % MB;
+  }
+  // The fused QKV epilogue's row lookups (position, page, slot) are requested
+  // now and used after the k loop.
+  QkvRowSlot row_slot{0u, 0u, false};
+  if constexpr (EPI == kMidEpiQkvRope) {
+    const uint32_t row = gy * 32 * TM + threadIdx.x;
+    if (threadIdx.x < 32 * TM && row < m) row_slot = qkv_row_slot(row, qa);
+  }
+  const uint32_t kb_n = kb_count > (uint32_t)wave ? (kb_count - wave + WAVES - 1) / WAVES : 0u;  // k-blocks of this wave
+  f32x16 acc[TN][TM];
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+
+  if (kb_n > 0) {
+    // Buffer descriptors: the block's weight rows from k-block `wave` on
+    // (32-bit offsets: k < 2^24), and one k-block of its activation rows.
+    const uint64_t w0 = ((uint64_t)gx * 2 * TN * kb_count + wave) * 512, x0 = ((uint64_t)wave * mtiles + gy * 2 * TM) * 512;
+    auto wrs = __builtin_amdgcn_make_buffer_rsrc((void*)(w + w0), 0, (2u * TN * kb_count - wave) * 1024u, 0x00020000);
+    const uint32_t in_tile = (lane & 15) + 16 * (lane >> 5), second = (lane >> 4) & 1;
+    const uint32_t wofs = (second * kb_count * 64 + in_tile) * 16, xofs = (second * 64 + in_tile) * 16;
+    const uint32_t wpair = kb_count * 2048u;
+    // Stage: the operands of half a k-block.
+    u32x4 wr[D][TN], xr[D][TM];
+    const uint32_t halves = 2 * kb_n;
+    auto load = [&](auto slot_c, uint32_t hk) {
+      constexpr int S = decltype(slot_c)::value;
+      const uint32_t q = min(hk, halves - 1), kk = (q >> 1) * WAVES, half = (q & 1u) * 512;
+      const uint32_t ws = kk * 1024 + half;
+      auto xrs = __builtin_amdgcn_make_buffer_rsrc((void*)(xt + x0 + (uint64_t)kk * mtiles * 512), 0, 2 * TM * 1024u, 0x00020000);
+#pragma unroll
+      for (int i = 0; i < TN; ++i)
+        wr[S][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrs, wofs, ws + i * wpair, 0));
+#pragma unroll
+      for (int j = 0; j < TM; ++j)
+        xr[S][j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xrs, xofs, half + j * 2048, 0));
+    };
+    auto compute = [&](auto slot_c) {
+      constexpr int S = decltype(slot_c)::value;
+#pragma unroll
+      for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b8(wr[S][i]), b8(xr[S][j]), acc[i][j], 0, 0, 0);
+    };
+    mid_for<0, D - 1>([&](auto s) { load(s, decltype(s)::value); });
+    uint32_t hk = 0;
+    for (; hk + D <= halves; hk += D)
+      mid_for<0, D>([&](auto s) {
+        constexpr int S = decltype(s)::value;
+        load(std::integral_constant<int, (S + D - 1) % D>{}, hk + S + D - 1);
+        __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the MFMAs
+        compute(s);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    mid_for<0, D - 1>([&](auto s) {
+      if (hk + decltype(s)::value < halves) compute(s);
+    });
+  }
+
+  // D layout: lane l, element e holds weight row 8 (e / 4) + 4 (l / 32) + e % 4
+  // and activation row l % 32 of the 32 x 32 block.
+  const uint32_t hi = lane >> 5, c = lane & 31;
+  const uint32_t n0 = gx * kN;
+  constexpr int kSteps = (32 * kN / 4 + kThreads - 1) / kThreads;
+  bool bad = false;
+  // The residual is requested before the reduction (out may alias it, so the
+  // compiler cannot move a load over a store: one by one they would cost a
+  // memory round trip each).
+  constexpr bool kRes = EPI == FH_EPI_RESIDUAL;
+  uint2 rv[kRes ? TM : 1][kRes ? kSteps : 1];
+  if constexpr (kRes) {
+#pragma unroll
+    for (int j = 0; j < TM; ++j)
+#pragma unroll
+      for (int s = 0; s < kSteps; ++s) {
+        const int idx = min((int)threadIdx.x + s * kThreads, 32 * kN / 4 - 1);
+        const uint32_t row = min((gy * TM + j) * 32 + idx / (kN / 4), m - 1);
+        rv[j][s] = *reinterpret_cast<const uint2*>(residual + (uint64_t)row * ldo + n0 + idx % (kN / 4) * 4);
+      }
+  }
+  uint2 packed[EPI == kMidEpiQkvRope ? TM : 1][EPI == kMidEpiQkvRope ? kSteps : 1];
+  mid_for<0, TM>([&](auto j_c) {
+    constexpr int j = decltype(j_c)::value;
+    if constexpr (j > 0) __syncthreads();
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        *reinterpret_cast<f32x4*>(&red[wave][c][32 * i + 8 * e + 4 * hi]) =
+            f32x4{acc[i][j][4 * e], acc[i][j][4 * e + 1], acc[i][j][4 * e + 2], acc[i][j][4 * e + 3]};
+    __syncthreads();
+    // Four consecutive columns of one row, the waves' partials in wave order.
+    auto sum4 = [&](int r, int col) {
+      f32x4 v = *reinterpret_cast<const f32x4*>(&red[0][r][col]);
+#pragma unroll
+      for (int q = 1; q < WAVES; ++q) {
+        const f32x4 p = *reinterpret_cast<const f32x4*>(&red[q][r][col]);
+        v = f32x4{v[0] + p[0], v[1] + p[1], v[2] + p[2], v[3] + p[3]};
+      }
+      return v;
+    };
+    const uint32_t row0 = (gy * TM + j) * 32;
+    if constexpr (EPI == FH_EPI_SWIGLU) {
+      // Column group i holds a gate tile (16 columns) and its up tile. Threads
+      // walk the output in tile order: 4-column half, row, 8-column group, row tile.
+      for (int idx = threadIdx.x; idx < 32 * kN / 8; idx += kThreads) {
+        const int half = idx & 1, r = (idx >> 1) & 15, g = (idx >> 5) % (2 * TN), mt = (idx >> 5) / (2 * TN);
+        const uint32_t row = row0 + 16 * mt + r;
+        if (row >= m) continue;
+        const int col = 32 * (g >> 1) + 8 * (g & 1) + 4 * half;
+        const f32x4 gate = sum4(16 * mt + r, col), up = sum4(16 * mt + r, col + 16);
+        uint32_t y[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = swiglu_bf16(round_bf16(gate[e]), round_bf16(up[e]), bad);
+        *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(out) + act_offset_m(row, n0 / 2 + 8 * g + 4 * half, mtiles)) =
+            make_uint2(y[0] | (y[1] << 16), y[2] | (y[3] << 16));
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < kSteps; ++s) {
+        const int idx = threadIdx.x + s * kThreads;
+        if (32 * kN / 4 % kThreads != 0 && idx >= 32 * kN / 4) break;
+        const int r = idx / (kN / 4), col = idx % (kN / 4) * 4;
+        const uint32_t row = row0 + r;
+        const f32x4 v = sum4(r, col);
+        if constexpr (EPI == kMidEpiQkvRope) {
+          packed[j][s] = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+        } else if (row < m) {
+          const uint64_t o = (uint64_t)row * ldo + n0 + col;
+          if constexpr (EPI == FH_EPI_F32) {
+            *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(out) + o) = v;
+          } else if constexpr (EPI == FH_EPI_BF16) {
+            *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(out) + o) =
+                make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+          } else {
+            const uint2 r0 = rv[j][s];
+            *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(out) + o) =
+                make_uint2(pack_bf16x2((0.0f + v[0]) + lo_bf16(r0.x), (0.0f + v[1]) + hi_bf16(r0.x)),
+                           pack_bf16x2((0.0f + v[2]) + lo_bf16(r0.y), (0.0f + v[3]) + hi_bf16(r0.y)));
+          }
+        }
+      }
+    }
+  });
+  if constexpr (EPI == FH_EPI_SWIGLU) {
+    if (bad) raise_error(err, ERR_NONFINITE);
+  }
+  if constexpr (EPI == kMidEpiQkvRope) {
+    // The head's rows staged as bf16 (the projection's rounding), then one
+    // lane per row runs the lane-per-head kernel's code (qk_head.hpp).
+    uint32_t* rows_lds = reinterpret_cast<uint32_t*>(lds_raw);
+    __syncthreads();  // every wave is done reading the reduction's LDS
+    mid_for<0, TM>([&](auto j_c) {
+      constexpr int j = decltype(j_c)::value;
+#pragma unroll
+      for (int s = 0; s < kSteps; ++s) {
+        const int idx = threadIdx.x + s * kThreads;
+        *reinterpret_cast<uint2*>(rows_lds + (32 * j + idx / (kN / 4)) * kMidQkPitch + idx % (kN / 4) * 2) = packed[j][s];
+      }
+    });
+    __syncthreads();
+    const uint32_t row = gy * 32 * TM + threadIdx.x;
+    if (threadIdx.x < 32 * TM && row < m)
+      qknorm_rope_kv_head<TM >= 4 ? 32 : 8, true>(reinterpret_cast<const qk_u32x4*>(rows_lds + threadIdx.x * kMidQkPitch), row, gx, qa,
+                                    row_slot);
+  }
+}
+
+// Block shapes: 32 tn weight rows x 32 tm activation rows, and what
+// mid_cost needs of each: the operand GB/s of a CU running such blocks alone,
+// and microseconds per launch and per 256 blocks around the k loop (prologue,
+// reduction, epilogue).
+struct MidShape {
+  uint32_t tn, tm;
+  float cu_gbs, launch_us, round_us;
+};
+constexpr MidShape kMidShapes[] = {{4, 4, 66.f, 0.8f, 7.9f}, {4, 2, 73.f, 2.3f, 0.6f}, {2, 4, 83.f, 2.5f, 1.3f},
+                                   {2, 2, 75.f, 1.3f, 0.f},  {1, 2, 80.f, 2.5f, 0.1f}, {1, 1, 64.f, 3.4f, 0.f}};
+
+// Estimated microseconds of one launch: the operand bytes of all blocks at
+// 18.4 TB/s, but no less than those of the blocks one CU runs at its own
+// rate, plus the shape's overheads. Its constants and those of the other two
+// kernels' estimates (gemm_band_cost, block_cost) are fitted together to the
+// times of every shape at 40 row counts from 33 to 8192 of the Qwen3
+// projections (296 points): the estimate picks a kernel and block within 9 %
+// of the fastest one at every point, 0.6 % on average, and never one more
+// than 5 % slower than the 256 x 256 blocks alone, which are 1.67 times
+// slower on average.
+float mid_cost(const MidShape& s, uint32_t m, uint32_t n, uint32_t k) {
+  const float blocks = (float)(n / (32 * s.tn)) * ((m + 32 * s.tm - 1) / (32 * s.tm));
+  const float block_kb = 2.048f * (s.tn + s.tm) * (k / 32);  // operand kilobytes of a block
+  const float all = blocks * block_kb / 18400.f;
+  const float cu = ceilf(blocks / 256.f) * block_kb / s.cu_gbs;
+  return s.launch_us + blocks / 256.f * s.round_us + fmaxf(all, cu);
+}
+
+bool mid_pick(uint32_t m, uint32_t n, uint32_t k, bool whole_heads, MidShape* pick, float* cost) {
+  bool found = false;
+  for (const MidShape& s : kMidShapes) {
+    if (n % (32 * s.tn) != 0 || (whole_heads && s.tn != 4)) continue;
+    const float c = mid_cost(s, m, n, k);
+    if (!found || c < *cost) {
+      *pick = s;
+      *cost = c;
+      found = true;
+    }
+  }
+  return found;
+}
+
+template <int TN, int TM, int WAVES, int D, int OCC, int EPI>
+void launch_mid_variant(const uint16_t* xt, const uint16_t* w, uint32_t m, uint32_t n, uint32_t k,
+                        const uint16_t* residual, void* out, uint32_t ldo, const QkvRopeArgs& qa, uint32_t* err,
+                        hipStream_t s) {
+  hipLaunchKernelGGL((gemm_mid_kernel<TN, TM, WAVES, D, OCC, EPI>), dim3(n / (32 * TN), (m + 32 * TM - 1) / (32 * TM)),
+                     dim3(WAVES * 64), 0, s, xt, w, m, act_mtiles(m), k / 32, residual, out, ldo, qa, err);
+}
+
+// Waves per workgroup, stages and workgroups per CU of each shape: 4 waves
+// while the accumulators (16 TN TM registers) leave no room for more, 8 for
+// the small blocks, whose waves would else have too little in flight.
+template <int EPI>
+hipError_t launch_mid_shape(MidShape v, const uint16_t* xt, const uint16_t* w, uint32_t m, uint32_t n, uint32_t k,
+                            const uint16_t* residual, void* out, uint32_t ldo, const QkvRopeArgs& qa, uint32_t* err,
+                            hipStream_t s) {
+#define FH_MID(TN_, TM_, WAVES_, D_, OCC_) \
+  launch_mid_variant<TN_, TM_, WAVES_, D_, OCC_, EPI>(xt, w, m, n, k, residual, out, ldo, qa, err, s)
+  if (v.tn == 4 && v.tm == 4) {
+    FH_MID(4, 4, 4, 4, 1);
+  } else if (v.tn == 4) {
+    FH_MID(4, 2, 4, 4, 2);
+  } else if constexpr (EPI != kMidEpiQkvRope) {
+    if (v.tn == 2 && v.tm == 4)
+      FH_MID(2, 4, 4, 4, 2);
+    else if (v.tn == 2)
+      FH_MID(2, 2, 4, 6, 2);
+    else if (v.tm == 2)
+      FH_MID(1, 2, 8, 6, 2);
+    else
+      FH_MID(1, 1, 8, 12, 2);
+  } else {
+    return hipErrorInvalidValue;
+  }
+#undef FH_MID
+  return hipGetLastError();
+}
+
+}  // namespace
+
+float gemm_mid_cost(uint32_t m, uint32_t n, uint32_t k, bool whole_heads) {
+  MidShape v{};
+  float cost = 0.f;
+  return m > kMaxRows && n % 32 == 0 && k % 32 == 0 && k > 0 &&
+                 mid_pick(m, n, k, whole_heads, &v, &cost)
+             ? cost
+             : -1.f;
+}
+
+hipError_t launch_gemm_mid(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_t m, uint32_t n, uint32_t k,
+                           uint32_t epilogue, const uint16_t* residual, void* out, uint32_t ldo, uint32_t* err,
+                           hipStream_t s) {
+  MidShape v{};
+  float cost = 0.f;
+  if (m <= kMaxRows || n % 32 != 0 || k % 32 != 0 || k == 0 || !mid_pick(m, n, k, false, &v, &cost))
+    return hipErrorInvalidValue;
+  const QkvRopeArgs none{};
+#define FH_MID_EPI(E) \
+  case E: return launch_mid_shape<E>(v, x_tiled, w_tiled, m, n, k, residual, out, ldo, none, err, s)
+  switch (epilogue) {
+    FH_MID_EPI(FH_EPI_BF16);
+    FH_MID_EPI(FH_EPI_RESIDUAL);
+    FH_MID_EPI(FH_EPI_SWIGLU);
+    FH_MID_EPI(FH_EPI_F32);
+    default: return hipErrorInvalidValue;
+  }
+#undef FH_MID_EPI
+}
+
+hipError_t launch_gemm_mid_qkv_rope(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_t m, uint32_t n,
+                                    uint32_t k, const QkvRopeArgs& qa, hipStream_t s) {
+  MidShape v{};
+  float cost = 0.f;
+  if (m <= kMaxRows || n != (qa.qh + 2 * qa.kvh) * 128 || k % 32 != 0 || k == 0 || !mid_pick(m, n, k, true, &v, &cost))
+    return hipErrorInvalidValue;
+  return launch_mid_shape<kMidEpiQkvRope>(v, x_tiled, w_tiled, m, n, k, nullptr, nullptr, 0u, qa, nullptr, s);
+}
+
+}  // namespace fh

@@ -123,11 +123,26 @@ hipError_t launch_swiglu(const uint16_t* gate, const uint16_t* up, uint16_t* out
 hipError_t launch_gemm_large(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_t m, uint32_t n, uint32_t k,
                              uint32_t epilogue, const uint16_t* residual, void* out, uint32_t ldo, uint32_t* err,
                              hipStream_t s);
+// Mid-sized batches (k_gemm_mid.hip): m > kMaxRows, n % 32 == 0, the same
+// operands as launch_gemm_large. gemm_mid_cost estimates the launch's
+// microseconds (whole_heads: the QKV form), negative where it has no form.
+float gemm_mid_cost(uint32_t m, uint32_t n, uint32_t k, bool whole_heads);
+hipError_t launch_gemm_mid(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_t m, uint32_t n, uint32_t k,
+                           uint32_t epilogue, const uint16_t* residual, void* out, uint32_t ldo, uint32_t* err,
+                           hipStream_t s);
+hipError_t launch_gemm_mid_qkv_rope(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_t m, uint32_t n,
+                                    uint32_t k, const QkvRopeArgs& qa, hipStream_t s);
+// Chunks of 256-row x 128-column blocks (k_gemm_band.hip): n % 128 == 0.
+float gemm_band_cost(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue);
+hipError_t launch_gemm_band(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_t m, uint32_t n, uint32_t k,
+                            uint32_t epilogue, const uint16_t* residual, void* out, uint32_t ldo, uint32_t* err,
+                            hipStream_t s);
+hipError_t launch_gemm_band_qkv_rope(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_t m, uint32_t n,
+                                     uint32_t k, const QkvRopeArgs& qa, hipStream_t s);
 // The QKV projection of a prefill chunk with QK-norm, RoPE and the KV
 // append fused into its epilogue (qk_head.hpp), q written row-major to
-// qa.q_out. Only for the 256 x 256-block kernel: returns
-// hipErrorInvalidValue when m <= 256 or n % 256 != 0 (run the projection and
-// launch_qknorm_rope_kv instead).
+// qa.q_out. Returns hipErrorInvalidValue when m <= 256 or n % 256 != 0 (run
+// the projection and launch_qknorm_rope_kv instead).
 hipError_t launch_gemm_qkv_rope(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_t m, uint32_t n, uint32_t k,
                                 const QkvRopeArgs& qa, hipStream_t s);
 hipError_t launch_gemm(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_t m, uint32_t n, uint32_t k,

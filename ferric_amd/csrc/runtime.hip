@@ -1050,7 +1050,7 @@ hipError_t enqueue_prefill(fh_ctx* ctx, uint32_t R, uint32_t nout, uint32_t nblo
     q.run(cls, f);
     ++n;
   };
-  // The fused QKV epilogue needs the 256 x 256-block projection kernel.
+  // Beyond kPanelRows rows the projection kernels have the fused QKV epilogue.
   const bool fused_qkv = R > 256 && ctx->nqkv % 256 == 0 && fh::act_mtiles(R) % 16 == 0;
   // Chunks of up to kPanelRows rows (a speculative verify) write split-K
   // partials for QKV, O and down: the QK-norm, the post-attention norm and
@@ -1163,8 +1163,8 @@ hipError_t enqueue_prefill(fh_ctx* ctx, uint32_t R, uint32_t nout, uint32_t nblo
 // the decode path's op order (batched.rs:1746-2454). Up to 256 rows (a
 // speculative verify) the projections are the panel GEMM with split-K
 // partials folded by the norms, as in a decode step; beyond that the
-// compute-bound 256 x 256-block kernel with the residual (and, for QKV, the
-// QK-norm, RoPE and KV append) in its epilogues. Attention runs over blocks
+// compute-bound kernels with the residual (and, for QKV, the QK-norm, RoPE
+// and KV append) in their epilogues. Attention runs over blocks
 // of consecutive rows of one sequence (each K/V page read once per block),
 // and the final norm + FP32 head + argmax over the requested output rows
 // only.

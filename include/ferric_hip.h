@@ -235,9 +235,9 @@ fh_status fh_op_rmsnorm(const uint16_t* x, const uint16_t* weight, uint16_t* y, 
  * FH_EPI_F32 (FP32 out, the LM head). m <= 32 streams the weight (decode, split-K allowed);
  * m > 32 needs n % 128 == 0 and ldo % 4 == 0: up to 256 rows FH_EPI_PARTIAL, FH_EPI_SWIGLU
  * and FH_EPI_F32 run the panel kernel (activation panel shared through LDS; split-K allowed
- * for FH_EPI_PARTIAL), the other epilogues the weight-streaming kernel over row chunks
- * (splits = 1); beyond 256 rows the compute-bound prefill kernel (256 x 256 blocks through
- * LDS when n % 256 == 0, else 128 x 128 blocks; splits = 1, no FH_EPI_PARTIAL). Replaces
+ * for FH_EPI_PARTIAL); the other epilogues and batches beyond 256 rows (splits = 1, no
+ * FH_EPI_PARTIAL) run the compute-bound kernels, blocks of 32 x 32 up to 256 x 256 outputs
+ * as m, n and k fill the GPU. Replaces
  * gemm.rs:161/:605 and
  * device/qwen3-tp-batch32-kernels-v5/src/projection.rs:15/:142/:241, collective.rs:25,
  * activation.rs:32 and device/qwen3-tp-fp32-head32-kernels-v8/src/projection.rs:66/:186. */

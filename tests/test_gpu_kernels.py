@@ -308,6 +308,33 @@ def test_gemm_large_m_residual_and_swiglu_epilogues(m):
         assert np.mean(got == ref) > 0.97
 
 
+# The block shapes of mid-sized batches (32 tn weight rows x 32 tm activation
+# rows, waves splitting k) and the 256-row x 128-column blocks, at their edges:
+# fewer k-blocks than waves and k-blocks not a multiple of them, row blocks
+# with one valid row, waves whose rows are all padding, weights not a multiple
+# of 256 rows. Same bounds as the other epilogues above: FP32 reassociation
+# (F32_BOUND), one bf16 rounding of such a sum, SwiGLU of two of them.
+@pytest.mark.parametrize("m,n,k,epi", [
+    (33, 128, 64, "bf16"), (33, 128, 32, "f32"),  # 4 x 4 tiles, 2 and 1 k-blocks for 4 waves
+    (777, 4096, 544, "residual"),                 # 4 x 4, 17 k-blocks, 9 rows in the last block
+    (600, 4096, 4096, "residual"), (450, 6144, 2048, "swiglu"), (640, 4096, 2048, "f32"),  # 4 x 4
+    (257, 6144, 4096, "bf16"), (513, 24576, 96, "swiglu"), (777, 4096, 1056, "f32"),       # 4 x 2
+    (289, 4096, 2048, "bf16"), (300, 4096, 4128, "f32"),                                   # 2 x 4
+    (65, 4096, 256, "residual"), (129, 2048, 1056, "bf16"), (300, 8192, 128, "swiglu"),    # 2 x 2
+    (257, 1024, 2048, "bf16"), (509, 1024, 3072, "residual"), (97, 1024, 96, "f32"),       # 1 x 2, 2 x 2
+    (40, 4096, 4096, "residual"), (48, 1024, 2080, "bf16"), (300, 384, 4096, "f32"),       # 1 x 1
+    (521, 8192, 2048, "residual"), (705, 6144, 4096, "bf16"), (600, 8192, 4096, "swiglu"), (513, 12800, 2080, "f32"),  # 256 x 128
+])
+def test_gemm_mid_sized_batches(m, n, k, epi):
+    code = {"bf16": _lib.EPI_BF16, "f32": _lib.EPI_F32, "swiglu": _lib.EPI_SWIGLU, "residual": _lib.EPI_RESIDUAL}[epi]
+    got, ref = _gemm_case(m, n, k, code, 41 * m + n + k)
+    if epi == "f32":
+        assert np.max(np.abs(got - ref)) <= F32_BOUND
+    else:
+        assert du.bf16_close(got, ref, ulps=3 if epi == "swiglu" else 1)
+        assert np.mean(got == ref) > 0.97
+
+
 @pytest.mark.parametrize("splits", [0, 1, 3])
 @pytest.mark.parametrize("rows,width", [(1, 1024), (32, 4096), (9, 4096), (100, 1024), (256, 4096), (300, 1024)])
 def test_residual_rmsnorm(splits, rows, width):

@@ -702,6 +702,16 @@ def test_prefill_chunk_8b_fused_qkv_epilogue():
     _prefill_case(cfg, limits, [150, 140], [100, 3000], 512, 43, "prefill 8b fused qkv")
 
 
+@pytest.mark.parametrize("prompts", [[270, 160], [300, 221, 200]])
+def test_prefill_chunk_8b_fused_qkv_epilogue_of_mid_sized_blocks(prompts):
+    # 8B layer geometry, one layer: at 431 rows the QKV projection runs 128 x
+    # 128 blocks (one head each, the last with 47 valid rows), at 722 rows the
+    # 256-row ones, with QK-norm, RoPE and the KV append in their epilogues.
+    cfg = dict(ferric_amd.QWEN3_8B, layers=1, vocabulary=4096)
+    limits = PagedLimits(context_tokens=2048, physical_page_count=200, page_table_stride=128)
+    _prefill_case(cfg, limits, prompts, [900], 768, 47, "prefill 8b mid-sized blocks")
+
+
 def test_prefill_qknorm_inside_block_attention_is_bit_identical():
     # A chunk of up to 256 rows whose attention blocks write no slot another
     # block reads runs the QK-norm, RoPE and KV append inside the attention
