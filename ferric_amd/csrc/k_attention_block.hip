@@ -1,5 +1,5 @@
-// K4 for prefill chunks: causal attention of blocks of consecutive rows of
-// one sequence.
+// K4 for prefill chunks of up to kPanelRows rows: causal attention of blocks
+// of consecutive rows of one sequence (larger chunks: k_attention_prefill.hip).
 //
 // Reference semantics: the batched prefill runs the paged decode attention
 // per row with that row's position (device/qwen3-all-kernels-v1/src/

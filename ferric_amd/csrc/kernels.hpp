@@ -237,6 +237,16 @@ hipError_t launch_attention_blocks(const uint16_t* q, const uint16_t* k_cache, c
                                    uint32_t qh, uint32_t kvh, uint32_t stride, uint32_t pages, uint32_t context,
                                    uint32_t* err, hipStream_t s, const AttnQkn* qkn = nullptr);
 
+// The same for chunks of long blocks (k_attention_prefill.hip): each block of
+// a chunk of `rows` rows has at most attention_prefill_block_rows(rows, qh,
+// kvh) rows. out has `rows` rows.
+uint32_t attention_prefill_block_rows(uint32_t rows, uint32_t qh, uint32_t kvh);
+hipError_t launch_attention_prefill(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_cache,
+                                    const uint32_t* positions, const uint32_t* table, const uint32_t* blocks,
+                                    uint32_t nblocks, uint16_t* out, uint32_t out_tiled, uint32_t rows, uint32_t qh,
+                                    uint32_t kvh, uint32_t stride, uint32_t pages, uint32_t context, uint32_t* err,
+                                    hipStream_t s);
+
 // logits
 // With host_choices (coherent pinned memory), the choices and the error word
 // (at host_err) are also stored there, so the host reads them without a

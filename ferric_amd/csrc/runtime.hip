@@ -976,14 +976,21 @@ fh_status fh_write_kv_page(fh_ctx* ctx, uint32_t layer, uint32_t which, uint32_t
   return FH_OK;
 }
 
+// Chunks of more than kPanelRows rows run the attention kernel of long blocks
+// (k_attention_prefill.hip); smaller ones, which run the QK-norm inside the
+// attention where they can, the one of short blocks.
+bool prefill_long_blocks(uint32_t nrows) { return nrows > fh::kPanelRows; }
+
 // Attention blocks of a prefill chunk: runs of rows of one sequence at
 // consecutive positions whose page lists extend one another (so the block's
 // last row's table serves every row of it), at most attention_block_rows()
-// rows each, stored as first row | rows << 16. Longest first: a block reads
+// (attention_prefill_block_rows()) rows each, stored as first row | rows << 16. Longest first: a block reads
 // the pages up to its last row's position, and workgroups are dispatched in
 // block order, so the short ones fill the tail.
 uint32_t prefill_blocks(const fh_ctx* ctx, const fh_row* rows, uint32_t nrows, uint32_t* blocks) {
-  const uint32_t bq = fh::attention_block_rows(ctx->md.query_heads, ctx->md.kv_heads);
+  const uint32_t bq = prefill_long_blocks(nrows)
+                          ? fh::attention_prefill_block_rows(nrows, ctx->md.query_heads, ctx->md.kv_heads)
+                          : fh::attention_block_rows(ctx->md.query_heads, ctx->md.kv_heads);
   uint32_t nblocks = 0;
   for (uint32_t i = 0; i < nrows;) {
     uint32_t j = i + 1;
@@ -991,7 +998,7 @@ uint32_t prefill_blocks(const fh_ctx* ctx, const fh_row* rows, uint32_t nrows, u
            rows[j].position == rows[j - 1].position + 1 && rows[j].page_count >= rows[j - 1].page_count &&
            std::memcmp(rows[j].pages, rows[j - 1].pages, (size_t)rows[j - 1].page_count * 4) == 0)
       ++j;
-    blocks[nblocks++] = i | ((j - i) << 16);  // i < 16384, j - i <= 64
+    blocks[nblocks++] = i | ((j - i) << 16);  // i < 16384, j - i <= 128
     i = j;
   }
   std::stable_sort(blocks, blocks + nblocks, [&](uint32_t a, uint32_t b) {
@@ -1097,6 +1104,9 @@ hipError_t enqueue_prefill(fh_ctx* ctx, uint32_t R, uint32_t nout, uint32_t nblo
     const fh::AttnQkn qa{p.part, sq, fh::partial_slab_rows(R), W.q_norm, W.k_norm, ctx->cos_t, ctx->sin_t,
                          kc,     vc, md.rms_epsilon};
     L(FH_KC_ATTENTION, [&] {
+      if (prefill_long_blocks(R))
+        return fh::launch_attention_prefill(p.qrot, kc, vc, d_pos, d_tab, d_blocks, nblocks, p.attn, 1, R, QH, KVH,
+                                            stride, pages, C, err, s);
       return fh::launch_attention_blocks(p.qrot, kc, vc, d_pos, d_tab, d_blocks, nblocks, p.attn, 1, R, QH, KVH,
                                          stride, pages, C, err, s, qkn_blocks ? &qa : nullptr);
     });

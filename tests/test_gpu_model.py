@@ -846,6 +846,95 @@ def test_prefill_ignores_unwritten_slots_of_the_last_page():
         pair.close()
 
 
+# Chunks of more than 256 rows: the attention of long blocks. Query heads per
+# KV head 1, 2, 4 and 8, and the three splits of the 4 waves over vectors and
+# keys (32-, 64- and 128-vector blocks as the chunk grows); prompts whose
+# lengths leave blocks of one row, pages and key tiles partly filled, decode
+# rows at context lengths around tile and page-table-chunk edges beside them,
+# and rows interleaved by sequence (one-row blocks).
+@pytest.mark.parametrize("qh,kvh,prompts,decode,interleave", [
+    (32, 8, [290], [63, 64, 65, 127, 129], False), (16, 8, [129, 145], [1023, 1024, 1025, 1500], False),
+    (8, 8, [257], [], False), (8, 8, [1030, 1100], [16], False), (16, 8, [600, 500], [15, 17], False),
+    (32, 8, [700], [2000], False), (32, 8, [1057], [1], False), (32, 4, [1025, 33], [40], False),
+    (32, 4, [300], [500], False), (32, 8, [100, 100, 100], [], True),
+])
+def test_prefill_attention_of_long_blocks(qh, kvh, prompts, decode, interleave):
+    cfg = dict(ferric_amd.QWEN3_0_6B, layers=1, hidden=512, query_heads=qh, kv_heads=kvh, intermediate=512,
+               vocabulary=4096)
+    limits = PagedLimits(context_tokens=2304, physical_page_count=700, page_table_stride=144)
+    seed = 61 + qh + kvh + sum(prompts)
+    pair = Pair(cfg, limits, seed=seed, rows=8, prefill_rows=2304)
+    try:
+        rng = np.random.default_rng(seed)
+        dec = pair.admit_with_prefix(decode) if decode else []
+        sids = [pair.pool.admit(0) for _ in prompts]
+        if interleave:
+            rows = [(s, int(rng.integers(0, 4096))) for t in range(prompts[0]) for s in sids]
+        else:
+            rows = [(s, int(t)) for s, n in zip(sids, prompts) for t in rng.integers(0, 4096, n)]
+        rows += [(s, int(rng.integers(0, 4096))) for s in dec]
+        outs = sorted(set(range(0, len(rows), len(rows) // 40 + 1)) | set(range(len(rows) - len(dec) - 1, len(rows))))
+        batch, out, ref = pair.step(rows, outs)
+        _mark_written(pair, batch)
+        pair.check(batch, out, ref, f"long blocks {qh}/{kvh} {prompts}")
+        pair.check_kv()
+    finally:
+        pair.close()
+
+
+def test_prefill_attention_of_long_blocks_ignores_unwritten_slots():
+    # As test_prefill_ignores_unwritten_slots_of_the_last_page, 300 rows from
+    # position 37 to 336: slots 1..15 of the last page hold NaN and infinity
+    # patterns that neither the outputs nor the error word may notice.
+    cfg = dict(ferric_amd.QWEN3_0_6B, layers=2)
+    limits = PagedLimits(context_tokens=1024, physical_page_count=64, page_table_stride=64)
+    pair = Pair(cfg, limits, seed=53, rows=8, prefill_rows=512)
+    try:
+        (a,) = pair.admit_with_prefix([37])
+        st = pair.pool.sequences[a]
+        pair.pool._ensure(st, 337)
+        page = int(st.pages[336 // 16])
+        for layer in range(cfg["layers"]):
+            for which in (0, 1):
+                got = pair.gpu.read_kv_page(layer, which, page).reshape(16, -1)
+                ref = pair.cpu.kv(layer, which).reshape(limits.physical_page_count, 16, -1)
+                for slot in range(1, 16):
+                    got[slot] = ref[page, slot] = (0x7FC0, 0x7F80, 0xFFC1)[slot % 3]
+                pair.gpu.write_kv_page(layer, which, page, got.reshape(-1))
+        rng = np.random.default_rng(53)
+        rows = [(a, int(t)) for t in rng.integers(0, cfg["vocabulary"], 300)]
+        batch, out, ref = pair.step(rows, [0, 150, 299])
+        assert batch.rows[len(rows) - 1].position == 336
+        _mark_written(pair, batch)
+        pair.check(batch, out, ref, "long blocks beside unwritten NaN slots")
+        pair.check_kv()
+    finally:
+        pair.close()
+
+
+def test_nonfinite_score_of_a_long_block_reaches_the_host():
+    # A NaN in one key of a 300-token prefix: every row of the chunk that
+    # attends to it is nonfinite, and the chunk fails.
+    cfg = dict(ferric_amd.QWEN3_0_6B, layers=1, vocabulary=4096)
+    limits = PagedLimits(context_tokens=1024, physical_page_count=64, page_table_stride=64)
+    r = TpBatchRunner(cfg, limits, row_capacity=8, use_graphs=False, prefill_rows=512)
+    try:
+        r.synthesize_weights(9, 0.02)
+        pool = PagePool(limits, seed=9)
+        s = pool.admit(300)
+        batch = pool.prepare([(s, 7 + t) for t in range(270)])
+        r.kv_fill_synthetic(9, 1.0, [batch.rows[0]], [1], 1024)
+        page = int(batch.rows[0].physical_pages[5])
+        kv = r.read_kv_page(0, 0, page)
+        kv[3] = 0x7FC0
+        r.write_kv_page(0, 0, page, kv)
+        with pytest.raises(FerricError) as e:
+            r.execute_batch(batch, [269])
+        assert e.value.status == 6, e.value
+    finally:
+        r.close()
+
+
 class ParityRunner:
     """A TpBatchRunner stand-in for the speculative decoder that runs every
     batch on the GPU and on the oracle (same prepared rows and page tables,
