@@ -69,9 +69,8 @@ __device__ __forceinline__ void wave_fence() {
 // EPI == kBandEpiQkvRope (the QKV projection of a prefill chunk): 4 column groups
 // are one head (128 columns) of the wave's 64 rows. The wave stages them in
 // LDS as bf16 rows (the projection's rounding) and lane r runs the per-head
-// QK-norm, RoPE and KV append of row r (qk_head.hpp): the same lane code and
-// order as the lane-per-head kernel, without the QKV output's round trip
-// through HBM or a second launch.
+// QK-norm, RoPE and KV append of row r (qk_head.hpp), without the QKV output's
+// round trip through HBM or a second launch.
 constexpr int kBandEpiQkvRope = 16;
 constexpr int kQkPitch = 68;     // words per staged head row: 64 + 4 keeps rows 16-byte aligned, reads conflict-free
 constexpr int kStagePitch = 68;  // floats per staged row of 64 columns
@@ -248,7 +247,7 @@ __global__ __launch_bounds__(64 * kBandWaves, 2) void gemm_band_kernel(const uin
           }
       wave_fence();
       if (row0 + lane < m)
-        qknorm_rope_kv_head<32, true>(reinterpret_cast<const qk_u32x4*>(rows_lds + lane * kQkPitch), row0 + lane,
+        qknorm_rope_kv_head<32>(reinterpret_cast<const qk_u32x4*>(rows_lds + lane * kQkPitch), row0 + lane,
                                 gx * (CG / 4) + head, qa, row_slot);
     });
   } else {

@@ -238,7 +238,7 @@ __global__ __launch_bounds__(WAVES * 64, OCC) void gemm_mid_kernel(const uint16_
   }
   if constexpr (EPI == kMidEpiQkvRope) {
     // The head's rows staged as bf16 (the projection's rounding), then one
-    // lane per row runs the lane-per-head kernel's code (qk_head.hpp).
+    // lane per row runs the QK-norm, RoPE and KV append (qk_head.hpp).
     uint32_t* rows_lds = reinterpret_cast<uint32_t*>(lds_raw);
     __syncthreads();  // every wave is done reading the reduction's LDS
     mid_for<0, TM>([&](auto j_c) {
@@ -252,7 +252,7 @@ __global__ __launch_bounds__(WAVES * 64, OCC) void gemm_mid_kernel(const uint16_
     __syncthreads();
     const uint32_t row = gy * 32 * TM + threadIdx.x;
     if (threadIdx.x < 32 * TM && row < m)
-      qknorm_rope_kv_head<TM >= 4 ? 32 : 8, true>(reinterpret_cast<const qk_u32x4*>(rows_lds + threadIdx.x * kMidQkPitch), row, gx, qa,
+      qknorm_rope_kv_head<(TM >= 4 ? 32 : 8)>(reinterpret_cast<const qk_u32x4*>(rows_lds + threadIdx.x * kMidQkPitch), row, gx, qa,
                                     row_slot);
   }
 }

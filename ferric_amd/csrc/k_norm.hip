@@ -316,20 +316,111 @@ __global__ __launch_bounds__(kNormThreads) void residual_rmsnorm_kernel(uint16_t
   if (bad) raise_error(err, ERR_NONFINITE);
 }
 
-// The same computation for bf16 QKV rows (S = 0, the prefill path), one
-// lane per (row, head) (qk_head.hpp): the lane holds the head's 128 values
-// and runs the serial sum of squares (ascending element order, each square
-// rounded before the add, exactly as above) itself, so no cross-lane chain
-// limits a chunk of thousands of rows. Value heads are copied raw into the
-// slot.
-__global__ __launch_bounds__(256, 2) void qknorm_rope_kv_rows_kernel(const uint16_t* __restrict__ qkv, QkvRopeArgs a,
-                                                                     uint32_t rows) {
-  const uint32_t all = a.qh + 2 * a.kvh;
-  const uint64_t gid = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-  if (gid >= (uint64_t)rows * all) return;
-  const uint32_t row = (uint32_t)(gid / all), head = (uint32_t)(gid % all);
-  qknorm_rope_kv_head(reinterpret_cast<const qk_u32x4*>(qkv + (uint64_t)row * all * 128 + (uint64_t)head * 128), row,
-                      head, a, qkv_row_slot(row, a));
+// The same computation for bf16 QKV rows (S = 0) of many rows. A workgroup
+// takes 64 consecutive (row, head)s, 16 KiB of contiguous QKV rows: they come
+// into LDS with coalesced loads, one lane per (row, head) adds its 128 squares
+// in element order (each square rounded before the add, exactly as above: the
+// only serial part), then all lanes normalize and rotate, 8 dims of each half
+// at a time, and store whole 16-byte pieces. (One lane per (row, head) for
+// everything read and wrote 256 bytes per lane and ran 1000 rows of the 8B
+// shape in 750 waves: 25 us, 9.7 here; 257 rows 22 -> 5.5, 8000 rows 98 -> 47.)
+constexpr int kRowsHeads = 64;   // (row, head)s per workgroup
+constexpr int kRowsPitch = 68;   // words per staged head: 64 + 4 spreads the lanes' reads over the banks
+
+__global__ __launch_bounds__(256) void qknorm_rope_kv_rows_kernel(const uint16_t* __restrict__ qkv, QkvRopeArgs a,
+                                                                  uint32_t rows) {
+  __shared__ __attribute__((aligned(16))) uint32_t x_s[kRowsHeads * kRowsPitch];
+  __shared__ float inv_s[kRowsHeads];
+  const uint32_t all = a.qh + 2 * a.kvh, heads = a.qh + a.kvh;
+  const uint64_t total = (uint64_t)rows * all, first = (uint64_t)blockIdx.x * kRowsHeads;
+  const uint32_t count = (uint32_t)(total - first < kRowsHeads ? total - first : kRowsHeads);
+  const uint4* src = reinterpret_cast<const uint4*>(qkv + first * 128);
+#pragma unroll
+  for (int i = 0; i < kRowsHeads * 16 / 256; ++i) {
+    const uint32_t c = threadIdx.x + i * 256;  // 16-byte chunk: (row, head) c / 16, dims 8 (c % 16) .. + 7
+    if (c < count * 16) *reinterpret_cast<uint4*>(&x_s[(c >> 4) * kRowsPitch + (c & 15u) * 4]) = src[c];
+  }
+  __syncthreads();
+  bool bad = false;
+  if (threadIdx.x < count) {
+    const uint4* xr = reinterpret_cast<const uint4*>(&x_s[threadIdx.x * kRowsPitch]);
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const uint4 v = xr[i];
+      const uint32_t words[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float e0 = lo_bf16(words[k]), e1 = hi_bf16(words[k]);
+        const float s0 = e0 * e0, s1 = e1 * e1;
+        sum = sum + s0;
+        sum = sum + s1;
+      }
+    }
+    const float inv = inverse_rms(sum, 128.0f, a.eps);
+    // (A nonfinite element makes the sum nonfinite; value heads are not checked.)
+    if ((uint32_t)((first + threadIdx.x) % all) < heads) bad = !is_finite_f32(sum) | !is_finite_f32(inv);
+    inv_s[threadIdx.x] = inv;
+  }
+  __syncthreads();
+  // Piece p: (row, head) p / 8 of the workgroup, dims 8 (p % 8) .. + 7 and the
+  // same + 64.
+#pragma unroll
+  for (int i = 0; i < kRowsHeads * 8 / 256; ++i) {
+    const uint32_t p = threadIdx.x + i * 256, hl = p >> 3, g = p & 7u;
+    if (hl >= count) break;
+    const uint32_t row = (uint32_t)((first + hl) / all), head = (uint32_t)((first + hl) % all);
+    const QkvRowSlot rs = qkv_row_slot(row, a);
+    if (!rs.slot_ok && head == 0 && g == 0) raise_error(a.err, ERR_PAGE);
+    uint4 xa = *reinterpret_cast<const uint4*>(&x_s[hl * kRowsPitch + 4 * g]);
+    uint4 xb = *reinterpret_cast<const uint4*>(&x_s[hl * kRowsPitch + 32 + 4 * g]);
+    uint16_t* dst = nullptr;
+    if (head >= heads) {
+      if (rs.slot_ok) dst = a.v_cache + ((uint64_t)rs.slot + (head - heads)) * 128;
+    } else {
+      if (head < a.qh)
+        dst = a.q_out + ((uint64_t)row * a.qh + head) * 128;
+      else if (rs.slot_ok)
+        dst = a.k_cache + ((uint64_t)rs.slot + (head - a.qh)) * 128;
+      const uint16_t* wn = head < a.qh ? a.q_norm : a.k_norm;
+      const uint4 wa = *reinterpret_cast<const uint4*>(wn + 8 * g), wb = *reinterpret_cast<const uint4*>(wn + 64 + 8 * g);
+      const uint64_t trig = (uint64_t)(rs.pos < a.context ? rs.pos : 0) * 64 + 8 * g;
+      const float4* ct = reinterpret_cast<const float4*>(a.cos_t + trig);
+      const float4* st = reinterpret_cast<const float4*>(a.sin_t + trig);
+      const float4 c0 = ct[0], c1 = ct[1], s0 = st[0], s1 = st[1];
+      const float cs[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+      const float sn[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+      const uint32_t as[4] = {xa.x, xa.y, xa.z, xa.w}, bs[4] = {xb.x, xb.y, xb.z, xb.w};
+      const uint32_t was[4] = {wa.x, wa.y, wa.z, wa.w}, wbs[4] = {wb.x, wb.y, wb.z, wb.w};
+      const float inv = inv_s[hl];
+      uint32_t ra[4], rb[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        uint32_t oa[2], ob[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const float an = bf16_to_f32(norm_weight_bf16(e ? hi_bf16(as[k]) : lo_bf16(as[k]), inv,
+                                                        e ? hi_bf16(was[k]) : lo_bf16(was[k])));
+          const float bn = bf16_to_f32(norm_weight_bf16(e ? hi_bf16(bs[k]) : lo_bf16(bs[k]), inv,
+                                                        e ? hi_bf16(wbs[k]) : lo_bf16(wbs[k])));
+          const float c = cs[2 * k + e], s = sn[2 * k + e];
+          const float a_cos = an * c, b_sin = bn * s, b_cos = bn * c, a_sin = an * s;
+          oa[e] = f32_to_bf16(a_cos - b_sin);
+          ob[e] = f32_to_bf16(b_cos + a_sin);
+          bad |= ((oa[e] & 0x7f80u) == 0x7f80u) | ((ob[e] & 0x7f80u) == 0x7f80u);
+        }
+        ra[k] = oa[0] | (oa[1] << 16);
+        rb[k] = ob[0] | (ob[1] << 16);
+      }
+      xa = make_uint4(ra[0], ra[1], ra[2], ra[3]);
+      xb = make_uint4(rb[0], rb[1], rb[2], rb[3]);
+    }
+    if (dst) {
+      *reinterpret_cast<uint4*>(dst + 8 * g) = xa;
+      *reinterpret_cast<uint4*>(dst + 64 + 8 * g) = xb;
+    }
+  }
+  if (bad) raise_error(a.err, ERR_NONFINITE);
 }
 
 // RMSNorm of many rows into activation tile order (the prefill path, no
@@ -418,6 +509,68 @@ __global__ __launch_bounds__(kTileThreads) void rmsnorm_tile_rows_kernel(const u
   if (bad || (t == 0 && bad_s)) raise_error(err, ERR_NONFINITE);
 }
 
+// The same for fewer rows: one wave per row, 4 rows per workgroup, so that a
+// chunk of some hundred rows gives every CU a workgroup (the 16-row-tile
+// kernel gives 777 rows to 49 of them: 15.0 us at width 4096, 6.1 here; 257 rows
+// 12.8 -> 4.8, 3000 rows 17.6 -> 14.5; beyond kWaveRowsMax rows its whole-tile
+// stores win: 8192 rows 30 us there, 44 here).
+// Lane l holds chunks l, l + 64, ... of its row (16 bytes each, all requested
+// at once); squares are summed per lane in chunk order, then by the wave's
+// butterfly. A tile row piece is 16 bytes, so the 4 workgroups of a 16-row
+// tile run on one XCD, whose L2 merges their lines. width <= 512 CH.
+template <int CH>
+__global__ __launch_bounds__(kNormThreads) void rmsnorm_wave_rows_kernel(const uint16_t* __restrict__ x,
+                                                                         const uint16_t* __restrict__ w,
+                                                                         uint16_t* __restrict__ y, uint32_t rows,
+                                                                         uint32_t y_mtiles, uint32_t width, float eps,
+                                                                         uint32_t* err) {
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, b = blockIdx.x;
+  // Workgroups go to the 8 XCDs round-robin: 32 in a row hold 8 tiles.
+  const uint32_t tile = (b >> 5) * 8 + (b & 7u), row = tile * kTileRows + ((b >> 3) & 3u) * 4 + wave;
+  if (tile * kTileRows >= rows) return;
+  const uint32_t chunks = width / 8;
+  const bool live = row < rows;
+  uint4 v[CH], wv[CH];
+#pragma unroll
+  for (int j = 0; j < CH; ++j) {
+    const uint32_t c = lane + 64 * j;
+    v[j] = live && c < chunks ? *reinterpret_cast<const uint4*>(x + (uint64_t)row * width + c * 8) : make_uint4(0u, 0u, 0u, 0u);
+    wv[j] = c < chunks ? *reinterpret_cast<const uint4*>(w + c * 8) : make_uint4(0u, 0u, 0u, 0u);
+  }
+  float sum = 0.f;
+#pragma unroll
+  for (int j = 0; j < CH; ++j) {
+    const uint32_t words[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float a = lo_bf16(words[k]), c = hi_bf16(words[k]);
+      sum = sum + a * a;
+      sum = sum + c * c;
+    }
+  }
+  sum = wave_sum(sum);
+  const float inv = inverse_rms(sum, (float)width, eps);
+  bool bad = live && (!is_finite_f32(sum) || !is_finite_f32(inv));
+#pragma unroll
+  for (int j = 0; j < CH; ++j) {
+    const uint32_t c = lane + 64 * j;
+    if (c >= chunks) break;
+    uint32_t o[4] = {0u, 0u, 0u, 0u};  // rows past the batch in the last tile: zeros
+    if (live) {
+      const uint32_t xs[4] = {v[j].x, v[j].y, v[j].z, v[j].w}, ws[4] = {wv[j].x, wv[j].y, wv[j].z, wv[j].w};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t a = norm_weight_bf16(lo_bf16(xs[k]), inv, lo_bf16(ws[k]));
+        const uint32_t e = norm_weight_bf16(hi_bf16(xs[k]), inv, hi_bf16(ws[k]));
+        bad |= ((a & 0x7f80u) == 0x7f80u) | ((e & 0x7f80u) == 0x7f80u);
+        o[k] = a | (e << 16);
+      }
+    }
+    *reinterpret_cast<uint4*>(y + act_offset_m(row, c * 8, y_mtiles)) = make_uint4(o[0], o[1], o[2], o[3]);
+  }
+  if (bad) raise_error(err, ERR_NONFINITE);
+}
+
 // Row-major <-> activation tile order, one 16-byte chunk per thread.
 __global__ __launch_bounds__(kNormThreads) void tile_activation_kernel(const uint16_t* __restrict__ x,
                                                                        uint16_t* __restrict__ xt, uint32_t m,
@@ -435,11 +588,26 @@ __global__ __launch_bounds__(kNormThreads) void tile_activation_kernel(const uin
   }
 }
 
+// Eight elements per thread in 16-byte loads and stores (12.3 M elements: 22.3 ->
+// 14.5 us, 5.1 TB/s; 98 M: 174 -> 106 us), then the elements past the last whole eight. aligned: all three pointers are 16-byte aligned;
+// else every element on its own.
 __global__ __launch_bounds__(kNormThreads) void swiglu_kernel(const uint16_t* __restrict__ gate,
                                                               const uint16_t* __restrict__ up,
-                                                              uint16_t* __restrict__ out, uint64_t n, uint32_t* err) {
+                                                              uint16_t* __restrict__ out, uint64_t n,
+                                                              uint32_t aligned, uint32_t* err) {
   bool bad = false;
-  for (uint64_t i = (uint64_t)blockIdx.x * kNormThreads + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kNormThreads)
+  const uint64_t first = (uint64_t)blockIdx.x * kNormThreads + threadIdx.x, step = (uint64_t)gridDim.x * kNormThreads;
+  const uint64_t eights = aligned ? n / 8 : 0;
+  for (uint64_t i = first; i < eights; i += step) {
+    const uint4 g = reinterpret_cast<const uint4*>(gate)[i], u = reinterpret_cast<const uint4*>(up)[i];
+    const uint32_t gs[4] = {g.x, g.y, g.z, g.w}, us[4] = {u.x, u.y, u.z, u.w};
+    uint32_t o[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      o[k] = swiglu_bf16(lo_bf16(gs[k]), lo_bf16(us[k]), bad) | (swiglu_bf16(hi_bf16(gs[k]), hi_bf16(us[k]), bad) << 16);
+    reinterpret_cast<uint4*>(out)[i] = make_uint4(o[0], o[1], o[2], o[3]);
+  }
+  for (uint64_t i = eights * 8 + first; i < n; i += step)
     out[i] = (uint16_t)swiglu_bf16(bf16_to_f32(gate[i]), bf16_to_f32(up[i]), bad);
   if (bad) raise_error(err, ERR_NONFINITE);
 }
@@ -455,6 +623,11 @@ hipError_t launch_rmsnorm(const uint16_t* x, const uint16_t* w, uint16_t* y, uin
 // Row counts up to which the norms run one wave or workgroup per row (and
 // head) rather than the many-row kernels.
 constexpr uint32_t kWaveNormRows = 256;
+// Row counts up to which the RMSNorm of many rows runs one wave per row (5000
+// rows of width 4096: 20.8 us against 23.6 with 16-row tiles; 8000: 43 against 30).
+constexpr uint32_t kWaveRowsMax = 5120;
+// Row counts up to which the QK-norm of bf16 rows runs one wave per (row, head).
+constexpr uint32_t kWaveQkRows = 64;
 
 hipError_t launch_qknorm_rope_kv(const uint16_t* qkv, const float* qkv_part, uint32_t splits, const uint16_t* q_norm,
                                  const uint16_t* k_norm, const float* cos_t, const float* sin_t,
@@ -462,13 +635,17 @@ hipError_t launch_qknorm_rope_kv(const uint16_t* qkv, const float* qkv_part, uin
                                  uint16_t* k_cache, uint16_t* v_cache, uint32_t rows, uint32_t qh, uint32_t kvh,
                                  uint32_t stride, uint32_t pages, uint32_t context, float eps, uint32_t* err,
                                  hipStream_t s) {
-  // bf16 rows: up to 256 rows one wave per (row, head) as in decode (the
-  // 8B shape at 160 rows: 6400 waves); beyond that one lane per (row, head).
-  if (!qkv_part && rows > kWaveNormRows) {
-    const uint64_t lanes = (uint64_t)rows * (qh + 2 * kvh);
+  // bf16 rows: a few rows one wave per (row, head) as in decode; beyond that
+  // 64 (row, head)s per workgroup (8B shape, 256 rows: 11.1 -> 5.5 us).
+  // (Its 16-byte accesses need aligned operands; others keep the waves.)
+  const uintptr_t bits = (uintptr_t)qkv | (uintptr_t)q_norm | (uintptr_t)k_norm | (uintptr_t)cos_t | (uintptr_t)sin_t |
+                         (uintptr_t)q_out | (uintptr_t)k_cache | (uintptr_t)v_cache;
+  if (!qkv_part && rows > kWaveQkRows && (bits & 15u) == 0) {
+    const uint64_t heads = (uint64_t)rows * (qh + 2 * kvh);
     const QkvRopeArgs a{q_norm, k_norm, cos_t, sin_t, positions, table, q_out, k_cache, v_cache,
                         qh,     kvh,    stride, pages, context, eps,   err};
-    hipLaunchKernelGGL(qknorm_rope_kv_rows_kernel, dim3((unsigned)((lanes + 255) / 256)), dim3(256), 0, s, qkv, a, rows);
+    hipLaunchKernelGGL(qknorm_rope_kv_rows_kernel, dim3((unsigned)((heads + kRowsHeads - 1) / kRowsHeads)), dim3(256), 0, s,
+                       qkv, a, rows);
     return hipGetLastError();
   }
   const dim3 grid((qh + 2 * kvh + kHeadsPerGroup - 1) / kHeadsPerGroup, rows);
@@ -497,6 +674,16 @@ hipError_t launch_residual_rmsnorm(uint16_t* hidden, const float* partials, uint
                                    uint32_t* err, hipStream_t s) {
   // One workgroup per row up to 256 rows (160 rows: 160 workgroups, where
   // the 16-row-tile kernel would run 10), one per 16-row tile beyond.
+  if (!partials && y_tiled && rows > kWaveNormRows && rows <= kWaveRowsMax && width % 32 == 0 && width <= 4096) {
+    const dim3 grid((rows + kTileRows * 8 - 1) / (kTileRows * 8) * 32);
+    if (width <= 1024)
+      hipLaunchKernelGGL(rmsnorm_wave_rows_kernel<2>, grid, dim3(kNormThreads), 0, s, hidden, w, y, rows,
+                         act_mtiles(rows), width, eps, err);
+    else
+      hipLaunchKernelGGL(rmsnorm_wave_rows_kernel<8>, grid, dim3(kNormThreads), 0, s, hidden, w, y, rows,
+                         act_mtiles(rows), width, eps, err);
+    return hipGetLastError();
+  }
   if (!partials && y_tiled && rows > kWaveNormRows && width % 32 == 0 && width <= 4096) {
     hipLaunchKernelGGL(rmsnorm_tile_rows_kernel, dim3((rows + kTileRows - 1) / kTileRows), dim3(kTileThreads), 0, s,
                        hidden, w, y, rows, act_mtiles(rows), width, eps, err);
@@ -539,10 +726,12 @@ hipError_t launch_tile_activation(const uint16_t* x, uint16_t* x_tiled, uint32_t
 
 hipError_t launch_swiglu(const uint16_t* gate, const uint16_t* up, uint16_t* out, uint64_t n, uint32_t* err,
                          hipStream_t s) {
-  uint64_t g = (n + kNormThreads - 1) / kNormThreads;
+  const bool aligned = (((uintptr_t)gate | (uintptr_t)up | (uintptr_t)out) & 15u) == 0;
+  const uint64_t per = aligned ? 8 * kNormThreads : kNormThreads;
+  uint64_t g = (n + per - 1) / per;
   if (g > 65536) g = 65536;
-  if (g == 0) g = 1;
-  hipLaunchKernelGGL(swiglu_kernel, dim3((unsigned)g), dim3(kNormThreads), 0, s, gate, up, out, n, err);
+  hipLaunchKernelGGL(swiglu_kernel, dim3((unsigned)g), dim3(kNormThreads), 0, s, gate, up, out, n, aligned ? 1u : 0u,
+                     err);
   return hipGetLastError();
 }
 

@@ -368,6 +368,14 @@ def test_residual_rmsnorm(splits, rows, width):
     assert np.mean(got == ref) > 0.99
 
 
+# One wave per row (257 to 5120 rows: a last tile of 1 and of 11 rows, a width
+# of less than a wave's 64 chunks, widths that leave a wave's last chunks
+# partly used) and the 16-row tiles beyond.
+@pytest.mark.parametrize("rows,width", [(257, 4096), (523, 4096), (300, 512), (400, 1056), (289, 96), (5200, 256)])
+def test_rmsnorm_of_many_rows(rows, width):
+    test_residual_rmsnorm(0, rows, width)
+
+
 def test_residual_narrowing_is_the_reference_rounding():
     # hidden = bf16((0 + P) + 0) narrows arbitrary FP32 partials: ties to
     # even, carries into the exponent, subnormals, overflow to infinity and
@@ -862,6 +870,31 @@ def test_paged_attention_long_context():
                                      int(positions[i]), kvh, h // (qh // kvh))
             worst = max(worst, du.bf16_rel_err(got[i, h], ref))
     assert worst <= 1e-2, worst
+
+
+# Many bf16 rows: 64 (row, head)s per workgroup, the last one partly filled;
+# heads per row that do and do not divide 64.
+@pytest.mark.parametrize("qh,kvh,rows", [(32, 8, 64), (32, 8, 65), (16, 8, 131), (8, 8, 257), (32, 4, 300)])
+def test_qknorm_rope_kv_of_many_rows_bit_exact(qh, kvh, rows):
+    test_qknorm_rope_kv_bit_exact(qh, kvh, 0, rows)
+
+
+# Element counts around the eight of a thread and operands off the 16-byte
+# alignment its loads need: same elements as one launch per whole array.
+@pytest.mark.parametrize("n,offset", [(1, 0), (7, 0), (8, 0), (2049, 0), (4103, 1), (4096, 4), (16389, 8)])
+def test_swiglu_remainders_and_alignment(n, offset):
+    r = rng(n + offset)
+    gate, up = rand_bf16(r, n + offset, 4.0), rand_bf16(r, n + offset, 1.0)
+    out = du.to_dev(np.full(n + offset + 8, 0x1234, np.uint16))
+    err = du.empty(1, np.uint32)
+    dg, dup = du.to_dev(gate), du.to_dev(up)
+    _lib.check(LIB.fh_op_swiglu(du.ptr(dg) + 2 * offset, du.ptr(dup) + 2 * offset, du.ptr(out) + 2 * offset, n,
+                                du.ptr(err), du.stream()))
+    got = du.to_host(out, np.uint16)
+    ref = orc.swiglu(gate[offset:], up[offset:])
+    assert du.to_host(err, np.uint32)[0] == 0
+    assert du.bf16_ulp_diff(got[offset:offset + n], ref) <= 1
+    assert np.all(got[:offset] == 0x1234) and np.all(got[offset + n:] == 0x1234)
 
 
 def test_swiglu_standalone():
