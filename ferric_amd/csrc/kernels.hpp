@@ -13,25 +13,49 @@ namespace fh {
 void set_thread_error(const char* msg);
 
 // Attention partitions: each partition workgroup covers split_pages pages of
-// 16 tokens (16 or 32; its 8 waves take split_pages / 8 pages each). Batches
-// of at most 64 (row, query head) pairs, and models of at most 16 query heads
-// (2 per KV head in Qwen3-0.6B, half the work per page of the 8B's 4), take
-// 16-page partitions. Measured on MI355X: one Qwen3-8B row at a 4096-token
-// context 13.1 us against 15.7 us for 32 pages (15.2 us for 8); 4 and 32
-// rows of the 8B: 32 pages best (32 rows, contexts U[512, 8192]: attention
-// 3.63 against 4.29 ms per step with 16); 32 rows of the 0.6B, contexts
-// U[128, 2048]: 0.866 against 0.933 ms per step with 32 (2.04 against 2.12
-// ms per step). A context capacity of 257..512 tokens takes one 32-page
-// partition whatever the batch, so every row finishes in its partition with
-// no records and no merge (a speculative round's 0.6B draft, 32 rows at
-// 256-410 tokens of a 512-token capacity: 14.4 -> 11.8 us per launch, 1.155
-// -> 1.112 ms device time per step). attn_split_pages is the one policy
-// every launcher and workspace size uses.
+// 16 tokens (16 or 32; its 8 waves take split_pages / 8 pages each). Launches
+// of at most 256 workgroups of 16 pages at the context capacity (1024
+// partitions of a (row, query head) at 4 query heads per KV head) and models
+// of at most 16 query heads (2 per KV head in Qwen3-0.6B, half the work per
+// page of the 8B's 4) take 16-page partitions: with CUs idle anyway a wave's
+// chain over 2 pages is shorter than over 4. Measured on MI355X, us per
+// attention at 16 / 32 pages, 8B heads: 1 row of 4096 tokens 11.9 / 15.3, 4
+// rows at U[300, 2048] of a 2048-token capacity 12.0 / 15.3, 8 rows at U[200,
+// 1000] of 1024 11.8 / 15.2; beyond: 2 rows at U[512, 8192] of 8192 19.8 /
+// 16.1, 8 rows at U[300, 2048] 17.2 / 16.3, 32 rows at U[512, 8192] 149 / 129.
+// 32 rows of the 0.6B, contexts U[128, 2048]: 0.866 against 0.933 ms per step
+// with 32 (2.04 against 2.12 ms per step). A context capacity of 257..512
+// tokens takes one 32-page partition whatever the batch, so every row finishes
+// in its partition with no records and no merge (a speculative round's 0.6B
+// draft, 32 rows at 256-410 tokens of a 512-token capacity: 14.4 -> 11.8 us
+// per launch, 1.155 -> 1.112 ms device time per step). attn_split_pages is the
+// one policy every launcher and workspace size uses.
 constexpr uint32_t kAttnMaxSplitPages = 32;
 constexpr uint32_t kAttnMinSplitPages = 16;
+constexpr uint32_t kAttnSmallPartitions = 1024;
+inline uint32_t attn_max_splits(uint32_t context_tokens, uint32_t split_pages) {
+  return (context_tokens + split_pages * 16 - 1) / (split_pages * 16);
+}
 inline uint32_t attn_split_pages(uint32_t rows, uint32_t query_heads, uint32_t context_tokens) {
   if (context_tokens > kAttnMinSplitPages * 16 && context_tokens <= kAttnMaxSplitPages * 16) return kAttnMaxSplitPages;
-  return (uint64_t)rows * query_heads <= 64 || query_heads <= 16 ? 16u : 32u;
+  if (query_heads <= 16) return kAttnMinSplitPages;
+  const uint64_t partitions = (uint64_t)rows * query_heads * attn_max_splits(context_tokens, kAttnMinSplitPages);
+  return partitions <= kAttnSmallPartitions ? kAttnMinSplitPages : kAttnMaxSplitPages;
+}
+// Partition records of a launch, and the most that any launch of at most
+// `rows` rows needs (16-page partitions of a few rows can outnumber 32-page
+// ones of more).
+inline uint64_t attn_records(uint32_t rows, uint32_t query_heads, uint32_t context_tokens) {
+  return (uint64_t)rows * query_heads *
+         attn_max_splits(context_tokens, attn_split_pages(rows, query_heads, context_tokens));
+}
+inline uint64_t attn_records_up_to(uint32_t rows, uint32_t query_heads, uint32_t context_tokens) {
+  const uint64_t own = attn_records(rows, query_heads, context_tokens);
+  const uint64_t per_row = (uint64_t)query_heads * attn_max_splits(context_tokens, kAttnMinSplitPages);
+  const uint32_t small = (uint32_t)(kAttnSmallPartitions / per_row);
+  if (small == 0 || small >= rows) return own;
+  const uint64_t fewer = attn_records(small, query_heads, context_tokens);
+  return own > fewer ? own : fewer;
 }
 // Floats per attention partial record: running max, denominator, numerator[128].
 constexpr uint32_t kAttnPartialFloats = 2 + 128;
@@ -59,9 +83,6 @@ inline bool gemm_partial_rows_ok(uint32_t m, uint32_t n) {
   return m <= kMaxRows || (m <= kPanelRows && n % kPanelCols == 0);
 }
 
-inline uint32_t attn_max_splits(uint32_t context_tokens, uint32_t split_pages) {
-  return (context_tokens + split_pages * 16 - 1) / (split_pages * 16);
-}
 // Whether a decode launch merges its partitions in the partition kernel
 // (arrival counters) rather than in a second launch. Publishing the records
 // coherently adds a store and counter round trip to every partition

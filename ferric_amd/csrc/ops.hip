@@ -213,7 +213,11 @@ fh_status fh_op_paged_attention_noalloc(const uint16_t* q, const uint16_t* k_cac
   const uint32_t g = query_heads / kv_heads;
   if (g != 1 && g != 2 && g != 4 && g != 8) return FH_ERR_INVALID_ARGUMENT;
   const uint32_t split_pages = fh::attn_split_pages(rows, query_heads, context_tokens);
-  const uint64_t records = (uint64_t)rows * query_heads * fh::attn_max_splits(context_tokens, split_pages);
+  // Up to 64 (row, query head) pairs are counted at 16-page partitions, also
+  // where the launch takes 32: the limit stays where callers know it.
+  const uint64_t pairs = (uint64_t)rows * query_heads;
+  const uint64_t records = pairs <= 64 ? pairs * fh::attn_max_splits(context_tokens, fh::kAttnMinSplitPages)
+                                       : fh::attn_records(rows, query_heads, context_tokens);
   if (records > kNoAllocAttnRecords) {
     fh::set_thread_error("fh_op_paged_attention_noalloc: rows x query_heads x partitions of the context exceeds "
                          "the 16384 partition records of its static array");
@@ -233,8 +237,7 @@ fh_status fh_op_paged_attention_noalloc(const uint16_t* q, const uint16_t* k_cac
 }
 
 uint64_t fh_attention_scratch_bytes(uint32_t rows, uint32_t query_heads, uint32_t context_tokens) {
-  return (uint64_t)rows * query_heads *
-         fh::attn_max_splits(context_tokens, fh::attn_split_pages(rows, query_heads, context_tokens)) * fh::kAttnPartialFloats * 4;
+  return fh::attn_records_up_to(rows, query_heads, context_tokens) * fh::kAttnPartialFloats * 4;
 }
 
 fh_status fh_op_qknorm_paged_attention(const float* qkv_partials, uint32_t qkv_splits, const uint16_t* q_norm,

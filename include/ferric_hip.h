@@ -308,7 +308,7 @@ fh_status fh_op_qknorm_rope_kv(const void* qkv, uint32_t qkv_splits, const uint1
 /* K4 paged GQA decode attention: split-context partitions then an ordered merge.
  * q: [rows][qh*128]; out: [rows][qh*128] bf16 row-major, or activation tile order when
  * out_tiled (the output projection's input, fh_activation_rows(rows) rows);
- * scratch: fh_attention_scratch_bytes().
+ * scratch: fh_attention_scratch_bytes(), enough for every call of at most `rows` rows.
  * Replaces qwen3_paged_gqa_decode_bf16_f32_v1 (paged_decode.rs:222) and the split8
  * partial/merge pair (device/qwen3-tp-c1-split8-attention-kernels-v21/src/attention.rs:16, :214). */
 uint64_t fh_attention_scratch_bytes(uint32_t rows, uint32_t query_heads, uint32_t context_tokens);
@@ -344,7 +344,8 @@ fh_status fh_op_qknorm_paged_attention(const float* qkv_partials, uint32_t qkv_s
  * library has launched on until the process ends. A launch needs rows x query_heads x
  * ceil(context_tokens / (16 x split_pages)) records, where split_pages is 32 (512-token
  * partitions) when 256 < context_tokens <= 512, else 16 (256-token partitions) when
- * rows x query_heads <= 64 or query_heads <= 16, else 32; larger launches return
+ * rows x query_heads x ceil(context_tokens / 256) <= 1024 or query_heads <= 16, else 32
+ * (counted as 16 when rows x query_heads <= 64); larger launches return
  * FH_ERR_INVALID_ARGUMENT.
  * Calls that overlap on one GPU share that array and race. Same kernels and results
  * as fh_op_paged_attention. */

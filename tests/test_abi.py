@@ -116,6 +116,17 @@ def test_scratch_sizes():
     assert lib.fh_gemm_default_splits(1024, 2048) == 4  # capped at 16 k-blocks per split
 
 
+def test_attention_scratch_of_a_batch_serves_every_smaller_one():
+    # Few rows take smaller partitions (more records per row) than many.
+    lib = ferric_amd.load()
+    for heads in (8, 16, 32):
+        for context in (1, 256, 257, 512, 513, 1024, 2048, 4097, 8192, 40960):
+            sizes = [lib.fh_attention_scratch_bytes(rows, heads, context) for rows in range(1, 65)]
+            assert sizes == sorted(sizes), (heads, context)
+    assert lib.fh_attention_scratch_bytes(4, 32, 2048) == 4 * 32 * 8 * 130 * 4  # 16-page partitions
+    assert lib.fh_attention_scratch_bytes(16, 32, 2048) == 16 * 32 * 4 * 130 * 4  # 32-page ones
+
+
 def test_ops_reject_bad_shapes_before_any_launch():
     lib = ferric_amd.load()
     p = ctypes.c_void_p(16)  # never dereferenced: validation fails first

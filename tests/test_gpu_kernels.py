@@ -879,6 +879,33 @@ def test_qknorm_rope_kv_of_many_rows_bit_exact(qh, kvh, rows):
     test_qknorm_rope_kv_bit_exact(qh, kvh, 0, rows)
 
 
+# The two partition sizes on either side of their rule (16 pages up to 1024
+# partitions of a (row, query head) at the context capacity): the last launch
+# of 16-page partitions, the first of 32, capacities one token past a multiple.
+@pytest.mark.parametrize("rows,context", [(4, 2048), (5, 2048), (8, 1024), (9, 1024), (1, 8192), (1, 8193), (3, 2305)])
+def test_paged_attention_partition_rule(rows, context):
+    r = rng(rows + context)
+    qh, kvh, stride = 32, 8, (context + 15) // 16
+    pages = stride + 5
+    kc, vc = _paged_pool(r, pages, kvh)
+    q = rand_bf16(r, rows * qh * 128, 1.0)
+    table = np.stack([r.permutation(pages)[:stride] for _ in range(rows)]).astype(np.uint32)
+    positions = np.array([context - 1] + [int(p) for p in r.integers(0, context, rows - 1)], np.uint32)
+    scratch = torch.zeros(LIB.fh_attention_scratch_bytes(rows, qh, context) // 4, dtype=torch.float32, device="cuda")
+    out, err = du.empty(rows * qh * 128, np.uint16), du.empty(1, np.uint32)
+    dkc, dvc, dq, dpos, dtab = (du.to_dev(a) for a in (kc, vc, q, positions, table))
+    _lib.check(LIB.fh_op_paged_attention(du.ptr(dq), du.ptr(dkc), du.ptr(dvc), du.ptr(dpos), du.ptr(dtab),
+                                         du.ptr(out), 0, du.ptr(scratch), rows, qh, kvh, stride, pages, context,
+                                         du.ptr(err), du.stream()))
+    assert du.to_host(err, np.uint32)[0] == 0
+    got = du.to_host(out, np.uint16).reshape(rows, qh, 128)
+    for i in range(rows):
+        for h in range(i % 4, qh, 7):
+            ref = orc.attention_head(q[(i * qh + h) * 128:(i * qh + h + 1) * 128], kc, vc, table[i], pages,
+                                     int(positions[i]), kvh, h // (qh // kvh))
+            assert du.bf16_rel_err(got[i, h], ref) <= 1e-2
+
+
 # Element counts around the eight of a thread and operands off the 16-byte
 # alignment its loads need: same elements as one launch per whole array.
 @pytest.mark.parametrize("n,offset", [(1, 0), (7, 0), (8, 0), (2049, 0), (4103, 1), (4096, 4), (16389, 8)])
