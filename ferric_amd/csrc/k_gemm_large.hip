@@ -283,6 +283,18 @@ LargeKernel pick_kernel(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, b
   return band >= 0.f && band < mid ? LargeKernel::kBand : LargeKernel::kMid;
 }
 
+// Whether a SwiGLU or FP32 projection of up to kPanelRows rows streams its
+// weight through the panel kernel: where its 128-column slices fill more than
+// half of the CUs, up to 224 rows. Fewer slices leave too many CUs idle, and
+// with more rows the panel's LDS traffic exceeds its weight stream. Panel
+// against the blocks (us, cold weights): 152 slices (19456 x 2560) 64 rows 24
+// / 26, 160 rows 35 / 38; 128 slices (16384 x 4096) 40 rows 33 / 29, 160 rows
+// 48 / 43; 48 slices (6144 x 1024) 48 rows 10.8 / 7.5, 160 rows 17.6 / 9.5; 32
+// slices (4096 x 4096) 30 / 12.5, 44 / 18.7; 192 slices (24576 x 4096) 200
+// rows 67 / 71, 240 rows 75 / 69; 1187 slices (151936 x 4096) 160 rows 283 /
+// 317, 240 rows 400 / 357.
+bool panel_streams(uint32_t m, uint32_t n) { return m <= 224 && n > 128 * kPanelCols; }
+
 }  // namespace
 
 hipError_t launch_gemm_qkv_rope(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_t m, uint32_t n, uint32_t k,
@@ -307,8 +319,7 @@ hipError_t launch_gemm_large(const uint16_t* x_tiled, const uint16_t* w_tiled, u
                              hipStream_t s) {
   if (m <= kMaxRows) return launch_gemm(x_tiled, w_tiled, m, n, k, epilogue, 1, residual, out, ldo, err, s);
   if (n % kPanelCols != 0 || k % 32 != 0) return hipErrorInvalidValue;
-  // Up to kPanelRows rows the SwiGLU and FP32 epilogues have the panel kernel.
-  if (m <= kPanelRows && (epilogue == FH_EPI_SWIGLU || epilogue == FH_EPI_F32))
+  if ((epilogue == FH_EPI_SWIGLU || epilogue == FH_EPI_F32) && panel_streams(m, n))
     return launch_gemm(x_tiled, w_tiled, m, n, k, epilogue, 1, residual, out, ldo, err, s);
   switch (pick_kernel(m, n, k, epilogue, false)) {
     case LargeKernel::kMid:

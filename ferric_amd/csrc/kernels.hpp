@@ -197,6 +197,17 @@ hipError_t launch_gemm_rownorm(const uint16_t* w_tiled, uint32_t n, uint32_t k, 
 uint32_t gemm_default_splits(uint32_t n, uint32_t k);
 // Split-K factor for kMaxRows < m <= kPanelRows (n % kPanelCols == 0).
 uint32_t gemm_panel_splits(uint32_t n, uint32_t k);
+// Whether m rows (kMaxRows < m <= kPanelRows) of a projection whose consumer
+// folds split-K slabs are better written as one slab by the FP32 epilogue of
+// the blocks of k_gemm_mid.hip: weights of up to 16 MiB from 65 rows on,
+// where the activations every split of the panel kernel reads again outweigh
+// the weight. Panel splits against one slab (us): 1024 x 2048 64 rows 7.0 /
+// 7.3, 96 rows 8.2 / 7.1, 256 rows 14.8 / 7.0; 4096 x 2048 96 rows 9.1 / 9.2,
+// 160 rows 11.8 / 11.5, 256 rows 17.0 / 11.6; beyond, 2560 x 4096 96 rows 9.7
+// / 11.6, 160 rows 12.6 / 14.8.
+inline bool gemm_one_slab(uint32_t m, uint32_t n, uint32_t k) {
+  return m > 64 && m <= kPanelRows && (uint64_t)n * k <= 8u << 20;
+}
 
 // attention
 // out: [rows][qh*128] row-major, or activation tile order when out_tiled.

@@ -1059,14 +1059,22 @@ hipError_t enqueue_prefill(fh_ctx* ctx, uint32_t R, uint32_t nout, uint32_t nblo
   };
   // Beyond kPanelRows rows the projection kernels have the fused QKV epilogue.
   const bool fused_qkv = R > 256 && ctx->nqkv % 256 == 0 && fh::act_mtiles(R) % 16 == 0;
-  // Chunks of up to kPanelRows rows (a speculative verify) write split-K
-  // partials for QKV, O and down: the QK-norm, the post-attention norm and
+  // Chunks of up to kPanelRows rows (a speculative verify) write FP32
+  // partials for QKV, O and down (split-K slabs, or one slab where
+  // gemm_one_slab() says so): the QK-norm, the post-attention norm and
   // the next layer's input norm (after the last layer the final norm, whose
   // output is unused here) fold them, as in a decode step. Larger chunks
   // keep the residual in the projection epilogues.
   const bool split_k = R <= fh::kPanelRows;
-  const uint32_t sq = R <= kMaxRows ? ctx->s_qkv : p.s_qkv, so = R <= kMaxRows ? ctx->s_o : p.s_o,
-                 sd = R <= kMaxRows ? ctx->s_down : p.s_down;
+  const bool q_one = fh::gemm_one_slab(R, ctx->nqkv, H), o_one = fh::gemm_one_slab(R, H, Q),
+             d_one = fh::gemm_one_slab(R, H, I);
+  const uint32_t sq = R <= kMaxRows ? ctx->s_qkv : q_one ? 1u : p.s_qkv,
+                 so = R <= kMaxRows ? ctx->s_o : o_one ? 1u : p.s_o,
+                 sd = R <= kMaxRows ? ctx->s_down : d_one ? 1u : p.s_down;
+  auto partial = [&](const uint16_t* x, const uint16_t* w, uint32_t n, uint32_t k, bool one_slab, uint32_t splits) {
+    return one_slab ? fh::launch_gemm_large(x, w, R, n, k, FH_EPI_F32, nullptr, p.part, n, err, s)
+                    : fh::launch_gemm(x, w, R, n, k, FH_EPI_PARTIAL, splits, nullptr, p.part, n, err, s);
+  };
   // Split-K chunks whose blocks write no slot another block reads run the
   // QK-norm, RoPE and KV append inside the attention workgroups (one launch
   // fewer per layer).
@@ -1089,8 +1097,7 @@ hipError_t enqueue_prefill(fh_ctx* ctx, uint32_t R, uint32_t nout, uint32_t nblo
       L(FH_KC_QKV_GEMM, [&] { return fh::launch_gemm_qkv_rope(p.xn, W.qkv, R, ctx->nqkv, H, qa, s); });
     } else {
       L(FH_KC_QKV_GEMM, [&] {
-        return split_k ? fh::launch_gemm(p.xn, W.qkv, R, ctx->nqkv, H, FH_EPI_PARTIAL, sq, nullptr, p.part,
-                                         ctx->nqkv, err, s)
+        return split_k ? partial(p.xn, W.qkv, ctx->nqkv, H, q_one, sq)
                        : fh::launch_gemm_large(p.xn, W.qkv, R, ctx->nqkv, H, FH_EPI_BF16, nullptr, p.qkv,
                                                ctx->nqkv, err, s);
       });
@@ -1112,7 +1119,7 @@ hipError_t enqueue_prefill(fh_ctx* ctx, uint32_t R, uint32_t nout, uint32_t nblo
     });
     if (split_k) {
       L(FH_KC_O_GEMM, [&] {
-        return fh::launch_gemm(p.attn, W.o, R, H, Q, FH_EPI_PARTIAL, so, nullptr, p.part, H, err, s);
+        return partial(p.attn, W.o, H, Q, o_one, so);
       });
       L(FH_KC_RMSNORM, [&] {
         return fh::launch_residual_rmsnorm(p.hidden, p.part, so, W.post_norm, p.xn, 1, R, H, md.rms_epsilon, err,
@@ -1133,7 +1140,7 @@ hipError_t enqueue_prefill(fh_ctx* ctx, uint32_t R, uint32_t nout, uint32_t nblo
     if (split_k) {
       const uint16_t* next_norm = l + 1 < md.layers ? ctx->layers[l + 1].in_norm : ctx->final_norm;
       L(FH_KC_DOWN_GEMM, [&] {
-        return fh::launch_gemm(p.act, W.down, R, H, I, FH_EPI_PARTIAL, sd, nullptr, p.part, H, err, s);
+        return partial(p.act, W.down, H, I, d_one, sd);
       });
       L(FH_KC_RMSNORM, [&] {
         return fh::launch_residual_rmsnorm(p.hidden, p.part, sd, next_norm, p.xn, 1, R, H, md.rms_epsilon, err, s);
@@ -1171,8 +1178,8 @@ hipError_t enqueue_prefill(fh_ctx* ctx, uint32_t R, uint32_t nout, uint32_t nblo
 
 // A prefill chunk (row_capacity < nrows <= prefill_rows), launched eagerly:
 // the decode path's op order (batched.rs:1746-2454). Up to 256 rows (a
-// speculative verify) the projections are the panel GEMM with split-K
-// partials folded by the norms, as in a decode step; beyond that the
+// speculative verify) the projections write FP32 partials folded by the
+// norms, as in a decode step; beyond that the
 // compute-bound kernels with the residual (and, for QKV, the QK-norm, RoPE
 // and KV append) in their epilogues. Attention runs over blocks
 // of consecutive rows of one sequence (each K/V page read once per block),

@@ -233,11 +233,11 @@ fh_status fh_op_rmsnorm(const uint16_t* x, const uint16_t* weight, uint16_t* y, 
  * epilogue: FH_EPI_BF16 (one RNE), FH_EPI_RESIDUAL (bf16((0 + acc) + residual), may alias out),
  * FH_EPI_SWIGLU (w from fh_op_tile_gate_up, n = 2*i, out [m][i] = swiglu(bf16(g), bf16(u))),
  * FH_EPI_F32 (FP32 out, the LM head). m <= 32 streams the weight (decode, split-K allowed);
- * m > 32 needs n % 128 == 0 and ldo % 4 == 0: up to 256 rows FH_EPI_PARTIAL, FH_EPI_SWIGLU
- * and FH_EPI_F32 run the panel kernel (activation panel shared through LDS; split-K allowed
- * for FH_EPI_PARTIAL); the other epilogues and batches beyond 256 rows (splits = 1, no
- * FH_EPI_PARTIAL) run the compute-bound kernels, blocks of 32 x 32 up to 256 x 256 outputs
- * as m, n and k fill the GPU. Replaces
+ * m > 32 needs n % 128 == 0 and ldo % 4 == 0: FH_EPI_PARTIAL (up to 256 rows, split-K
+ * allowed) and, up to 224 rows of a weight of more than 16384 rows, FH_EPI_SWIGLU and
+ * FH_EPI_F32 run the panel kernel (weight stream, activation panel shared through LDS); the
+ * rest (splits = 1, no FH_EPI_PARTIAL) runs the compute-bound kernels, blocks of 32 x 32 up
+ * to 256 x 256 outputs as m, n and k fill the GPU. Replaces
  * gemm.rs:161/:605 and
  * device/qwen3-tp-batch32-kernels-v5/src/projection.rs:15/:142/:241, collective.rs:25,
  * activation.rs:32 and device/qwen3-tp-fp32-head32-kernels-v8/src/projection.rs:66/:186. */

@@ -335,6 +335,20 @@ def test_gemm_mid_sized_batches(m, n, k, epi):
         assert np.mean(got == ref) > 0.97
 
 
+# FP32 and SwiGLU of 33 to 256 rows, on both sides of the lines between the
+# weight stream (more than 128 slices of 128 columns, up to 224 rows) and the
+# blocks. Bounds as above.
+@pytest.mark.parametrize("m", [33, 64, 224, 225, 256])
+@pytest.mark.parametrize("n,k,epi", [(16384, 96, "swiglu"), (16512, 96, "f32"), (16512, 64, "swiglu"), (1024, 2048, "f32")])
+def test_gemm_stream_or_blocks(m, n, k, epi):
+    got, ref = _gemm_case(m, n, k, _lib.EPI_SWIGLU if epi == "swiglu" else _lib.EPI_F32, 43 * m + n + k)
+    if epi == "f32":
+        assert np.max(np.abs(got - ref)) <= F32_BOUND
+    else:
+        assert du.bf16_close(got, ref, ulps=3)
+        assert np.mean(got == ref) > 0.97
+
+
 @pytest.mark.parametrize("splits", [0, 1, 3])
 @pytest.mark.parametrize("rows,width", [(1, 1024), (32, 4096), (9, 4096), (100, 1024), (256, 4096), (300, 1024)])
 def test_residual_rmsnorm(splits, rows, width):
