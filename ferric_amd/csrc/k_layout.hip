@@ -148,6 +148,17 @@ __global__ void clear_word_kernel(uint32_t* word) {
   if (threadIdx.x == 0) *word = 0u;
 }
 
+// One workgroup per row: whole-line stores of lists that stay in L2.
+__global__ __launch_bounds__(kThreads) void expand_lists_kernel(const uint32_t* __restrict__ list,
+                                                                const uint32_t* __restrict__ lists,
+                                                                uint32_t* __restrict__ table, uint32_t stride,
+                                                                uint32_t* __restrict__ word) {
+  const uint32_t* from = lists + (uint64_t)list[blockIdx.x] * stride;
+  uint32_t* to = table + (uint64_t)blockIdx.x * stride;
+  for (uint32_t c = threadIdx.x; c < stride; c += kThreads) to[c] = from[c];
+  if (blockIdx.x == 0 && threadIdx.x == 0) *word = 0u;
+}
+
 // System-scope loads read the coherent pinned buffer past every GPU cache, so
 // each step sees what the host wrote before the launch.
 // The first launch of a decode step. The metadata block (tokens, positions,
@@ -257,6 +268,12 @@ hipError_t launch_gather_rows(const uint16_t* src, const uint32_t* index, uint16
 
 hipError_t launch_clear_word(uint32_t* word, hipStream_t s) {
   hipLaunchKernelGGL(clear_word_kernel, dim3(1), dim3(64), 0, s, word);
+  return hipGetLastError();
+}
+
+hipError_t launch_expand_lists(const uint32_t* list, const uint32_t* lists, uint32_t* table, uint32_t rows,
+                               uint32_t stride, uint32_t* word, hipStream_t s) {
+  hipLaunchKernelGGL(expand_lists_kernel, dim3(rows), dim3(kThreads), 0, s, list, lists, table, stride, word);
   return hipGetLastError();
 }
 

@@ -111,6 +111,9 @@ hipError_t launch_kv_fill(uint16_t* cache, const uint32_t* table, const uint32_t
 hipError_t launch_gather_rows(const uint16_t* src, const uint32_t* index, uint16_t* dst, uint32_t rows,
                               uint32_t width, hipStream_t s);
 hipError_t launch_clear_word(uint32_t* word, hipStream_t s);
+// table[i][0 .. stride) = lists[list[i]][0 .. stride) for i < rows, and *word = 0.
+hipError_t launch_expand_lists(const uint32_t* list, const uint32_t* lists, uint32_t* table, uint32_t rows,
+                               uint32_t stride, uint32_t* word, hipStream_t s);
 // The first launch of a decode step (one workgroup per row): copies `words`
 // 32-bit words of step metadata from coherent pinned host memory to device
 // memory (in place of a host-to-device copy), sets the error word to 0 or

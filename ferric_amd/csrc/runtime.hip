@@ -36,6 +36,7 @@ constexpr uint32_t kMaxRows = 32;
 // Prefill chunks: attention runs over this many rows per launch pair (bounds
 // the partition-state scratch), and at most this many output rows get logits.
 constexpr uint32_t kMaxPrefillOutputs = 256;
+constexpr uint32_t kRowsPerList = 4;  // prefill rows per page list from which the lists are uploaded, not the table
 
 thread_local std::string g_create_error;
 
@@ -120,8 +121,11 @@ struct fh_ctx {
     float* logits = nullptr;       // [kMaxPrefillOutputs][vocab]
     void* argmax_scratch = nullptr;
     uint32_t* choices = nullptr;
-    uint32_t* d_meta = nullptr;    // tokens[P] | positions[P] | output rows[kMaxPrefillOutputs] | blocks[P] | table[P][stride]
+    // tokens[P] | positions[P] | output rows[kMaxPrefillOutputs] | blocks[P] | page list of each row[P] |
+    // table[P][stride]; on the host the last part holds the page lists that are uploaded.
+    uint32_t* d_meta = nullptr;
     uint32_t* h_meta = nullptr;
+    uint32_t* d_lists = nullptr;   // [P / kRowsPerList][stride]: the lists the first launch expands into the table
     uint32_t* h_out = nullptr;     // choices[kMaxPrefillOutputs] | error word
   } pre;
   const float* last_logits = nullptr;  // what fh_read_logits copies
@@ -165,12 +169,12 @@ struct fh_ctx {
     uint32_t row = 0;
     uint32_t conflict = 0;
     uint32_t multi = 0;  // listed by more than one row of the batch
+    uint32_t slots = 0;  // slots written by the batch's rows, one bit each
   };
   std::vector<PageOwner> page_owner;
   std::vector<uint8_t> row_dup;  // per row of the batch: a page listed twice
   bool batch_private_slots = false;  // no row lists a page another row of the batch writes
   bool last_qkn = false;             // the last decode step ran QK-norm/KV append inside attention
-  std::vector<uint64_t> slot_scratch;
   uint64_t stamp = 0;
 };
 
@@ -307,6 +311,9 @@ fh_status check_kind_layer(fh_ctx* ctx, uint32_t kind, uint32_t layer) {
   return FH_OK;
 }
 
+// Whether two rows of a batch give one page list (the same words in memory).
+bool same_list(const fh_row& a, const fh_row& b) { return a.pages == b.pages && a.page_count == b.page_count; }
+
 // ---- batch validation (batched.rs:1678-1744, 1519-1530) -------------------
 fh_status validate_batch(fh_ctx* ctx, uint64_t batch_id, const fh_row* rows, uint32_t nrows,
                          const uint32_t* output_rows, uint32_t nout) {
@@ -330,6 +337,14 @@ fh_status validate_batch(fh_ctx* ctx, uint64_t batch_id, const fh_row* rows, uin
     const fh_row& r = rows[i];
     if (r.page_count > stride || (r.page_count && r.pages == nullptr))
       return fail(ctx, FH_ERR_INVALID_ROW, "invalid paged row geometry or aliased write slot");
+    // A third and later row with the list of the two rows before it (a prompt's
+    // rows share one) finds every page as they left it: listed by several
+    // rows, with the same conflicts. An 8000-row prompt has 4 million listings.
+    if (i > 1 && same_list(r, rows[i - 1]) && same_list(r, rows[i - 2]) && r.sequence == rows[i - 1].sequence &&
+        r.sequence == rows[i - 2].sequence) {
+      dup[i] = dup[i - 1];
+      continue;
+    }
     uint8_t row_dup = 0;
     for (uint32_t j = 0; j < r.page_count; ++j) {
       const uint32_t pg = r.pages[j];
@@ -341,6 +356,7 @@ fh_status validate_batch(fh_ctx* ctx, uint64_t batch_id, const fh_row* rows, uin
         o.logical = j;
         o.conflict = 0;
         o.multi = 0;
+        o.slots = 0;
       } else {
         row_dup |= o.row == i;
         o.multi |= o.row != i;
@@ -351,8 +367,7 @@ fh_status validate_batch(fh_ctx* ctx, uint64_t batch_id, const fh_row* rows, uin
     dup[i] = row_dup;
   }
   // Pass 2, per row in order: geometry, unique pages, unique write slots.
-  std::vector<uint64_t>& slots = ctx->slot_scratch;
-  slots.clear();
+  bool slot_twice = false;
   for (uint32_t i = 0; i < nrows; ++i) {
     const fh_row& r = rows[i];
     const uint32_t logical = r.position / kPageTokens;
@@ -360,8 +375,10 @@ fh_status validate_batch(fh_ctx* ctx, uint64_t batch_id, const fh_row* rows, uin
         r.pages[logical] != r.writable_page)
       return fail(ctx, FH_ERR_INVALID_ROW, "invalid paged row geometry or aliased write slot");
     if (dup[i]) return fail(ctx, FH_ERR_INVALID_ROW, "invalid paged row geometry or aliased write slot");
-    slots.push_back((uint64_t)r.pages[logical] * kPageTokens + r.position % kPageTokens);
-    const fh_ctx::PageOwner& o = owner[r.pages[logical]];
+    fh_ctx::PageOwner& o = owner[r.pages[logical]];
+    const uint32_t slot = 1u << (r.position % kPageTokens);
+    slot_twice |= (o.slots & slot) != 0;
+    o.slots |= slot;
     if (o.conflict || o.sequence != r.sequence || o.logical != logical)
       return fail(ctx, FH_ERR_SHARED_PAGE, "batch writes a page shared with another sequence or logical position");
   }
@@ -371,8 +388,7 @@ fh_status validate_batch(fh_ctx* ctx, uint64_t batch_id, const fh_row* rows, uin
   ctx->batch_private_slots = true;
   for (uint32_t i = 0; i < nrows; ++i)
     if (owner[rows[i].writable_page].multi) ctx->batch_private_slots = false;
-  std::sort(slots.begin(), slots.end());
-  if (std::adjacent_find(slots.begin(), slots.end()) != slots.end())
+  if (slot_twice)
     return fail(ctx, FH_ERR_INVALID_ROW, "invalid paged row geometry or aliased write slot");
   for (uint32_t i = 0; i < nout; ++i)
     if (output_rows[i] >= nrows || (i > 0 && output_rows[i] <= output_rows[i - 1]))
@@ -753,9 +769,10 @@ fh_status fh_create(const fh_model_desc* md_in, const fh_ctx_options* op_in, fh_
     TRY(dalloc(ctx, &p.logits, (uint64_t)kMaxPrefillOutputs * V));
     TRY(dalloc(ctx, reinterpret_cast<uint8_t**>(&p.argmax_scratch), fh_argmax_scratch_bytes(kMaxPrefillOutputs)));
     TRY(dalloc(ctx, &p.choices, kMaxPrefillOutputs));
-    const uint64_t pmeta = 3ull * P + kMaxPrefillOutputs + (uint64_t)P * op.page_table_stride;
+    const uint64_t pmeta = 4ull * P + kMaxPrefillOutputs + (uint64_t)P * op.page_table_stride;
     TRY(dalloc(ctx, &p.d_meta, pmeta));
     TRY(halloc(ctx, &p.h_meta, pmeta));
+    TRY(dalloc(ctx, &p.d_lists, (uint64_t)(P / kRowsPerList + 1) * op.page_table_stride));
     TRY(halloc(ctx, &p.h_out, kMaxPrefillOutputs + 1));
     // Padding rows of the tiled buffers are read (never used) by the GEMM.
     e = fh::launch_fill_u16(p.xn, tiled_rows * H, 0, ctx->stream);
@@ -996,7 +1013,8 @@ uint32_t prefill_blocks(const fh_ctx* ctx, const fh_row* rows, uint32_t nrows, u
     uint32_t j = i + 1;
     while (j < nrows && j - i < bq && rows[j].sequence == rows[i].sequence &&
            rows[j].position == rows[j - 1].position + 1 && rows[j].page_count >= rows[j - 1].page_count &&
-           std::memcmp(rows[j].pages, rows[j - 1].pages, (size_t)rows[j - 1].page_count * 4) == 0)
+           (rows[j].pages == rows[j - 1].pages ||
+            std::memcmp(rows[j].pages, rows[j - 1].pages, (size_t)rows[j - 1].page_count * 4) == 0))
       ++j;
     blocks[nblocks++] = i | ((j - i) << 16);  // i < 16384, j - i <= 128
     i = j;
@@ -1035,8 +1053,8 @@ bool prefill_blocks_private(const fh_row* rows, const uint32_t* blocks, uint32_t
 // Enqueues (or, dry, only counts) the launches of a prefill chunk of R rows
 // with nout output rows, whose metadata (tokens, positions, output rows,
 // nblocks attention blocks, page tables) is already in pre.d_meta.
-hipError_t enqueue_prefill(fh_ctx* ctx, uint32_t R, uint32_t nout, uint32_t nblocks, bool blocks_private,
-                           uint64_t* launches, bool dry = false) {
+hipError_t enqueue_prefill(fh_ctx* ctx, uint32_t R, uint32_t nout, uint32_t nblocks, uint32_t nlists,
+                           bool blocks_private, uint64_t* launches, bool dry = false) {
   const fh_model_desc& md = ctx->md;
   const fh_ctx_options& op = ctx->opt;
   auto& p = ctx->pre;
@@ -1048,7 +1066,8 @@ hipError_t enqueue_prefill(fh_ctx* ctx, uint32_t R, uint32_t nout, uint32_t nblo
   const uint32_t* d_pos = p.d_meta + P;
   const uint32_t* d_out = p.d_meta + 2 * P;
   const uint32_t* d_blocks = p.d_meta + 2 * P + kMaxPrefillOutputs;
-  const uint32_t* d_tab = p.d_meta + 3 * P + kMaxPrefillOutputs;
+  const uint32_t* d_list = p.d_meta + 3 * P + kMaxPrefillOutputs;
+  uint32_t* d_tab = p.d_meta + 4 * P + kMaxPrefillOutputs;
   Enq q{ctx, dry};
   if (!dry) (void)hipGetLastError();
   uint32_t* err = ctx->err;
@@ -1080,7 +1099,9 @@ hipError_t enqueue_prefill(fh_ctx* ctx, uint32_t R, uint32_t nout, uint32_t nblo
   // fewer per layer).
   const bool qkn_blocks = split_k && !fused_qkv && blocks_private &&
                           fh::attention_blocks_qkn_supported(QH, KVH, sq);
-  L(FH_KC_EMBEDDING, [&] { return fh::launch_clear_word(err, s); });
+  L(FH_KC_EMBEDDING, [&] {
+    return nlists ? fh::launch_expand_lists(d_list, p.d_lists, d_tab, R, stride, err, s) : fh::launch_clear_word(err, s);
+  });
   L(FH_KC_EMBEDDING, [&] { return fh::launch_embedding(d_tok, ctx->embed, p.hidden, R, H, V, err, s); });
   for (uint32_t l = 0; l < md.layers; ++l) {
     const LayerWeights& W = ctx->layers[l];
@@ -1196,13 +1217,25 @@ fh_status run_prefill(fh_ctx* ctx, uint64_t batch_id, const fh_row* rows, uint32
   uint32_t* pos = p.h_meta + P;
   uint32_t* outs = p.h_meta + 2 * P;
   uint32_t* blocks = p.h_meta + 2 * P + kMaxPrefillOutputs;
-  uint32_t* tab = p.h_meta + 3 * P + kMaxPrefillOutputs;
+  uint32_t* list = p.h_meta + 3 * P + kMaxPrefillOutputs;
+  uint32_t* tab = p.h_meta + 4 * P + kMaxPrefillOutputs;
+  uint32_t lists = 0;
   for (uint32_t i = 0; i < nrows; ++i) {
     tok[i] = rows[i].token;
     pos[i] = rows[i].position;
-    uint32_t* t = tab + (uint64_t)i * stride;
-    std::memcpy(t, rows[i].pages, rows[i].page_count * 4);
-    std::fill(t + rows[i].page_count, t + stride, 0xffffffffu);
+    lists += i == 0 || !same_list(rows[i], rows[i - 1]);
+    list[i] = lists - 1;
+  }
+  // Where kRowsPerList rows or more share a page list, each list is written
+  // and uploaded once and the first launch expands them into the per-row
+  // table (an 8000-row prompt: 2 KB for 16 MB); a table of less than 128 KB,
+  // which costs no more than the second copy, is uploaded as it is.
+  const uint32_t nlists = lists <= nrows / kRowsPerList && (uint64_t)nrows * stride >= 32768 ? lists : 0;
+  for (uint32_t i = 0, t = 0; i < nrows; ++i) {
+    if (nlists && i > 0 && list[i] == list[i - 1]) continue;
+    uint32_t* to = tab + (uint64_t)t++ * stride;
+    std::memcpy(to, rows[i].pages, rows[i].page_count * 4);
+    std::fill(to + rows[i].page_count, to + stride, 0xffffffffu);
   }
   for (uint32_t i = 0; i < nout; ++i) outs[i] = output_rows[i];
   const uint32_t nblocks = prefill_blocks(ctx, rows, nrows, blocks);
@@ -1213,13 +1246,15 @@ fh_status run_prefill(fh_ctx* ctx, uint64_t batch_id, const fh_row* rows, uint32
   };
   hipStream_t s = ctx->stream;
   uint32_t* err = ctx->err;
-  const uint64_t meta_bytes = (3ull * P + kMaxPrefillOutputs + (uint64_t)nrows * stride) * 4;
+  const uint64_t meta_bytes = (4ull * P + kMaxPrefillOutputs + (nlists ? 0ull : (uint64_t)nrows * stride)) * 4;
   hipError_t e = hipMemcpyAsync(p.d_meta, p.h_meta, meta_bytes, hipMemcpyHostToDevice, s);
+  if (e == hipSuccess && nlists)
+    e = hipMemcpyAsync(p.d_lists, tab, (uint64_t)nlists * stride * 4, hipMemcpyHostToDevice, s);
   if (e != hipSuccess) return poison(FH_ERR_DEVICE, std::string("metadata upload: ") + hipGetErrorString(e));
   hipEventRecord(ctx->ev_begin, s);
   if (ctx->profiling) ctx->prof_launches.clear();
   uint64_t n = 0;
-  e = enqueue_prefill(ctx, nrows, nout, nblocks, priv, &n);
+  e = enqueue_prefill(ctx, nrows, nout, nblocks, nlists, priv, &n);
   if (e != hipSuccess) return poison(FH_ERR_DEVICE, std::string("launch: ") + hipGetErrorString(e) + ctx->launch_detail);
   hipEventRecord(ctx->ev_end, s);
   if (nout) e = hipMemcpyAsync(p.h_out, p.choices, nout * 4, hipMemcpyDeviceToHost, s);
@@ -1372,7 +1407,7 @@ fh_status fh_expected_dispatch_count(fh_ctx* ctx, uint64_t batch_id, const fh_ro
     std::vector<uint32_t> blocks(nrows);
     const uint32_t nblocks = prefill_blocks(ctx, rows, nrows, blocks.data());
     const bool priv = nrows <= fh::kPanelRows && prefill_blocks_private(rows, blocks.data(), nblocks);
-    enqueue_prefill(ctx, nrows, nout, nblocks, priv, &n, true);
+    enqueue_prefill(ctx, nrows, nout, nblocks, 0, priv, &n, true);
   }
   else
     enqueue_step(ctx, nrows, &n, true);

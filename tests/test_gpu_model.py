@@ -538,6 +538,40 @@ def test_batch_validation_mirrors_the_reference():
         r.close()
 
 
+def test_batch_validation_of_rows_with_one_page_list():
+    # From the third row on, rows that share a page list with the two before
+    # them are not checked page by page again: what the first two established
+    # (a page listed twice, by several rows, by another sequence) must hold.
+    cfg = dict(ferric_amd.QWEN3_0_6B, layers=1)
+    limits = PagedLimits(context_tokens=256, physical_page_count=32, page_table_stride=16)
+    r = TpBatchRunner(cfg, limits, row_capacity=8, use_graphs=False)
+    try:
+        r.synthesize_weights(1, 0.02)
+        pages, twice = (4, 9), (4, 4)
+        four = [PreparedRow(1, 5, 3 + i, pages, 4) for i in range(4)]
+        bid = [100]
+
+        def run(rows):
+            bid[0] += 1
+            return r.execute_batch(PreparedBatch(bid[0], rows, limits), [0])
+
+        assert len(run(four).choices) == 1
+        for rows, status in [
+            ([PreparedRow(1, 5, 3 + i, twice, 4) for i in range(4)], 3),                    # duplicate page in each
+            (four + [PreparedRow(1, 6, 5, pages, 4)], 3),                                   # slot of the third row again
+            (four + [PreparedRow(2, 6, 20, (7, 4), 4)], 4),                                 # page of another sequence
+            (four + [PreparedRow(2, 6, 3, pages, 4)], 4),                                   # the list of another sequence
+            (four + [PreparedRow(1, 6, 20, (9, 4), 4)], 4),                                 # other logical positions
+            ([PreparedRow(2, 6, 3, (7, 9), 7)] + [PreparedRow(1, 5, 16 + i, pages, 9) for i in range(4)], 4),
+        ]:
+            with pytest.raises(FerricError) as e:
+                run(rows)
+            assert e.value.status == status, (rows, e.value)
+        assert len(run(four + [PreparedRow(2, 6, 3, (7, 9), 7)]).choices) == 1  # page 9 is read only
+    finally:
+        r.close()
+
+
 @pytest.mark.parametrize("graphs", [True, False])
 def test_device_error_of_a_decode_step_reaches_the_host(graphs):
     # A decode step's error word and choices come back through pinned host
@@ -761,6 +795,40 @@ def test_prefill_qknorm_inside_block_attention_is_bit_identical():
     assert kv_a.keys() == kv_b.keys()
     for key in kv_a:
         assert np.array_equal(kv_a[key], kv_b[key]), key
+
+
+@pytest.mark.parametrize("tokens", [(200, 100), (297, 3)])
+def test_prefill_page_lists_shared_and_given_per_row(tokens):
+    # A chunk whose rows share page lists uploads each list once and expands
+    # them on the device; the same chunk with a list of its own per row uploads
+    # the whole table. 300 rows x 128 pages are beyond the size from which the
+    # lists are uploaded. Equal bit for bit.
+    cfg = dict(ferric_amd.QWEN3_0_6B, layers=2)
+    limits = PagedLimits(context_tokens=2048, physical_page_count=64, page_table_stride=128)
+    rng = np.random.default_rng(77)
+    prompts = [rng.integers(0, cfg["vocabulary"], n) for n in tokens]
+    outs = [tokens[0] - 1, sum(tokens) - 1]
+    got = []
+    for own in (False, True):
+        runner = TpBatchRunner(cfg, limits, row_capacity=32, use_graphs=False, prefill_rows=512)
+        try:
+            runner.synthesize_weights(78, 0.02)
+            pool = PagePool(limits, seed=79)
+            sids = [pool.admit(0) for _ in prompts]
+            batch = pool.prepare([(s, int(t)) for s, p in zip(sids, prompts) for t in p])
+            if own:
+                rows = [PreparedRow(r.sequence, r.token, r.position, tuple(list(r.physical_pages)),
+                                    r.writable_physical_page) for r in batch.rows]
+                batch = PreparedBatch(batch.id, rows, limits)
+            choices = list(runner.execute_batch(batch, outs).choices)
+            kv = [runner.read_kv_cache(layer, which) for layer in range(cfg["layers"]) for which in (0, 1)]
+            got.append((choices, runner.read_logits().copy(), kv))
+        finally:
+            runner.close()
+    assert got[0][0] == got[1][0]
+    assert np.array_equal(got[0][1].view(np.uint32), got[1][1].view(np.uint32))
+    for a, b in zip(got[0][2], got[1][2]):
+        assert np.array_equal(a, b)
 
 
 @pytest.mark.parametrize("nseq", [40, 80])
