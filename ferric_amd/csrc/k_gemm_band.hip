@@ -72,7 +72,6 @@ __device__ __forceinline__ void wave_fence() {
 // QK-norm, RoPE and KV append of row r (qk_head.hpp), without the QKV output's
 // round trip through HBM or a second launch.
 constexpr int kBandEpiQkvRope = 16;
-constexpr int kQkPitch = 68;     // words per staged head row: 64 + 4 keeps rows 16-byte aligned, reads conflict-free
 constexpr int kStagePitch = 68;  // floats per staged row of 64 columns
 
 template <int EPI>
@@ -246,9 +245,7 @@ __global__ __launch_bounds__(64 * kBandWaves, 2) void gemm_band_kernel(const uin
                 make_uint2(pack_bf16x2(a[4 * e], a[4 * e + 1]), pack_bf16x2(a[4 * e + 2], a[4 * e + 3]));
           }
       wave_fence();
-      if (row0 + lane < m)
-        qknorm_rope_kv_head<32>(reinterpret_cast<const qk_u32x4*>(rows_lds + lane * kQkPitch), row0 + lane,
-                                gx * (CG / 4) + head, qa, row_slot);
+      qknorm_rope_kv_wave<64>(rows_lds, row0, m, gx * (CG / 4) + head, qa, row_slot);
     });
   } else {
     float* stage = reinterpret_cast<float*>(lds_raw) + (uint32_t)wave * 64 * kStagePitch;

@@ -73,12 +73,11 @@ __device__ __forceinline__ void static_for(F&& f) {
 //
 // EPI == kEpiQkvRope (the QKV projection of a prefill chunk): a wave's 8
 // n-tiles are exactly one head (128 columns) of 64 rows. After the k loop the
-// wave stages them in LDS as bf16 rows (the projection's rounding) and lane r
-// runs the per-head QK-norm, RoPE and KV append of row r (qk_head.hpp): the
-// same lane code and order as the lane-per-head kernel, without the QKV
-// output's round trip through HBM or a second launch.
+// wave stages them in LDS as bf16 rows (the projection's rounding) and runs
+// their QK-norm, RoPE and KV append (qknorm_rope_kv_wave, qk_head.hpp): the
+// same code and order as the kernel of many rows, without the QKV output's
+// round trip through HBM or a second launch.
 constexpr int kEpiQkvRope = 16;
-constexpr int kQkPitch = 68;  // words per staged row: 64 + 4 keeps rows 16-byte aligned, reads conflict-free
 
 template <int EPI, int LX = 3, int LW = 4>
 __global__ __launch_bounds__(512) void gemm_large_xd_kernel(const uint16_t* __restrict__ xt,
@@ -211,10 +210,7 @@ __global__ __launch_bounds__(512) void gemm_large_xd_kernel(const uint16_t* __re
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const uint32_t row = mt0 * 16 + lane;
-    if (row < m)
-      qknorm_rope_kv_head<32>(reinterpret_cast<const qk_u32x4*>(rows_lds + lane * kQkPitch), row,
-                              gx * 2 + wn, qa, row_slot);
+    qknorm_rope_kv_wave<64>(rows_lds, mt0 * 16, m, gx * 2 + wn, qa, row_slot);
     return;
   }
   if (mt0 * 16 >= m) return;  // this wave's rows are all padding

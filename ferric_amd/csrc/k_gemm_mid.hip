@@ -55,7 +55,6 @@ __device__ __forceinline__ void mid_for(F&& f) {
 // The QKV projection with QK-norm, RoPE and the KV append in its epilogue
 // (TN = 4: a workgroup's columns are one head).
 constexpr int kMidEpiQkvRope = 16;
-constexpr int kMidQkPitch = 68;  // words per staged head row: 64 + 4 keeps rows 16-byte aligned, reads conflict-free
 
 template <int TN, int TM, int WAVES, int D, int OCC, int EPI>
 __global__ __launch_bounds__(WAVES * 64, OCC) void gemm_mid_kernel(const uint16_t* __restrict__ xt,
@@ -65,8 +64,9 @@ __global__ __launch_bounds__(WAVES * 64, OCC) void gemm_mid_kernel(const uint16_
                                                                    const QkvRopeArgs qa, uint32_t* err) {
   constexpr int kN = 32 * TN, kPitch = kN + 4, kThreads = WAVES * 64;
   constexpr size_t kRedBytes = sizeof(float) * WAVES * 32 * kPitch;
-  constexpr size_t kStageBytes = EPI == kMidEpiQkvRope ? 4ull * 32 * TM * kMidQkPitch : 0;
-  static_assert(EPI != kMidEpiQkvRope || (TN == 4 && 32 * TM <= kThreads), "one head per workgroup, a lane per row");
+  constexpr size_t kStageBytes = EPI == kMidEpiQkvRope ? 4ull * 32 * TM * kQkPitch : 0;
+  constexpr int kQkRows = 32 * TM / WAVES;  // rows a wave of the fused QKV epilogue takes
+  static_assert(EPI != kMidEpiQkvRope || (TN == 4 && kQkRows % 8 == 0 && kQkRows <= 64), "one head per workgroup");
   static_assert(kRedBytes >= kStageBytes, "the staged head rows reuse the reduction's LDS");
   __shared__ __attribute__((aligned(16))) unsigned char lds_raw[kRedBytes];
   auto& red = *reinterpret_cast<float(*)[WAVES][32][kPitch]>(lds_raw);
@@ -90,8 +90,8 @@ __global__ __launch_bounds__(WAVES * 64, OCC) void gemm_mid_kernel(const uint16_
   // now and used after the k loop.
   QkvRowSlot row_slot{0u, 0u, false};
   if constexpr (EPI == kMidEpiQkvRope) {
-    const uint32_t row = gy * 32 * TM + threadIdx.x;
-    if (threadIdx.x < 32 * TM && row < m) row_slot = qkv_row_slot(row, qa);
+    const uint32_t row = gy * 32 * TM + wave * kQkRows + lane;
+    if (lane < kQkRows && row < m) row_slot = qkv_row_slot(row, qa);
   }
   const uint32_t kb_n = kb_count > (uint32_t)wave ? (kb_count - wave + WAVES - 1) / WAVES : 0u;  // k-blocks of this wave
   f32x16 acc[TN][TM];
@@ -237,8 +237,8 @@ __global__ __launch_bounds__(WAVES * 64, OCC) void gemm_mid_kernel(const uint16_
     if (bad) raise_error(err, ERR_NONFINITE);
   }
   if constexpr (EPI == kMidEpiQkvRope) {
-    // The head's rows staged as bf16 (the projection's rounding), then one
-    // lane per row runs the QK-norm, RoPE and KV append (qk_head.hpp).
+    // The head's rows staged as bf16 (the projection's rounding), then each
+    // wave runs the QK-norm, RoPE and KV append of its share (qk_head.hpp).
     uint32_t* rows_lds = reinterpret_cast<uint32_t*>(lds_raw);
     __syncthreads();  // every wave is done reading the reduction's LDS
     mid_for<0, TM>([&](auto j_c) {
@@ -246,14 +246,11 @@ __global__ __launch_bounds__(WAVES * 64, OCC) void gemm_mid_kernel(const uint16_
 #pragma unroll
       for (int s = 0; s < kSteps; ++s) {
         const int idx = threadIdx.x + s * kThreads;
-        *reinterpret_cast<uint2*>(rows_lds + (32 * j + idx / (kN / 4)) * kMidQkPitch + idx % (kN / 4) * 2) = packed[j][s];
+        *reinterpret_cast<uint2*>(rows_lds + (32 * j + idx / (kN / 4)) * kQkPitch + idx % (kN / 4) * 2) = packed[j][s];
       }
     });
     __syncthreads();
-    const uint32_t row = gy * 32 * TM + threadIdx.x;
-    if (threadIdx.x < 32 * TM && row < m)
-      qknorm_rope_kv_head<(TM >= 4 ? 32 : 8)>(reinterpret_cast<const qk_u32x4*>(rows_lds + threadIdx.x * kMidQkPitch), row, gx, qa,
-                                    row_slot);
+    qknorm_rope_kv_wave<kQkRows>(rows_lds + wave * kQkRows * kQkPitch, gy * 32 * TM + wave * kQkRows, m, gx, qa, row_slot);
   }
 }
 

@@ -325,11 +325,10 @@ __global__ __launch_bounds__(kNormThreads) void residual_rmsnorm_kernel(uint16_t
 // everything read and wrote 256 bytes per lane and ran 1000 rows of the 8B
 // shape in 750 waves: 25 us, 9.7 here; 257 rows 22 -> 5.5, 8000 rows 98 -> 47.)
 constexpr int kRowsHeads = 64;   // (row, head)s per workgroup
-constexpr int kRowsPitch = 68;   // words per staged head: 64 + 4 spreads the lanes' reads over the banks
 
 __global__ __launch_bounds__(256) void qknorm_rope_kv_rows_kernel(const uint16_t* __restrict__ qkv, QkvRopeArgs a,
                                                                   uint32_t rows) {
-  __shared__ __attribute__((aligned(16))) uint32_t x_s[kRowsHeads * kRowsPitch];
+  __shared__ __attribute__((aligned(16))) uint32_t x_s[kRowsHeads * kQkPitch];
   __shared__ float inv_s[kRowsHeads];
   const uint32_t all = a.qh + 2 * a.kvh, heads = a.qh + a.kvh;
   const uint64_t total = (uint64_t)rows * all, first = (uint64_t)blockIdx.x * kRowsHeads;
@@ -338,25 +337,12 @@ __global__ __launch_bounds__(256) void qknorm_rope_kv_rows_kernel(const uint16_t
 #pragma unroll
   for (int i = 0; i < kRowsHeads * 16 / 256; ++i) {
     const uint32_t c = threadIdx.x + i * 256;  // 16-byte chunk: (row, head) c / 16, dims 8 (c % 16) .. + 7
-    if (c < count * 16) *reinterpret_cast<uint4*>(&x_s[(c >> 4) * kRowsPitch + (c & 15u) * 4]) = src[c];
+    if (c < count * 16) *reinterpret_cast<uint4*>(&x_s[(c >> 4) * kQkPitch + (c & 15u) * 4]) = src[c];
   }
   __syncthreads();
   bool bad = false;
   if (threadIdx.x < count) {
-    const uint4* xr = reinterpret_cast<const uint4*>(&x_s[threadIdx.x * kRowsPitch]);
-    float sum = 0.f;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const uint4 v = xr[i];
-      const uint32_t words[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const float e0 = lo_bf16(words[k]), e1 = hi_bf16(words[k]);
-        const float s0 = e0 * e0, s1 = e1 * e1;
-        sum = sum + s0;
-        sum = sum + s1;
-      }
-    }
+    const float sum = qk_square_sum(&x_s[threadIdx.x * kQkPitch]);
     const float inv = inverse_rms(sum, 128.0f, a.eps);
     // (A nonfinite element makes the sum nonfinite; value heads are not checked.)
     if ((uint32_t)((first + threadIdx.x) % all) < heads) bad = !is_finite_f32(sum) | !is_finite_f32(inv);
@@ -372,53 +358,7 @@ __global__ __launch_bounds__(256) void qknorm_rope_kv_rows_kernel(const uint16_t
     const uint32_t row = (uint32_t)((first + hl) / all), head = (uint32_t)((first + hl) % all);
     const QkvRowSlot rs = qkv_row_slot(row, a);
     if (!rs.slot_ok && head == 0 && g == 0) raise_error(a.err, ERR_PAGE);
-    uint4 xa = *reinterpret_cast<const uint4*>(&x_s[hl * kRowsPitch + 4 * g]);
-    uint4 xb = *reinterpret_cast<const uint4*>(&x_s[hl * kRowsPitch + 32 + 4 * g]);
-    uint16_t* dst = nullptr;
-    if (head >= heads) {
-      if (rs.slot_ok) dst = a.v_cache + ((uint64_t)rs.slot + (head - heads)) * 128;
-    } else {
-      if (head < a.qh)
-        dst = a.q_out + ((uint64_t)row * a.qh + head) * 128;
-      else if (rs.slot_ok)
-        dst = a.k_cache + ((uint64_t)rs.slot + (head - a.qh)) * 128;
-      const uint16_t* wn = head < a.qh ? a.q_norm : a.k_norm;
-      const uint4 wa = *reinterpret_cast<const uint4*>(wn + 8 * g), wb = *reinterpret_cast<const uint4*>(wn + 64 + 8 * g);
-      const uint64_t trig = (uint64_t)(rs.pos < a.context ? rs.pos : 0) * 64 + 8 * g;
-      const float4* ct = reinterpret_cast<const float4*>(a.cos_t + trig);
-      const float4* st = reinterpret_cast<const float4*>(a.sin_t + trig);
-      const float4 c0 = ct[0], c1 = ct[1], s0 = st[0], s1 = st[1];
-      const float cs[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-      const float sn[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
-      const uint32_t as[4] = {xa.x, xa.y, xa.z, xa.w}, bs[4] = {xb.x, xb.y, xb.z, xb.w};
-      const uint32_t was[4] = {wa.x, wa.y, wa.z, wa.w}, wbs[4] = {wb.x, wb.y, wb.z, wb.w};
-      const float inv = inv_s[hl];
-      uint32_t ra[4], rb[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        uint32_t oa[2], ob[2];
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          const float an = bf16_to_f32(norm_weight_bf16(e ? hi_bf16(as[k]) : lo_bf16(as[k]), inv,
-                                                        e ? hi_bf16(was[k]) : lo_bf16(was[k])));
-          const float bn = bf16_to_f32(norm_weight_bf16(e ? hi_bf16(bs[k]) : lo_bf16(bs[k]), inv,
-                                                        e ? hi_bf16(wbs[k]) : lo_bf16(wbs[k])));
-          const float c = cs[2 * k + e], s = sn[2 * k + e];
-          const float a_cos = an * c, b_sin = bn * s, b_cos = bn * c, a_sin = an * s;
-          oa[e] = f32_to_bf16(a_cos - b_sin);
-          ob[e] = f32_to_bf16(b_cos + a_sin);
-          bad |= ((oa[e] & 0x7f80u) == 0x7f80u) | ((ob[e] & 0x7f80u) == 0x7f80u);
-        }
-        ra[k] = oa[0] | (oa[1] << 16);
-        rb[k] = ob[0] | (ob[1] << 16);
-      }
-      xa = make_uint4(ra[0], ra[1], ra[2], ra[3]);
-      xb = make_uint4(rb[0], rb[1], rb[2], rb[3]);
-    }
-    if (dst) {
-      *reinterpret_cast<uint4*>(dst + 8 * g) = xa;
-      *reinterpret_cast<uint4*>(dst + 64 + 8 * g) = xb;
-    }
+    bad |= qknorm_rope_kv_piece(&x_s[hl * kQkPitch], g, inv_s[hl], row, head, a, rs);
   }
   if (bad) raise_error(a.err, ERR_NONFINITE);
 }

@@ -1,7 +1,6 @@
-// QK-norm + RoPE + paged KV append of one (row, head) of a bf16 QKV row,
-// computed by one lane (the prefill path: the fused epilogues of the QKV
-// projection kernels, which stage their output rows in LDS and call this on
-// them), and its parts.
+// QK-norm + RoPE + paged KV append of bf16 QKV rows staged in LDS (the prefill
+// path: the fused epilogues of the QKV projection kernels and the kernel of
+// many rows), and its parts.
 //
 // Reference semantics: qwen3_rmsnorm_v1 at width 128 per head
 // (device/qwen3-all-kernels-v1/src/rmsnorm.rs:380-526; the serial sum of
@@ -127,92 +126,111 @@ __device__ __forceinline__ QkvRowSlot qkv_row_slot(uint32_t row, const QkvRopeAr
   return r;
 }
 
-// src: the head's 128 bf16 values (16-byte aligned, global or LDS). Query
-// heads 0 .. qh - 1 go to q_out, key heads qh .. qh + kvh - 1 (normed and
-// rotated) and value heads (raw) to the row's KV slot. kHoist: cos/sin pairs
-// requested at a time (fewer keep registers free; a caller with few waves
-// takes all 32 at once).
-template <int kHoist>
-__device__ __forceinline__ void qknorm_rope_kv_head(const qk_u32x4* src, uint32_t row, uint32_t head,
-                                                    const QkvRopeArgs& a, const QkvRowSlot rs) {
-  uint32_t x[64];  // x[i] = elements 2 i (low half) and 2 i + 1 (high half)
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const qk_u32x4 v = src[i];
-    x[4 * i] = v[0];
-    x[4 * i + 1] = v[1];
-    x[4 * i + 2] = v[2];
-    x[4 * i + 3] = v[3];
-  }
-  const uint32_t pos = rs.pos, slot = rs.slot;
-  const bool slot_ok = rs.slot_ok;
-  if (!slot_ok && head == 0) raise_error(a.err, ERR_PAGE);
-  const uint32_t heads = a.qh + a.kvh;
-  if (head >= heads) {
-    if (slot_ok) {
-      qk_u32x4* vo = reinterpret_cast<qk_u32x4*>(a.v_cache + ((uint64_t)slot + (head - heads)) * 128);
-#pragma unroll
-      for (int i = 0; i < 16; ++i) vo[i] = qk_u32x4{x[4 * i], x[4 * i + 1], x[4 * i + 2], x[4 * i + 3]};
-    }
-    return;
-  }
-  // (A nonfinite element makes the sum nonfinite, which is checked.)
+// Words per staged head row in LDS: 64 (128 bf16) + 4, so that rows stay
+// 16-byte aligned and the lanes' row reads spread over the banks.
+constexpr uint32_t kQkPitch = 68;
+
+// The sum of a staged head's 128 squares in element order, each square
+// rounded before the add: the only serial part.
+__device__ __forceinline__ float qk_square_sum(const uint32_t* x) {
+  const qk_u32x4* xr = reinterpret_cast<const qk_u32x4*>(x);
   float sum = 0.f;
 #pragma unroll
-  for (int i = 0; i < 64; ++i) {
-    const float e0 = lo_bf16(x[i]), e1 = hi_bf16(x[i]);
-    const float s0 = e0 * e0, s1 = e1 * e1;
-    sum = sum + s0;
-    sum = sum + s1;
-  }
-  const float inv = inverse_rms(sum, 128.0f, a.eps);
-  bool bad = !is_finite_f32(sum) | !is_finite_f32(inv);
-  // Keep only the packed words live across the reduction (the unpacked
-  // values are recomputed), or the lane runs out of registers.
-#pragma unroll
-  for (int i = 0; i < 64; ++i) asm volatile("" : "+v"(x[i]));
-  // Normalized in place, then rotated in place (pair words i and i + 32
-  // hold elements 2 i, 2 i + 1 and 2 i + 64, 2 i + 65).
-  const qk_u32x4* wn = reinterpret_cast<const qk_u32x4*>(head < a.qh ? a.q_norm : a.k_norm);
-#pragma unroll
   for (int i = 0; i < 16; ++i) {
-    const qk_u32x4 w = wn[i];
+    const qk_u32x4 v = xr[i];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t xi = x[4 * i + j];
-      const uint32_t lo = norm_weight_bf16(lo_bf16(xi), inv, lo_bf16(w[j]));
-      const uint32_t hi = norm_weight_bf16(hi_bf16(xi), inv, hi_bf16(w[j]));
-      x[4 * i + j] = lo | (hi << 16);
+    for (int k = 0; k < 4; ++k) {
+      const float e0 = lo_bf16(v[k]), e1 = hi_bf16(v[k]);
+      const float s0 = e0 * e0, s1 = e1 * e1;
+      sum = sum + s0;
+      sum = sum + s1;
     }
   }
-  const float* ct = a.cos_t + (uint64_t)(pos < a.context ? pos : 0) * 64;
-  const float* st = a.sin_t + (uint64_t)(pos < a.context ? pos : 0) * 64;
+  return sum;
+}
+
+// Dims 8 g .. 8 g + 7 and the same + 64 of a staged head x: normalized with
+// inv and rotated (query heads 0 .. qh - 1, to q_out; key heads qh ..
+// qh + kvh - 1, to the row's KV slot) or copied (value heads, to the slot).
+// Returns whether an output is nonfinite (value heads are not checked).
+__device__ __forceinline__ bool qknorm_rope_kv_piece(const uint32_t* x, uint32_t g, float inv, uint32_t row,
+                                                     uint32_t head, const QkvRopeArgs& a, const QkvRowSlot rs) {
+  const uint32_t heads = a.qh + a.kvh;
+  qk_u32x4 xa = *reinterpret_cast<const qk_u32x4*>(x + 4 * g), xb = *reinterpret_cast<const qk_u32x4*>(x + 32 + 4 * g);
+  uint16_t* dst = nullptr;
+  bool bad = false;
+  if (head >= heads) {
+    if (rs.slot_ok) dst = a.v_cache + ((uint64_t)rs.slot + (head - heads)) * 128;
+  } else {
+    if (head < a.qh)
+      dst = a.q_out + ((uint64_t)row * a.qh + head) * 128;
+    else if (rs.slot_ok)
+      dst = a.k_cache + ((uint64_t)rs.slot + (head - a.qh)) * 128;
+    const uint16_t* wn = head < a.qh ? a.q_norm : a.k_norm;
+    const qk_u32x4 wa = *reinterpret_cast<const qk_u32x4*>(wn + 8 * g);
+    const qk_u32x4 wb = *reinterpret_cast<const qk_u32x4*>(wn + 64 + 8 * g);
+    const uint64_t trig = (uint64_t)(rs.pos < a.context ? rs.pos : 0) * 64 + 8 * g;
+    const float4* ct = reinterpret_cast<const float4*>(a.cos_t + trig);
+    const float4* st = reinterpret_cast<const float4*>(a.sin_t + trig);
+    const float4 c0 = ct[0], c1 = ct[1], s0 = st[0], s1 = st[1];
+    const float cs[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+    const float sn[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
 #pragma unroll
-  for (int i = 0; i < 32; ++i) {
-    if (i % kHoist == 0) __builtin_amdgcn_sched_barrier(0);  // bounds how many cos/sin loads are hoisted
-    const float2 c = *reinterpret_cast<const float2*>(ct + 2 * i);
-    const float2 sn = *reinterpret_cast<const float2*>(st + 2 * i);
-    const float a0 = lo_bf16(x[i]), a1 = hi_bf16(x[i]);
-    const float b0 = lo_bf16(x[i + 32]), b1 = hi_bf16(x[i + 32]);
-    const float a0c = a0 * c.x, b0s = b0 * sn.x, b0c = b0 * c.x, a0s = a0 * sn.x;
-    const float a1c = a1 * c.y, b1s = b1 * sn.y, b1c = b1 * c.y, a1s = a1 * sn.y;
-    const uint32_t ra0 = f32_to_bf16(a0c - b0s);
-    const uint32_t rb0 = f32_to_bf16(b0c + a0s);
-    const uint32_t ra1 = f32_to_bf16(a1c - b1s);
-    const uint32_t rb1 = f32_to_bf16(b1c + a1s);
-    bad |= ((ra0 & 0x7f80u) == 0x7f80u) | ((rb0 & 0x7f80u) == 0x7f80u) | ((ra1 & 0x7f80u) == 0x7f80u) |
-           ((rb1 & 0x7f80u) == 0x7f80u);
-    x[i] = ra0 | (ra1 << 16);
-    x[i + 32] = rb0 | (rb1 << 16);
+    for (int k = 0; k < 4; ++k) {
+      uint32_t oa[2], ob[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const float an = bf16_to_f32(norm_weight_bf16(e ? hi_bf16(xa[k]) : lo_bf16(xa[k]), inv,
+                                                      e ? hi_bf16(wa[k]) : lo_bf16(wa[k])));
+        const float bn = bf16_to_f32(norm_weight_bf16(e ? hi_bf16(xb[k]) : lo_bf16(xb[k]), inv,
+                                                      e ? hi_bf16(wb[k]) : lo_bf16(wb[k])));
+        const float c = cs[2 * k + e], s = sn[2 * k + e];
+        const float a_cos = an * c, b_sin = bn * s, b_cos = bn * c, a_sin = an * s;
+        oa[e] = f32_to_bf16(a_cos - b_sin);
+        ob[e] = f32_to_bf16(b_cos + a_sin);
+        bad |= ((oa[e] & 0x7f80u) == 0x7f80u) | ((ob[e] & 0x7f80u) == 0x7f80u);
+      }
+      xa[k] = oa[0] | (oa[1] << 16);
+      xb[k] = ob[0] | (ob[1] << 16);
+    }
   }
-  qk_u32x4* dst = nullptr;
-  if (head < a.qh)
-    dst = reinterpret_cast<qk_u32x4*>(a.q_out + ((uint64_t)row * a.qh + head) * 128);
-  else if (slot_ok)
-    dst = reinterpret_cast<qk_u32x4*>(a.k_cache + ((uint64_t)slot + (head - a.qh)) * 128);
   if (dst) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) dst[i] = qk_u32x4{x[4 * i], x[4 * i + 1], x[4 * i + 2], x[4 * i + 3]};
+    *reinterpret_cast<qk_u32x4*>(dst + 8 * g) = xa;
+    *reinterpret_cast<qk_u32x4*>(dst + 64 + 8 * g) = xb;
+  }
+  return bad;
+}
+
+// kRows (16, 32 or 64) consecutive rows of one head, staged in LDS by this
+// wave (or behind a barrier): lane l < kRows adds row l's squares, then 8
+// lanes per row normalize, rotate and store whole 16-byte pieces, 8 rows at a
+// time. rs: lane l's row row0 + l. One lane per row for everything stored 256
+// bytes per lane and, in the kernels whose waves share a head's rows, left
+// half of the waves or more idle. us per launch of the fused projection with
+// one lane per row / this: 8000 rows of the 8B 372 / 333 (256 x 256 blocks),
+// 777 rows 64.6 / 60.5 (256 x 128), 0.6B 1200 rows 26.9 / 22.0, 509 rows 18.1
+// / 13.6 (128 x 64); bit-identical.
+template <int kRows>
+__device__ __forceinline__ void qknorm_rope_kv_wave(const uint32_t* staged, uint32_t row0, uint32_t m, uint32_t head,
+                                                    const QkvRopeArgs& a, const QkvRowSlot rs) {
+  const uint32_t lane = threadIdx.x & 63u, count = row0 < m ? min(m - row0, (uint32_t)kRows) : 0u;
+  const bool own = lane < count;
+  float inv = 0.f;
+  bool bad = false;
+  if (own && !rs.slot_ok && head == 0) raise_error(a.err, ERR_PAGE);
+  if (head < a.qh + a.kvh && own) {
+    const float sum = qk_square_sum(staged + lane * kQkPitch);
+    inv = inverse_rms(sum, 128.0f, a.eps);
+    // (A nonfinite element makes the sum nonfinite.)
+    bad = !is_finite_f32(sum) | !is_finite_f32(inv);
+  }
+#pragma unroll 4
+  for (uint32_t i = 0; i < kRows / 8; ++i) {
+    const uint32_t r = 8 * i + (lane >> 3);
+    const float inv_r = __shfl(inv, (int)r);
+    const QkvRowSlot rs_r{(uint32_t)__shfl((int)rs.pos, (int)r), (uint32_t)__shfl((int)rs.slot, (int)r),
+                          __shfl((int)rs.slot_ok, (int)r) != 0};
+    if (r < count) bad |= qknorm_rope_kv_piece(staged + r * kQkPitch, lane & 7u, inv_r, row0 + r, head, a, rs_r);
   }
   if (bad) raise_error(a.err, ERR_NONFINITE);
 }

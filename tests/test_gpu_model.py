@@ -736,7 +736,7 @@ def test_prefill_chunk_8b_fused_qkv_epilogue():
     _prefill_case(cfg, limits, [150, 140], [100, 3000], 512, 43, "prefill 8b fused qkv")
 
 
-@pytest.mark.parametrize("prompts", [[270, 160], [300, 221, 200]])
+@pytest.mark.parametrize("prompts", [[270, 160], [300, 221, 200], [257], [264]])
 def test_prefill_chunk_8b_fused_qkv_epilogue_of_mid_sized_blocks(prompts):
     # 8B layer geometry, one layer: at 431 rows the QKV projection runs 128 x
     # 128 blocks (one head each, the last with 47 valid rows), at 722 rows the
