@@ -52,6 +52,7 @@ inline uint64_t attn_records(uint32_t rows, uint32_t query_heads, uint32_t conte
 inline uint64_t attn_records_up_to(uint32_t rows, uint32_t query_heads, uint32_t context_tokens) {
   const uint64_t own = attn_records(rows, query_heads, context_tokens);
   const uint64_t per_row = (uint64_t)query_heads * attn_max_splits(context_tokens, kAttnMinSplitPages);
+  if (per_row == 0) return 0;
   const uint32_t small = (uint32_t)(kAttnSmallPartitions / per_row);
   if (small == 0 || small >= rows) return own;
   const uint64_t fewer = attn_records(small, query_heads, context_tokens);

@@ -127,6 +127,12 @@ def test_attention_scratch_of_a_batch_serves_every_smaller_one():
     assert lib.fh_attention_scratch_bytes(16, 32, 2048) == 16 * 32 * 4 * 130 * 4  # 32-page ones
 
 
+def test_attention_scratch_of_nothing_is_nothing():
+    lib = ferric_amd.load()
+    for sizes in [(0, 32, 2048), (4, 0, 2048), (4, 32, 0), (0, 0, 0)]:
+        assert lib.fh_attention_scratch_bytes(*sizes) == 0
+
+
 def test_ops_reject_bad_shapes_before_any_launch():
     lib = ferric_amd.load()
     p = ctypes.c_void_p(16)  # never dereferenced: validation fails first
