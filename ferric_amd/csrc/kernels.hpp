@@ -42,21 +42,24 @@ inline uint32_t attn_split_pages(uint32_t rows, uint32_t query_heads, uint32_t c
   const uint64_t partitions = (uint64_t)rows * query_heads * attn_max_splits(context_tokens, kAttnMinSplitPages);
   return partitions <= kAttnSmallPartitions ? kAttnMinSplitPages : kAttnMaxSplitPages;
 }
-// Partition records of a launch, and the most that any launch of at most
-// `rows` rows needs (16-page partitions of a few rows can outnumber 32-page
-// ones of more).
+// Partition records of a launch.
 inline uint64_t attn_records(uint32_t rows, uint32_t query_heads, uint32_t context_tokens) {
   return (uint64_t)rows * query_heads *
          attn_max_splits(context_tokens, attn_split_pages(rows, query_heads, context_tokens));
 }
+// Records enough for every launch of at most `rows` rows and `context_tokens`
+// tokens: those of this launch at 32-page partitions, or what a smaller one
+// can need at 16-page partitions, which the rule allows up to
+// kAttnSmallPartitions of them (8 rows of 32 heads: 960 records at 1280
+// tokens, 1024 at 1024 tokens). Up to 512 tokens every row is one partition,
+// and at most 16 heads take 16-page partitions at every other size.
 inline uint64_t attn_records_up_to(uint32_t rows, uint32_t query_heads, uint32_t context_tokens) {
   const uint64_t own = attn_records(rows, query_heads, context_tokens);
-  const uint64_t per_row = (uint64_t)query_heads * attn_max_splits(context_tokens, kAttnMinSplitPages);
-  if (per_row == 0) return 0;
-  const uint32_t small = (uint32_t)(kAttnSmallPartitions / per_row);
-  if (small == 0 || small >= rows) return own;
-  const uint64_t fewer = attn_records(small, query_heads, context_tokens);
-  return own > fewer ? own : fewer;
+  if (query_heads <= 16 || context_tokens <= kAttnMaxSplitPages * 16) return own;
+  const uint64_t large = (uint64_t)rows * query_heads * attn_max_splits(context_tokens, kAttnMaxSplitPages);
+  const uint64_t small = (uint64_t)rows * query_heads * attn_max_splits(context_tokens, kAttnMinSplitPages);
+  const uint64_t most_small = small < kAttnSmallPartitions ? small : kAttnSmallPartitions;
+  return large > most_small ? large : most_small;
 }
 // Floats per attention partial record: running max, denominator, numerator[128].
 constexpr uint32_t kAttnPartialFloats = 2 + 128;

@@ -308,7 +308,8 @@ fh_status fh_op_qknorm_rope_kv(const void* qkv, uint32_t qkv_splits, const uint1
 /* K4 paged GQA decode attention: split-context partitions then an ordered merge.
  * q: [rows][qh*128]; out: [rows][qh*128] bf16 row-major, or activation tile order when
  * out_tiled (the output projection's input, fh_activation_rows(rows) rows);
- * scratch: fh_attention_scratch_bytes(), enough for every call of at most `rows` rows.
+ * scratch: fh_attention_scratch_bytes(), enough for every call of at most `rows` rows and
+ * `context_tokens` tokens (same query heads).
  * Replaces qwen3_paged_gqa_decode_bf16_f32_v1 (paged_decode.rs:222) and the split8
  * partial/merge pair (device/qwen3-tp-c1-split8-attention-kernels-v21/src/attention.rs:16, :214). */
 uint64_t fh_attention_scratch_bytes(uint32_t rows, uint32_t query_heads, uint32_t context_tokens);
