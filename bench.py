@@ -102,13 +102,15 @@ def copy_probe(mib):
     print(json.dumps({"copy_probe_bytes_read": n, "copy_probe_bytes_written": n, "copies": 4}), flush=True)
 
 
-def attn_partition_tokens(rows, query_heads, context_tokens):
-    """Tokens per decode attention partition: 32 pages of 16, or 16 pages
-    when the launch has at most 1024 such partitions at the context capacity
-    or at most 16 query heads (the library's attn_split_pages)."""
+def attn_partition_tokens(rows, query_heads, kv_heads, context_tokens):
+    """Tokens per decode attention partition: 32 pages of 16, or 16 pages for
+    at most 16 query heads, at most 64 (row, query head) pairs or a launch of
+    few such partitions at the context capacity (the library's
+    attn_split_pages)."""
     if 256 < context_tokens <= 512:
         return 512
-    return 256 if query_heads <= 16 or rows * query_heads * -(-context_tokens // 256) <= 1024 else 512
+    partitions = rows * max(query_heads, 4 * kv_heads) * -(-context_tokens // 256)
+    return 256 if query_heads <= 16 or rows * query_heads <= 64 or partitions <= 1024 else 512
 
 
 def kernel_bytes(cfg, rows, positions, stride):
@@ -120,7 +122,7 @@ def kernel_bytes(cfg, rows, positions, stride):
     kv_read = int(np.sum(ctx)) * KV * 2 * 2  # K and V rows, bf16
     # Rows longer than one partition leave one FP32 record (max, denominator,
     # 128 numerators) per query head and partition.
-    tokens = attn_partition_tokens(rows, QH, stride * 16)
+    tokens = attn_partition_tokens(rows, QH, KVH, stride * 16)
     parts = (ctx + tokens - 1) // tokens
     merge_read = int(np.sum(np.where(parts > 1, parts, 0))) * QH * 130 * 4
     merged_rows = int(np.sum(parts > 1))

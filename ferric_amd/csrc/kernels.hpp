@@ -13,53 +13,59 @@ namespace fh {
 void set_thread_error(const char* msg);
 
 // Attention partitions: each partition workgroup covers split_pages pages of
-// 16 tokens (16 or 32; its 8 waves take split_pages / 8 pages each). Launches
-// of at most 256 workgroups of 16 pages at the context capacity (1024
-// partitions of a (row, query head) at 4 query heads per KV head) and models
-// of at most 16 query heads (2 per KV head in Qwen3-0.6B, half the work per
-// page of the 8B's 4) take 16-page partitions: with CUs idle anyway a wave's
-// chain over 2 pages is shorter than over 4. Measured on MI355X, us per
-// attention at 16 / 32 pages, 8B heads: 1 row of 4096 tokens 11.9 / 15.3, 4
-// rows at U[300, 2048] of a 2048-token capacity 12.0 / 15.3, 8 rows at U[200,
-// 1000] of 1024 11.8 / 15.2; beyond: 2 rows at U[512, 8192] of 8192 19.8 /
-// 16.1, 8 rows at U[300, 2048] 17.2 / 16.3, 32 rows at U[512, 8192] 149 / 129.
-// 32 rows of the 0.6B, contexts U[128, 2048]: 0.866 against 0.933 ms per step
-// with 32 (2.04 against 2.12 ms per step). A context capacity of 257..512
-// tokens takes one 32-page partition whatever the batch, so every row finishes
-// in its partition with no records and no merge (a speculative round's 0.6B
-// draft, 32 rows at 256-410 tokens of a 512-token capacity: 14.4 -> 11.8 us
-// per launch, 1.155 -> 1.112 ms device time per step). attn_split_pages is the
-// one policy every launcher and workspace size uses.
+// 16 tokens (16 or 32; its 8 waves take split_pages / 8 pages each). 16 pages
+// where CUs are idle anyway, so that a wave's chain is 2 pages, not 4:
+//  * at most 64 (row, query head) pairs, whatever the context capacity: a few
+//    rows' contexts are mostly far below a large capacity, and then their
+//    chain is what counts. us per attention at 16 / 32 pages, 8B heads, 2 rows
+//    at a 16384-token capacity: 2000 tokens 15.4 / 22.1, 8000 22.9 / 23.5,
+//    16000 35.2 / 32.7; 1 row at 32768: 2000 tokens 14.5 / 21.6, 30000 41.3 /
+//    34.5 (decode steps of 4 layers: 393 / 413 and 520 / 475).
+//  * launches of at most 256 workgroups of 16 pages at the context capacity
+//    and at most 1024 partitions of a (row, query head): 8B heads, 4 rows of a
+//    2048-token capacity 12.0 / 15.3, 8 rows of 1024 11.8 / 15.2; beyond, 8
+//    rows at U[300, 2048] of 2048 17.2 / 16.3, 32 rows at U[512, 8192] 149 /
+//    129; 32 heads of 1 per KV head, 8 rows of 1024 (1024 workgroups) at 300
+//    tokens 21.4 / 15.6.
+//  * models of at most 16 query heads (2 per KV head in Qwen3-0.6B, half the
+//    work per page of the 8B's 4): 32 rows of the 0.6B, contexts U[128, 2048]:
+//    0.866 against 0.933 ms per step with 32 (2.04 against 2.12 ms per step).
+// A context capacity of 257..512 tokens takes one 32-page partition whatever
+// the batch, so every row finishes in its partition with no records and no
+// merge (a speculative round's 0.6B draft, 32 rows at 256-410 tokens of a
+// 512-token capacity: 14.4 -> 11.8 us per launch, 1.155 -> 1.112 ms device
+// time per step). attn_split_pages is the one policy every launcher and
+// workspace size uses.
 constexpr uint32_t kAttnMaxSplitPages = 32;
 constexpr uint32_t kAttnMinSplitPages = 16;
+constexpr uint32_t kAttnFewPairs = 64;
 constexpr uint32_t kAttnSmallPartitions = 1024;
 inline uint32_t attn_max_splits(uint32_t context_tokens, uint32_t split_pages) {
   return (context_tokens + split_pages * 16 - 1) / (split_pages * 16);
 }
-inline uint32_t attn_split_pages(uint32_t rows, uint32_t query_heads, uint32_t context_tokens) {
+inline uint32_t attn_split_pages(uint32_t rows, uint32_t query_heads, uint32_t kv_heads, uint32_t context_tokens) {
   if (context_tokens > kAttnMinSplitPages * 16 && context_tokens <= kAttnMaxSplitPages * 16) return kAttnMaxSplitPages;
-  if (query_heads <= 16) return kAttnMinSplitPages;
-  const uint64_t partitions = (uint64_t)rows * query_heads * attn_max_splits(context_tokens, kAttnMinSplitPages);
-  return partitions <= kAttnSmallPartitions ? kAttnMinSplitPages : kAttnMaxSplitPages;
+  if (query_heads <= 16 || (uint64_t)rows * query_heads <= kAttnFewPairs) return kAttnMinSplitPages;
+  const uint64_t heads = query_heads > 4 * kv_heads ? query_heads : 4 * kv_heads;
+  return rows * heads * attn_max_splits(context_tokens, kAttnMinSplitPages) <= kAttnSmallPartitions ? kAttnMinSplitPages
+                                                                                                 : kAttnMaxSplitPages;
 }
-// Partition records of a launch.
-inline uint64_t attn_records(uint32_t rows, uint32_t query_heads, uint32_t context_tokens) {
-  return (uint64_t)rows * query_heads *
-         attn_max_splits(context_tokens, attn_split_pages(rows, query_heads, context_tokens));
-}
-// Records enough for every launch of at most `rows` rows and `context_tokens`
-// tokens: those of this launch at 32-page partitions, or what a smaller one
-// can need at 16-page partitions, which the rule allows up to
-// kAttnSmallPartitions of them (8 rows of 32 heads: 960 records at 1280
-// tokens, 1024 at 1024 tokens). Up to 512 tokens every row is one partition,
-// and at most 16 heads take 16-page partitions at every other size.
+// Partition records enough for every launch of at most `rows` rows and
+// `context_tokens` tokens: those of this launch at 32-page partitions, or what
+// a smaller one can need at 16-page partitions, which the rule allows to a few
+// rows and up to kAttnSmallPartitions of them (8 rows of 32 heads: 960 records
+// at 1280 tokens, 1024 at 1024 tokens). Up to 512 tokens every row is one
+// partition, and at most 16 heads take 16-page partitions at every other size.
 inline uint64_t attn_records_up_to(uint32_t rows, uint32_t query_heads, uint32_t context_tokens) {
-  const uint64_t own = attn_records(rows, query_heads, context_tokens);
-  if (query_heads <= 16 || context_tokens <= kAttnMaxSplitPages * 16) return own;
+  const bool one = context_tokens <= kAttnMaxSplitPages * 16;
   const uint64_t large = (uint64_t)rows * query_heads * attn_max_splits(context_tokens, kAttnMaxSplitPages);
   const uint64_t small = (uint64_t)rows * query_heads * attn_max_splits(context_tokens, kAttnMinSplitPages);
-  const uint64_t most_small = small < kAttnSmallPartitions ? small : kAttnSmallPartitions;
-  return large > most_small ? large : most_small;
+  if (one || query_heads <= 16) return one ? large : small;
+  const uint32_t few_rows = kAttnFewPairs / query_heads < rows ? kAttnFewPairs / query_heads : rows;
+  const uint64_t few = (uint64_t)few_rows * query_heads * attn_max_splits(context_tokens, kAttnMinSplitPages);
+  uint64_t most = small < kAttnSmallPartitions ? small : kAttnSmallPartitions;
+  if (few > most) most = few;
+  return large > most ? large : most;
 }
 // Floats per attention partial record: running max, denominator, numerator[128].
 constexpr uint32_t kAttnPartialFloats = 2 + 128;

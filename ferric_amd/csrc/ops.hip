@@ -212,12 +212,8 @@ fh_status fh_op_paged_attention_noalloc(const uint16_t* q, const uint16_t* k_cac
     return FH_ERR_INVALID_ARGUMENT;
   const uint32_t g = query_heads / kv_heads;
   if (g != 1 && g != 2 && g != 4 && g != 8) return FH_ERR_INVALID_ARGUMENT;
-  const uint32_t split_pages = fh::attn_split_pages(rows, query_heads, context_tokens);
-  // Up to 64 (row, query head) pairs are counted at 16-page partitions, also
-  // where the launch takes 32: the limit stays where callers know it.
-  const uint64_t pairs = (uint64_t)rows * query_heads;
-  const uint64_t records = pairs <= 64 ? pairs * fh::attn_max_splits(context_tokens, fh::kAttnMinSplitPages)
-                                       : fh::attn_records(rows, query_heads, context_tokens);
+  const uint32_t split_pages = fh::attn_split_pages(rows, query_heads, kv_heads, context_tokens);
+  const uint64_t records = (uint64_t)rows * query_heads * fh::attn_max_splits(context_tokens, split_pages);
   if (records > kNoAllocAttnRecords) {
     fh::set_thread_error("fh_op_paged_attention_noalloc: rows x query_heads x partitions of the context exceeds "
                          "the 16384 partition records of its static array");
@@ -254,7 +250,7 @@ fh_status fh_op_qknorm_paged_attention(const float* qkv_partials, uint32_t qkv_s
     return FH_ERR_INVALID_ARGUMENT;
   hipStream_t s = as_stream(stream);
   float* part = reinterpret_cast<float*>(scratch);
-  const uint32_t split_pages = fh::attn_split_pages(rows, query_heads, context_tokens);
+  const uint32_t split_pages = fh::attn_split_pages(rows, query_heads, kv_heads, context_tokens);
   const fh::AttnQkn qa{qkv_partials, qkv_splits, fh::partial_slab_rows(rows), q_norm, k_norm, cos_table, sin_table,
                        k_cache,      v_cache,    epsilon};
   (void)hipGetLastError();
@@ -280,7 +276,7 @@ fh_status fh_op_paged_attention(const uint16_t* q, const uint16_t* k_cache, cons
   if (g != 1 && g != 2 && g != 4 && g != 8) return FH_ERR_INVALID_ARGUMENT;
   hipStream_t s = as_stream(stream);
   float* part = reinterpret_cast<float*>(scratch);
-  const uint32_t split_pages = fh::attn_split_pages(rows, query_heads, context_tokens);
+  const uint32_t split_pages = fh::attn_split_pages(rows, query_heads, kv_heads, context_tokens);
   (void)hipGetLastError();
   hipError_t e = fh::launch_attention_partial(q, k_cache, v_cache, positions, page_table, part, out, out_tiled, 0,
                                               rows, rows, query_heads, kv_heads, stride, physical_pages,

@@ -127,9 +127,10 @@ def test_attention_scratch_of_a_batch_serves_every_smaller_one():
     assert lib.fh_attention_scratch_bytes(16, 32, 2048) == 16 * 32 * 4 * 130 * 4  # 32-page ones
 
 
-def launch_records(rows, heads, context):
+def launch_records(rows, heads, kv_heads, context):
     """Partition records one decode attention launch writes (the partition rule of fh_op_paged_attention_noalloc)."""
-    pages = 32 if 256 < context <= 512 or (heads > 16 and rows * heads * -(-context // 256) > 1024) else 16
+    small = heads <= 16 or rows * heads <= 64 or rows * max(heads, 4 * kv_heads) * -(-context // 256) <= 1024
+    pages = 32 if 256 < context <= 512 or not small else 16
     return rows * heads * -(-context // (16 * pages))
 
 
@@ -139,12 +140,20 @@ def test_attention_scratch_serves_every_smaller_batch_and_context(heads):
     # rows may: 8 rows of 32 heads need 1024 records at 1024 tokens, 960 at 1280.
     lib = ferric_amd.load()
     contexts = [1, 255, 256, 257, 511, 512, 513] + [c + d for c in range(768, 40961, 256) for d in (0, 1)]
-    need = np.array([[launch_records(rows, heads, c) for c in contexts] for rows in range(1, 33)])
+    need = np.max([[[launch_records(rows, heads, heads // g, c) for c in contexts] for rows in range(1, 33)]
+                   for g in (1, 2, 4, 8) if heads % g == 0], axis=0)
     most = np.maximum.accumulate(np.maximum.accumulate(need, axis=0), axis=1)
     got = np.array([[lib.fh_attention_scratch_bytes(rows, heads, c) for c in contexts] for rows in range(1, 33)])
     assert (got >= most * 130 * 4).all()
     # ... and the largest batch at the largest context is not asked for more than it needs itself.
     assert got[-1, -1] == need[-1, -1] * 130 * 4
+
+
+def test_attention_scratch_of_a_few_rows_is_that_of_small_partitions():
+    # At most 64 (row, query head) pairs take 256-token partitions at every capacity above 512 tokens.
+    lib = ferric_amd.load()
+    for rows, heads, context in [(1, 32, 40960), (2, 32, 8192), (2, 32, 16384), (1, 64, 32768), (3, 20, 24576)]:
+        assert lib.fh_attention_scratch_bytes(rows, heads, context) == rows * heads * context // 256 * 130 * 4
 
 
 def test_attention_scratch_of_nothing_is_nothing():

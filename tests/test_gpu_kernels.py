@@ -894,12 +894,15 @@ def test_qknorm_rope_kv_of_many_rows_bit_exact(qh, kvh, rows):
 
 
 # The two partition sizes on either side of their rule (16 pages up to 1024
-# partitions of a (row, query head) at the context capacity): the last launch
-# of 16-page partitions, the first of 32, capacities one token past a multiple.
-@pytest.mark.parametrize("rows,context", [(4, 2048), (5, 2048), (8, 1024), (9, 1024), (1, 8192), (1, 8193), (3, 2305)])
-def test_paged_attention_partition_rule(rows, context):
+# partitions of a (row, query head) and 256 workgroups at the context capacity,
+# and for up to 64 pairs): the last launch of 16-page partitions, the first of
+# 32, capacities one token past a multiple; 1 and 2 query heads per KV head.
+@pytest.mark.parametrize("rows,context,kvh", [(4, 2048, 8), (5, 2048, 8), (8, 1024, 8), (9, 1024, 8), (1, 8192, 8),
+                                              (1, 8193, 8), (3, 2305, 8), (2, 16384, 8), (2, 1025, 32), (3, 513, 32),
+                                              (4, 1024, 16), (5, 1024, 16)])
+def test_paged_attention_partition_rule(rows, context, kvh):
     r = rng(rows + context)
-    qh, kvh, stride = 32, 8, (context + 15) // 16
+    qh, stride = 32, (context + 15) // 16
     pages = stride + 5
     kc, vc = _paged_pool(r, pages, kvh)
     q = rand_bf16(r, rows * qh * 128, 1.0)
