@@ -339,15 +339,15 @@ bool band_ok(uint32_t m, uint32_t n, uint32_t k) { return m > kMaxRows && n % kB
 }  // namespace
 
 // Estimated microseconds of a launch (fitted with mid_cost, k_gemm_mid.hip):
-// rounds of the 256 CUs in units of a full block; a last block of at most 64
-// rows takes about a third of one (its weight fetch).
+// rounds of the 256 CUs in units of a full block, at least one; a last block of
+// at most 64 rows takes about a third of one (its weight fetch).
 float gemm_band_cost(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue) {
   if (!band_ok(m, n, k)) return -1.f;
   const uint32_t tail = m % kLargeBlockRows;
   const float part = tail == 0 ? 0.f : tail <= 64 ? 0.35f : (tail + 63) / 64 * 0.25f;
   const float blocks = (n / kBandCols) * (m / kLargeBlockRows + part);
   const float around = epilogue == FH_EPI_SWIGLU ? 5.9f : 4.9f;
-  return 2.4f + floorf((blocks + 255.f) / 256.f) * (around + (k / 32) * 0.41f);
+  return 2.4f + ceilf(blocks / 256.f) * (around + (k / 32) * 0.41f);
 }
 
 hipError_t launch_gemm_band(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_t m, uint32_t n, uint32_t k,

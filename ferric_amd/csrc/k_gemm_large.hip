@@ -293,6 +293,22 @@ bool panel_streams(uint32_t m, uint32_t n) { return m <= 224 && n > 128 * kPanel
 
 }  // namespace
 
+uint32_t gemm_block(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, bool fused_qkv) {
+  if (m <= kMaxRows || n == 0 || n % kPanelCols != 0 || k == 0 || k % 32 != 0) return 0;
+  if (fused_qkv) {
+    if (m <= kPanelRows || n % (16 * kBigTiles) != 0) return 0;
+  } else if (epilogue > FH_EPI_F32 ||
+             ((epilogue == FH_EPI_SWIGLU || epilogue == FH_EPI_F32) && panel_streams(m, n))) {
+    return 0;
+  }
+  switch (pick_kernel(m, n, k, fused_qkv ? (uint32_t)FH_EPI_BF16 : epilogue, fused_qkv)) {
+    case LargeKernel::kMid: return gemm_mid_block(m, n, k, fused_qkv);
+    case LargeKernel::kBand: return kLargeBlockRows << 16 | kPanelCols;
+    case LargeKernel::kBlock: break;
+  }
+  return (16 * kBigTiles) << 16 | 16 * kBigTiles;
+}
+
 hipError_t launch_gemm_qkv_rope(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_t m, uint32_t n, uint32_t k,
                                 const QkvRopeArgs& qa, hipStream_t s) {
   const uint32_t mtiles = act_mtiles(m);

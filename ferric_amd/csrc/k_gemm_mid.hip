@@ -344,6 +344,12 @@ float gemm_mid_cost(uint32_t m, uint32_t n, uint32_t k, bool whole_heads) {
              : -1.f;
 }
 
+uint32_t gemm_mid_block(uint32_t m, uint32_t n, uint32_t k, bool whole_heads) {
+  MidShape v{};
+  float cost = 0.f;
+  return mid_pick(m, n, k, whole_heads, &v, &cost) ? (32 * v.tm) << 16 | 32 * v.tn : 0u;
+}
+
 hipError_t launch_gemm_mid(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_t m, uint32_t n, uint32_t k,
                            uint32_t epilogue, const uint16_t* residual, void* out, uint32_t ldo, uint32_t* err,
                            hipStream_t s) {

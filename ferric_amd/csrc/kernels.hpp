@@ -157,10 +157,14 @@ hipError_t launch_swiglu(const uint16_t* gate, const uint16_t* up, uint16_t* out
 hipError_t launch_gemm_large(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_t m, uint32_t n, uint32_t k,
                              uint32_t epilogue, const uint16_t* residual, void* out, uint32_t ldo, uint32_t* err,
                              hipStream_t s);
+// The block of launch_gemm_large (fused_qkv: launch_gemm_qkv_rope), rows << 16
+// | columns; 0 where the weight is streamed or the shape is not supported.
+uint32_t gemm_block(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, bool fused_qkv);
 // Mid-sized batches (k_gemm_mid.hip): m > kMaxRows, n % 32 == 0, the same
 // operands as launch_gemm_large. gemm_mid_cost estimates the launch's
 // microseconds (whole_heads: the QKV form), negative where it has no form.
 float gemm_mid_cost(uint32_t m, uint32_t n, uint32_t k, bool whole_heads);
+uint32_t gemm_mid_block(uint32_t m, uint32_t n, uint32_t k, bool whole_heads);
 hipError_t launch_gemm_mid(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_t m, uint32_t n, uint32_t k,
                            uint32_t epilogue, const uint16_t* residual, void* out, uint32_t ldo, uint32_t* err,
                            hipStream_t s);

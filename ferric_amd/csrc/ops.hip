@@ -89,6 +89,10 @@ fh_status fh_op_gemm(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_t 
                                             as_stream(stream)));
 }
 
+uint32_t fh_gemm_block(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, uint32_t fused_qkv) {
+  return fh::gemm_block(m, n, k, epilogue, fused_qkv != 0);
+}
+
 uint32_t fh_activation_rows(uint32_t m) { return m ? fh::act_mtiles(m) * 16 : 0u; }
 
 uint32_t fh_gemm_default_splits(uint32_t n, uint32_t k) { return fh::gemm_default_splits(n, k); }

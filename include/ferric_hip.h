@@ -254,6 +254,10 @@ fh_status fh_op_gemm(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_t 
                      uint32_t* error_word, void* stream);
 /* Split-K factor the runtime uses for an n x k projection. */
 uint32_t fh_gemm_default_splits(uint32_t n, uint32_t k);
+/* Output block of the compute-bound kernel that fh_op_gemm (or, with fused_qkv, a prefill
+ * chunk's QKV projection with QK-norm, RoPE and KV append inside, epilogue ignored) takes for
+ * m > 32: rows << 16 | columns; 0 where the weight is streamed or the shape refused. */
+uint32_t fh_gemm_block(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, uint32_t fused_qkv);
 /* Rows a tiled activation buffer for m rows holds: 32 for m <= 32, else m rounded up to 256. */
 uint32_t fh_activation_rows(uint32_t m);
 /* Rows of one FH_EPI_PARTIAL slab for an m-row batch: 32 for m <= 32, 256 for 32 < m <= 256,

@@ -162,6 +162,23 @@ def test_attention_scratch_of_nothing_is_nothing():
         assert lib.fh_attention_scratch_bytes(*sizes) == 0
 
 
+def block(m, n, k, epilogue=_lib.EPI_BF16, fused_qkv=0):
+    b = ferric_amd.load().fh_gemm_block(m, n, k, epilogue, fused_qkv)
+    return b >> 16, b & 0xffff
+
+
+def test_narrow_projections_take_blocks_that_split_k():
+    # One or two 256-row x 128-column blocks would walk all of k on one or two
+    # CUs: weights of 128 and 256 rows take the small blocks, whose waves split k.
+    for n in (128, 256):
+        for m in range(33, 257):
+            for k in (64, 512, 1024, 2560, 4096, 12288):
+                for epilogue in (_lib.EPI_BF16, _lib.EPI_RESIDUAL, _lib.EPI_SWIGLU, _lib.EPI_F32):
+                    assert block(m, n, k, epilogue) < (256, 128), (m, n, k, epilogue)
+    assert block(40, 120, 64) == block(40, 128, 48) == block(32, 128, 64) == block(40, 128, 64, _lib.EPI_PARTIAL) == (0, 0)
+    assert block(300, 384, 1024, fused_qkv=1) == block(256, 256, 1024, fused_qkv=1) == (0, 0)  # not fused there
+
+
 def test_ops_reject_bad_shapes_before_any_launch():
     lib = ferric_amd.load()
     p = ctypes.c_void_p(16)  # never dereferenced: validation fails first
