@@ -127,6 +127,7 @@ SIGNATURES = [
     ("fh_op_gemm", _st, [_vp, _vp, _u32, _u32, _u32, _u32, _u32, _vp, _vp, _u32, _vp, _vp]),
     ("fh_gemm_default_splits", _u32, [_u32, _u32]),
     ("fh_gemm_block", _u32, [_u32] * 5),
+    ("fh_prefill_attention_form", _u32, [ctypes.POINTER(ctypes.c_uint32)] * 2 + [_u32] * 3),
     ("fh_activation_rows", _u32, [_u32]),
     ("fh_partial_slab_rows", _u32, [_u32]),
     ("fh_op_tile_activation", _st, [_vp, _vp, _u32, _u32, _vp]),

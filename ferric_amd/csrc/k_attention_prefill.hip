@@ -1,11 +1,11 @@
 // K4 for prefill chunks of long runs of rows: causal attention of blocks of
 // consecutive rows of one sequence. Same contract as k_attention_block.hip,
-// which keeps the chunks of short blocks (launch_attention_blocks' comment
-// gives the rule): for a row at position p, keys t = 0..p through the row's
+// which keeps the chunks of up to kPanelRows rows and those whose runs of rows
+// are short (attention_prefill_form): for a row at position p, keys t = 0..p through the row's
 // page table, score = (q . k_t) * f32(0x3db504f3), softmax, out = bf16(n / l)
 // (device/qwen3-all-kernels-v1/src/paged_decode.rs:222-572).
 //
-// A workgroup owns one block (128 / G rows; 64 / G or 32 / G in small chunks)
+// A workgroup owns one block (128 / G, 64 / G or 32 / G rows, by the form)
 // and one KV head; a wave owns 32 query vectors (vector j: row j / G, head
 // j % G), and the 4 waves share 64- or 128-key tiles of K and V, fetched global -> LDS directly (buffer
 // loads, 16 bytes per lane, double-buffered). Slots past the block's last
@@ -37,6 +37,7 @@
 // 16-key tiles (k_attention_block.hip) -> this kernel: one 8000-token 8B prompt
 // 2010 -> 775, 32 prompts of 256 tokens 94 -> 64, one of 777 tokens 42 -> 23
 // (29 without the waves along the keys), a 509-token 0.6B prompt 21 -> 13 (18).
+#include <cmath>
 #include <type_traits>
 
 #include "common.hpp"
@@ -345,34 +346,84 @@ __global__ __launch_bounds__(64 * kPreWaves, WK == 4 ? 1 : 2) void attn_prefill_
 
 }  // namespace
 
-// Waves along the keys for a chunk of `rows` rows: as few as give every CU a
-// workgroup (one sequence's rows; several sequences make more, shorter blocks).
-static int prefill_key_waves(uint32_t rows, uint32_t qh, uint32_t kvh) {
-  const uint64_t vectors = (uint64_t)rows * (qh / kvh);
-  for (int wk = 1; wk < 4; wk *= 2)
-    if ((vectors + 128 / wk - 1) / (128 / wk) * kvh >= 256) return wk;
-  return 4;
+namespace {
+
+// What attention_prefill_form needs of each form: keys per tile (short blocks:
+// four pages), workgroups that run at once (0: not a limit by itself), and
+// microseconds per launch, per tile of one workgroup's chain, per workgroup and
+// per tile of all of them (256 CUs), and per tile of each further round.
+struct PrefillForm {
+  uint32_t form, tile, slots;
+  float launch_us, chain_us, group_us, tile_us, round_us;
+};
+constexpr PrefillForm kPrefillForms[] = {{0, 64, 0, 9.0f, 0.f, 0.f, 1.75f, 0.f},
+                                         {1, 64, 512, 8.5f, 1.8f, 0.58f, 1.38f, 2.28f},
+                                         {2, 64, 512, 8.1f, 1.16f, 1.71f, 0.87f, 1.49f},
+                                         {4, 128, 256, 9.6f, 1.56f, 3.36f, 1.74f, 1.84f}};
+
+}  // namespace
+
+// The form with the lowest estimate: the longest workgroup's chain, the work
+// of all of them, or rounds of average ones, whichever is longest. Its
+// constants are fitted to the times of all forms over 840 chunks of 257 to
+// 8000 rows (1 to 2000 sequences of 1 to 4000 rows at contexts of 0 to 7000
+// tokens, alone and mixed; 1, 2, 4 and 8 query heads per KV head): it picks a
+// form 0.4 % slower than the fastest on average, 21 % at most, and never one
+// more than 15 % slower than the short blocks. Waves along the keys by the
+// chunk's rows alone, as before, were 28 % slower than the fastest on average:
+// a chunk of many short runs got long blocks that held a row or two. us per
+// layer by the rows alone / now / short blocks: 0.6B 300 sequences of 1 row 67 /
+// 14 / 14, 8B 300 x 1 68 / 17 / 17, 20 x 16 rows on 7000 tokens 288 / 198 / 191,
+// 10 x 32 on 7000 241 / 181 / 187; 2 x 1000 rows 42 / 33 / 105.
+uint32_t attention_prefill_form(const uint32_t* position, const uint32_t* rows, uint32_t nruns, uint32_t qh,
+                                uint32_t kvh) {
+  uint32_t best = 0;
+  float best_us = 0.f;
+  for (const PrefillForm& f : kPrefillForms) {
+    const uint32_t bq = attention_prefill_block_rows(f.form, qh, kvh);
+    uint64_t groups = 0, tiles = 0;
+    uint32_t longest = 0;
+    for (uint32_t i = 0; i < nruns; ++i)
+      for (uint32_t r = 0; r < rows[i]; r += bq) {
+        const uint32_t last = position[i] + (rows[i] - r < bq ? rows[i] : r + bq) - 1;
+        const uint32_t t = last / f.tile + 1;
+        ++groups;
+        tiles += t;
+        if (t > longest) longest = t;
+      }
+    const float n = (float)(groups * kvh), all = (float)(tiles * kvh), average = all / n;
+    // Short blocks: 4, 2 or 1 page phases (launch_attention_blocks).
+    const float chain = f.form ? f.chain_us : n <= 256.f ? 1.6f : n <= 512.f ? 2.74f : 3.6f;
+    float us = fmaxf(chain * longest, (f.group_us * n + f.tile_us * all) / 256.f);
+    if (f.slots) us = fmaxf(us, average * (chain + (ceilf(n / f.slots) - 1.f) * f.round_us));
+    us += f.launch_us;
+    if (f.form == 0 || us < best_us) {
+      best = f.form;
+      best_us = us;
+    }
+  }
+  return best;
 }
 
-uint32_t attention_prefill_block_rows(uint32_t rows, uint32_t qh, uint32_t kvh) {
-  return 128u / prefill_key_waves(rows, qh, kvh) / (qh / kvh);
+uint32_t attention_prefill_block_rows(uint32_t form, uint32_t qh, uint32_t kvh) {
+  return form ? 128u / form / (qh / kvh) : attention_block_rows(qh, kvh);
 }
 
-hipError_t launch_attention_prefill(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_cache,
-                                    const uint32_t* positions, const uint32_t* table, const uint32_t* blocks,
-                                    uint32_t nblocks, uint16_t* out, uint32_t out_tiled, uint32_t rows, uint32_t qh,
-                                    uint32_t kvh, uint32_t stride, uint32_t pages, uint32_t context, uint32_t* err,
-                                    hipStream_t s) {
+hipError_t launch_attention_prefill(uint32_t form, const uint16_t* q, const uint16_t* k_cache,
+                                    const uint16_t* v_cache, const uint32_t* positions, const uint32_t* table,
+                                    const uint32_t* blocks, uint32_t nblocks, uint16_t* out, uint32_t out_tiled,
+                                    uint32_t rows, uint32_t qh, uint32_t kvh, uint32_t stride, uint32_t pages,
+                                    uint32_t context, uint32_t* err, hipStream_t s) {
   if (nblocks == 0) return hipSuccess;
+  if (form != 1 && form != 2 && form != 4) return hipErrorInvalidValue;
   const uint32_t mt = out_tiled ? act_mtiles(rows) : 0u;
-  const int wk = prefill_key_waves(rows, qh, kvh);
 #define FH_PREFILL_WK(G_, WK_)                                                                            \
   hipLaunchKernelGGL((attn_prefill_kernel<G_, WK_>), dim3(kvh, nblocks), dim3(64 * kPreWaves), 0, s, q,   \
                      k_cache, v_cache, positions, table, blocks, out, mt, qh, kvh, stride, pages, context, err)
 #define FH_PREFILL(G_)         \
-  if (wk == 1)                 \
+  if (form == 1)               \
     FH_PREFILL_WK(G_, 1);      \
-  else if (wk == 2)            \
+  else if (form == 2)          \
     FH_PREFILL_WK(G_, 2);      \
   else                         \
     FH_PREFILL_WK(G_, 4)

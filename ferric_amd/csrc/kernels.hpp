@@ -286,15 +286,20 @@ hipError_t launch_attention_blocks(const uint16_t* q, const uint16_t* k_cache, c
                                    uint32_t qh, uint32_t kvh, uint32_t stride, uint32_t pages, uint32_t context,
                                    uint32_t* err, hipStream_t s, const AttnQkn* qkn = nullptr);
 
-// The same for chunks of long blocks (k_attention_prefill.hip): each block of
-// a chunk of `rows` rows has at most attention_prefill_block_rows(rows, qh,
-// kvh) rows. out has `rows` rows.
-uint32_t attention_prefill_block_rows(uint32_t rows, uint32_t qh, uint32_t kvh);
-hipError_t launch_attention_prefill(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_cache,
-                                    const uint32_t* positions, const uint32_t* table, const uint32_t* blocks,
-                                    uint32_t nblocks, uint16_t* out, uint32_t out_tiled, uint32_t rows, uint32_t qh,
-                                    uint32_t kvh, uint32_t stride, uint32_t pages, uint32_t context, uint32_t* err,
-                                    hipStream_t s);
+// The same with long blocks (k_attention_prefill.hip), for chunks of more than
+// kPanelRows rows. The form of such a chunk's attention is 0 (the short blocks
+// above) or the long blocks' waves along the keys (1, 2 or 4); its blocks have
+// at most attention_prefill_block_rows(form, qh, kvh) rows, cut from nruns runs
+// of rows of one sequence (run i: rows[i] rows from position[i] on). out has
+// `rows` rows.
+uint32_t attention_prefill_form(const uint32_t* position, const uint32_t* rows, uint32_t nruns, uint32_t qh,
+                                uint32_t kvh);
+uint32_t attention_prefill_block_rows(uint32_t form, uint32_t qh, uint32_t kvh);
+hipError_t launch_attention_prefill(uint32_t form, const uint16_t* q, const uint16_t* k_cache,
+                                    const uint16_t* v_cache, const uint32_t* positions, const uint32_t* table,
+                                    const uint32_t* blocks, uint32_t nblocks, uint16_t* out, uint32_t out_tiled,
+                                    uint32_t rows, uint32_t qh, uint32_t kvh, uint32_t stride, uint32_t pages,
+                                    uint32_t context, uint32_t* err, hipStream_t s);
 
 // logits
 // With host_choices (coherent pinned memory), the choices and the error word

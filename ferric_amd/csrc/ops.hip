@@ -93,6 +93,17 @@ uint32_t fh_gemm_block(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, ui
   return fh::gemm_block(m, n, k, epilogue, fused_qkv != 0);
 }
 
+uint32_t fh_prefill_attention_form(const uint32_t* positions, const uint32_t* rows, uint32_t runs,
+                                   uint32_t query_heads, uint32_t kv_heads) {
+  const uint32_t g = kv_heads ? query_heads / kv_heads : 0u;
+  if (!positions || !rows || runs == 0 || (g != 1 && g != 2 && g != 4 && g != 8) || g * kv_heads != query_heads) return 0;
+  uint64_t total = 0;
+  for (uint32_t i = 0; i < runs; ++i) total += rows[i];
+  const uint32_t form =
+      total > fh::kPanelRows ? fh::attention_prefill_form(positions, rows, runs, query_heads, kv_heads) : 0u;
+  return fh::attention_prefill_block_rows(form, query_heads, kv_heads) << 16 | form;
+}
+
 uint32_t fh_activation_rows(uint32_t m) { return m ? fh::act_mtiles(m) * 16 : 0u; }
 
 uint32_t fh_gemm_default_splits(uint32_t n, uint32_t k) { return fh::gemm_default_splits(n, k); }

@@ -172,6 +172,7 @@ struct fh_ctx {
     uint32_t slots = 0;  // slots written by the batch's rows, one bit each
   };
   std::vector<PageOwner> page_owner;
+  std::vector<uint32_t> run_position, run_rows;  // runs of rows of a prefill chunk (prefill_blocks)
   std::vector<uint8_t> row_dup;  // per row of the batch: a page listed twice
   bool batch_private_slots = false;  // no row lists a page another row of the batch writes
   bool last_qkn = false;             // the last decode step ran QK-norm/KV append inside attention
@@ -772,6 +773,8 @@ fh_status fh_create(const fh_model_desc* md_in, const fh_ctx_options* op_in, fh_
     const uint64_t pmeta = 4ull * P + kMaxPrefillOutputs + (uint64_t)P * op.page_table_stride;
     TRY(dalloc(ctx, &p.d_meta, pmeta));
     TRY(halloc(ctx, &p.h_meta, pmeta));
+    ctx->run_position.resize(P);
+    ctx->run_rows.resize(P);
     TRY(dalloc(ctx, &p.d_lists, (uint64_t)(P / kRowsPerList + 1) * op.page_table_stride));
     TRY(halloc(ctx, &p.h_out, kMaxPrefillOutputs + 1));
     // Padding rows of the tiled buffers are read (never used) by the GEMM.
@@ -993,32 +996,35 @@ fh_status fh_write_kv_page(fh_ctx* ctx, uint32_t layer, uint32_t which, uint32_t
   return FH_OK;
 }
 
-// Chunks of more than kPanelRows rows run the attention kernel of long blocks
-// (k_attention_prefill.hip); smaller ones, which run the QK-norm inside the
-// attention where they can, the one of short blocks.
-bool prefill_long_blocks(uint32_t nrows) { return nrows > fh::kPanelRows; }
-
-// Attention blocks of a prefill chunk: runs of rows of one sequence at
-// consecutive positions whose page lists extend one another (so the block's
-// last row's table serves every row of it), at most attention_block_rows()
-// (attention_prefill_block_rows()) rows each, stored as first row | rows << 16. Longest first: a block reads
-// the pages up to its last row's position, and workgroups are dispatched in
-// block order, so the short ones fill the tail.
-uint32_t prefill_blocks(const fh_ctx* ctx, const fh_row* rows, uint32_t nrows, uint32_t* blocks) {
-  const uint32_t bq = prefill_long_blocks(nrows)
-                          ? fh::attention_prefill_block_rows(nrows, ctx->md.query_heads, ctx->md.kv_heads)
-                          : fh::attention_block_rows(ctx->md.query_heads, ctx->md.kv_heads);
-  uint32_t nblocks = 0;
+// Attention blocks of a prefill chunk, cut from runs of rows of one sequence
+// at consecutive positions whose page lists extend one another (so a block's
+// last row's table serves every row of it), stored as first row | rows << 16.
+// *form: the attention's form (attention_prefill_form); chunks of up to
+// kPanelRows rows, which run the QK-norm inside the attention where they can,
+// take the short blocks. Longest first: a block reads the pages up to its last
+// row's position, and workgroups are dispatched in block order, so the short
+// ones fill the tail.
+uint32_t prefill_blocks(fh_ctx* ctx, const fh_row* rows, uint32_t nrows, uint32_t* blocks, uint32_t* form) {
+  std::vector<uint32_t>&position = ctx->run_position, &length = ctx->run_rows;  // prefill_rows entries each
+  uint32_t runs = 0;
   for (uint32_t i = 0; i < nrows;) {
     uint32_t j = i + 1;
-    while (j < nrows && j - i < bq && rows[j].sequence == rows[i].sequence &&
-           rows[j].position == rows[j - 1].position + 1 && rows[j].page_count >= rows[j - 1].page_count &&
+    while (j < nrows && rows[j].sequence == rows[i].sequence && rows[j].position == rows[j - 1].position + 1 &&
+           rows[j].page_count >= rows[j - 1].page_count &&
            (rows[j].pages == rows[j - 1].pages ||
             std::memcmp(rows[j].pages, rows[j - 1].pages, (size_t)rows[j - 1].page_count * 4) == 0))
       ++j;
-    blocks[nblocks++] = i | ((j - i) << 16);  // i < 16384, j - i <= 128
+    position[runs] = rows[i].position;
+    length[runs++] = j - i;
     i = j;
   }
+  const uint32_t QH = ctx->md.query_heads, KVH = ctx->md.kv_heads;
+  *form = nrows > fh::kPanelRows ? fh::attention_prefill_form(position.data(), length.data(), runs, QH, KVH) : 0u;
+  const uint32_t bq = fh::attention_prefill_block_rows(*form, QH, KVH);
+  uint32_t nblocks = 0, first = 0;
+  for (uint32_t r = 0; r < runs; first += length[r++])
+    for (uint32_t i = 0; i < length[r]; i += bq)
+      blocks[nblocks++] = (first + i) | (std::min(bq, length[r] - i) << 16);  // first row < 16384, at most 128 rows
   std::stable_sort(blocks, blocks + nblocks, [&](uint32_t a, uint32_t b) {
     return rows[(a & 0xffffu) + (a >> 16) - 1].position > rows[(b & 0xffffu) + (b >> 16) - 1].position;
   });
@@ -1053,7 +1059,7 @@ bool prefill_blocks_private(const fh_row* rows, const uint32_t* blocks, uint32_t
 // Enqueues (or, dry, only counts) the launches of a prefill chunk of R rows
 // with nout output rows, whose metadata (tokens, positions, output rows,
 // nblocks attention blocks, page tables) is already in pre.d_meta.
-hipError_t enqueue_prefill(fh_ctx* ctx, uint32_t R, uint32_t nout, uint32_t nblocks, uint32_t nlists,
+hipError_t enqueue_prefill(fh_ctx* ctx, uint32_t R, uint32_t nout, uint32_t nblocks, uint32_t form, uint32_t nlists,
                            bool blocks_private, uint64_t* launches, bool dry = false) {
   const fh_model_desc& md = ctx->md;
   const fh_ctx_options& op = ctx->opt;
@@ -1132,9 +1138,9 @@ hipError_t enqueue_prefill(fh_ctx* ctx, uint32_t R, uint32_t nout, uint32_t nblo
     const fh::AttnQkn qa{p.part, sq, fh::partial_slab_rows(R), W.q_norm, W.k_norm, ctx->cos_t, ctx->sin_t,
                          kc,     vc, md.rms_epsilon};
     L(FH_KC_ATTENTION, [&] {
-      if (prefill_long_blocks(R))
-        return fh::launch_attention_prefill(p.qrot, kc, vc, d_pos, d_tab, d_blocks, nblocks, p.attn, 1, R, QH, KVH,
-                                            stride, pages, C, err, s);
+      if (form)
+        return fh::launch_attention_prefill(form, p.qrot, kc, vc, d_pos, d_tab, d_blocks, nblocks, p.attn, 1, R, QH,
+                                            KVH, stride, pages, C, err, s);
       return fh::launch_attention_blocks(p.qrot, kc, vc, d_pos, d_tab, d_blocks, nblocks, p.attn, 1, R, QH, KVH,
                                          stride, pages, C, err, s, qkn_blocks ? &qa : nullptr);
     });
@@ -1238,7 +1244,8 @@ fh_status run_prefill(fh_ctx* ctx, uint64_t batch_id, const fh_row* rows, uint32
     std::fill(to + rows[i].page_count, to + stride, 0xffffffffu);
   }
   for (uint32_t i = 0; i < nout; ++i) outs[i] = output_rows[i];
-  const uint32_t nblocks = prefill_blocks(ctx, rows, nrows, blocks);
+  uint32_t form = 0;
+  const uint32_t nblocks = prefill_blocks(ctx, rows, nrows, blocks, &form);
   const bool priv = nrows <= fh::kPanelRows && prefill_blocks_private(rows, blocks, nblocks);
   auto poison = [&](fh_status s2, const std::string& msg) {
     ctx->poisoned = true;
@@ -1254,7 +1261,7 @@ fh_status run_prefill(fh_ctx* ctx, uint64_t batch_id, const fh_row* rows, uint32
   hipEventRecord(ctx->ev_begin, s);
   if (ctx->profiling) ctx->prof_launches.clear();
   uint64_t n = 0;
-  e = enqueue_prefill(ctx, nrows, nout, nblocks, nlists, priv, &n);
+  e = enqueue_prefill(ctx, nrows, nout, nblocks, form, nlists, priv, &n);
   if (e != hipSuccess) return poison(FH_ERR_DEVICE, std::string("launch: ") + hipGetErrorString(e) + ctx->launch_detail);
   hipEventRecord(ctx->ev_end, s);
   if (nout) e = hipMemcpyAsync(p.h_out, p.choices, nout * 4, hipMemcpyDeviceToHost, s);
@@ -1405,9 +1412,10 @@ fh_status fh_expected_dispatch_count(fh_ctx* ctx, uint64_t batch_id, const fh_ro
   uint64_t n = 0;
   if (nrows > ctx->opt.row_capacity) {
     std::vector<uint32_t> blocks(nrows);
-    const uint32_t nblocks = prefill_blocks(ctx, rows, nrows, blocks.data());
+    uint32_t form = 0;
+    const uint32_t nblocks = prefill_blocks(ctx, rows, nrows, blocks.data(), &form);
     const bool priv = nrows <= fh::kPanelRows && prefill_blocks_private(rows, blocks.data(), nblocks);
-    enqueue_prefill(ctx, nrows, nout, nblocks, 0, priv, &n, true);
+    enqueue_prefill(ctx, nrows, nout, nblocks, form, 0, priv, &n, true);
   }
   else
     enqueue_step(ctx, nrows, &n, true);

@@ -258,6 +258,11 @@ uint32_t fh_gemm_default_splits(uint32_t n, uint32_t k);
  * chunk's QKV projection with QK-norm, RoPE and KV append inside, epilogue ignored) takes for
  * m > 32: rows << 16 | columns; 0 where the weight is streamed or the shape refused. */
 uint32_t fh_gemm_block(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, uint32_t fused_qkv);
+/* Attention of a prefill chunk of `runs` runs of rows (run i: rows[i] rows of one sequence from
+ * positions[i] on): rows per block << 16 | form, where the form is 0 (short blocks) or the
+ * waves along the keys of the long blocks (1, 2 or 4); 0 where the heads are not supported. */
+uint32_t fh_prefill_attention_form(const uint32_t* positions, const uint32_t* rows, uint32_t runs,
+                                   uint32_t query_heads, uint32_t kv_heads);
 /* Rows a tiled activation buffer for m rows holds: 32 for m <= 32, else m rounded up to 256. */
 uint32_t fh_activation_rows(uint32_t m);
 /* Rows of one FH_EPI_PARTIAL slab for an m-row batch: 32 for m <= 32, 256 for 32 < m <= 256,

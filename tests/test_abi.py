@@ -179,6 +179,29 @@ def test_narrow_projections_take_blocks_that_split_k():
     assert block(300, 384, 1024, fused_qkv=1) == block(256, 256, 1024, fused_qkv=1) == (0, 0)  # not fused there
 
 
+def attention_form(runs, query_heads, kv_heads):
+    v = ferric_amd.load().fh_prefill_attention_form(u32([p for p, _ in runs]), u32([n for _, n in runs]), len(runs),
+                                                    query_heads, kv_heads)
+    return v >> 16, v & 0xffff
+
+
+def test_prefill_attention_form_follows_the_runs_of_a_chunk():
+    # The number of rows alone does not tell: many runs of a row or two take the
+    # short blocks (64 query vectors of a KV head), one long run long blocks.
+    for heads, kv in [(8, 8), (16, 8), (32, 8), (32, 4)]:
+        g = heads // kv
+        assert attention_form([(0, 1)] * 300, heads, kv) == (64 // g, 0)
+        for rows in (257, 777, 2000, 8000):
+            block, form = attention_form([(0, rows)], heads, kv)
+            assert form in (1, 2, 4) and block == 128 // form // g
+        assert attention_form([(5, 100), (0, 156)], heads, kv) == (64 // g, 0)  # up to 256 rows: short blocks
+    for runs in ([(0, 1)] * 1000, [(0, 2)] * 400):
+        assert attention_form(runs, 32, 8) == (16, 0)
+    for runs in ([(7000, 16)] * 20, [(2000, 32)] * 10, [(300, 1)] * 300):  # 8-row blocks: 1.4 to 1.5 times as long
+        assert attention_form(runs, 32, 8) in ((16, 0), (16, 2))
+    assert attention_form([(0, 300)], 24, 8) == attention_form([(0, 300)], 32, 0) == (0, 0)  # heads not supported
+
+
 def test_ops_reject_bad_shapes_before_any_launch():
     lib = ferric_amd.load()
     p = ctypes.c_void_p(16)  # never dereferenced: validation fails first

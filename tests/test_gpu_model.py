@@ -23,6 +23,7 @@ the yardstick for the GPU's (a third order). Bars (tests/spread.py):
     (pages[pos // 16], pos % 16); every other slot keeps its bits.
 """
 
+import ctypes
 import hashlib
 import json
 from pathlib import Path
@@ -945,6 +946,35 @@ def test_prefill_attention_of_long_blocks(qh, kvh, prompts, decode, interleave):
         batch, out, ref = pair.step(rows, outs)
         _mark_written(pair, batch)
         pair.check(batch, out, ref, f"long blocks {qh}/{kvh} {prompts}")
+        pair.check_kv()
+    finally:
+        pair.close()
+
+
+# Chunks of more than 256 rows made of many short runs of rows: the short blocks
+# (form 0) and the long ones of 128 and 64 vectors (forms 1 and 2) that hold
+# one run each, with 1, 2, 4 and 8 query heads per KV head.
+@pytest.mark.parametrize("qh,kvh,sequences,tokens,form", [
+    (32, 8, 300, 1, 0), (16, 8, 100, 5, 0), (8, 8, 100, 3, 0), (32, 4, 300, 1, 0),
+    (8, 8, 40, 9, 1), (16, 8, 60, 5, 1), (32, 8, 16, 17, 1), (32, 4, 100, 3, 1), (16, 8, 10, 33, 2), (32, 4, 10, 33, 2),
+])
+def test_prefill_attention_of_short_runs(qh, kvh, sequences, tokens, form):
+    got = ferric_amd.load().fh_prefill_attention_form((ctypes.c_uint32 * sequences)(),
+                                                      (ctypes.c_uint32 * sequences)(*[tokens] * sequences),
+                                                      sequences, qh, kvh)
+    assert got & 0xffff == form
+    cfg = dict(ferric_amd.QWEN3_0_6B, layers=1, hidden=512, query_heads=qh, kv_heads=kvh, intermediate=512,
+               vocabulary=4096)
+    limits = PagedLimits(context_tokens=512, physical_page_count=sequences * 3 + 8, page_table_stride=32)
+    seed = 71 + qh + kvh + sequences
+    pair = Pair(cfg, limits, seed=seed, rows=8, prefill_rows=512)
+    try:
+        rng = np.random.default_rng(seed)
+        sids = [pair.pool.admit(0) for _ in range(sequences)]
+        rows = [(s, int(t)) for s in sids for t in rng.integers(0, 4096, tokens)]
+        batch, out, ref = pair.step(rows, list(range(0, len(rows), len(rows) // 40 + 1)) + [len(rows) - 1])
+        _mark_written(pair, batch)
+        pair.check(batch, out, ref, f"short runs {qh}/{kvh} {sequences} x {tokens}")
         pair.check_kv()
     finally:
         pair.close()
