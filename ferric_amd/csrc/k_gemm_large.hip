@@ -262,19 +262,21 @@ __global__ __launch_bounds__(512) void gemm_large_xd_kernel(const uint16_t* __re
 // Estimated microseconds of a launch of 256 x 256 blocks (fitted with
 // mid_cost, k_gemm_mid.hip): whole rounds of the 256 CUs, a k-block taking
 // longer the more CUs run, and what a block costs around its k loop.
-float block_cost(uint32_t m, uint32_t n, uint32_t k) {
+float block_cost(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, bool fused_qkv) {
   const uint32_t blocks = n / (16 * kBigTiles) * ((m + 255) / 256);
-  const float kb_us = blocks < 100 ? 0.57f : blocks < 256 ? 0.66f : 0.73f;
-  return ((blocks + 255) / 256) * (12.5f + (k / 32) * kb_us);
+  const float kb_us = blocks < 100 ? 0.514f : blocks < 256 ? 0.703f : 0.689f;
+  const float around =
+      fused_qkv ? 12.93f : epilogue == FH_EPI_SWIGLU ? 13.97f : epilogue == FH_EPI_RESIDUAL ? 16.37f : 13.52f;
+  return ((blocks + 255) / 256) * (around + (k / 32) * kb_us);
 }
 
 // Which of the three kernels a projection of m rows runs.
 enum class LargeKernel { kMid, kBand, kBlock };
 
-LargeKernel pick_kernel(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, bool whole_heads) {
-  const float mid = gemm_mid_cost(m, n, k, whole_heads), band = gemm_band_cost(m, n, k, epilogue);
+LargeKernel pick_kernel(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, bool fused_qkv) {
+  const float mid = gemm_mid_cost(m, n, k, epilogue, fused_qkv), band = gemm_band_cost(m, n, k, epilogue, fused_qkv);
   const bool block_ok = m > kPanelRows && n % (16 * kBigTiles) == 0;
-  const float block = block_ok ? block_cost(m, n, k) : -1.f;
+  const float block = block_ok ? block_cost(m, n, k, epilogue, fused_qkv) : -1.f;
   if (block_ok && block <= mid && (band < 0.f || block <= band)) return LargeKernel::kBlock;
   return band >= 0.f && band < mid ? LargeKernel::kBand : LargeKernel::kMid;
 }
@@ -301,8 +303,8 @@ uint32_t gemm_block(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, bool 
              ((epilogue == FH_EPI_SWIGLU || epilogue == FH_EPI_F32) && panel_streams(m, n))) {
     return 0;
   }
-  switch (pick_kernel(m, n, k, fused_qkv ? (uint32_t)FH_EPI_BF16 : epilogue, fused_qkv)) {
-    case LargeKernel::kMid: return gemm_mid_block(m, n, k, fused_qkv);
+  switch (pick_kernel(m, n, k, epilogue, fused_qkv)) {
+    case LargeKernel::kMid: return gemm_mid_block(m, n, k, epilogue, fused_qkv);
     case LargeKernel::kBand: return kLargeBlockRows << 16 | kPanelCols;
     case LargeKernel::kBlock: break;
   }

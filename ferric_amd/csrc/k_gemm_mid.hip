@@ -256,37 +256,51 @@ __global__ __launch_bounds__(WAVES * 64, OCC) void gemm_mid_kernel(const uint16_
 
 // Block shapes: 32 tn weight rows x 32 tm activation rows, and what
 // mid_cost needs of each: the operand GB/s of a CU running such blocks alone,
-// and microseconds per launch and per 256 blocks around the k loop (prologue,
-// reduction, epilogue).
+// microseconds per launch and per 256 blocks around the k loop (prologue,
+// reduction, epilogue), and the same two where k is so short that nothing else
+// is left.
 struct MidShape {
   uint32_t tn, tm;
-  float cu_gbs, launch_us, round_us;
+  float cu_gbs, launch_us, round_us, least_us, least_round_us;
 };
-constexpr MidShape kMidShapes[] = {{4, 4, 66.f, 0.8f, 7.9f}, {4, 2, 73.f, 2.3f, 0.6f}, {2, 4, 83.f, 2.5f, 1.3f},
-                                   {2, 2, 75.f, 1.3f, 0.f},  {1, 2, 80.f, 2.5f, 0.1f}, {1, 1, 64.f, 3.4f, 0.f}};
+constexpr MidShape kMidShapes[] = {{4, 4, 69.0f, 0.66f, 10.82f, 8.11f, 0.01f}, {4, 2, 73.0f, 3.59f, 0.46f, 2.20f, 1.92f},
+                                    {2, 4, 77.3f, 3.32f, 1.55f, 4.84f, 0.67f}, {2, 2, 75.2f, 2.21f, 0.04f, 2.95f, 0.76f},
+                                    {1, 2, 65.0f, 2.07f, 0.39f, 2.70f, 0.62f}, {1, 1, 66.8f, 2.19f, 0.34f, 1.61f, 0.85f}};
+// Microseconds that the SwiGLU and the QK-norm epilogues take longer, per 256
+// blocks of 4 32 x 32 outputs.
+constexpr float kMidSwigluUs = 0.43f, kMidQkvUs = 0.47f;
 
 // Estimated microseconds of one launch: the operand bytes of all blocks at
-// 18.4 TB/s, but no less than those of the blocks one CU runs at its own
-// rate, plus the shape's overheads. Its constants and those of the other two
-// kernels' estimates (gemm_band_cost, block_cost) are fitted together to the
-// times of every shape at 40 row counts from 33 to 8192 of the Qwen3
-// projections (296 points): the estimate picks a kernel and block within 9 %
-// of the fastest one at every point, 0.6 % on average, and never one more
-// than 5 % slower than the 256 x 256 blocks alone, which are 1.67 times
-// slower on average.
-float mid_cost(const MidShape& s, uint32_t m, uint32_t n, uint32_t k) {
-  const float blocks = (float)(n / (32 * s.tn)) * ((m + 32 * s.tm - 1) / (32 * s.tm));
+// 17.8 TB/s, but no less than those of the blocks one CU runs at its own
+// rate, plus the shape's overheads; and no less than the launch takes at a k
+// of a few k-blocks. Its constants and those of the other two kernels'
+// estimates (gemm_band_cost, block_cost) are fitted together to the times of
+// every form at 3221 launches: 33 to 8192 rows of the Qwen3 projections, their
+// fused QKV form, other wide weights and weights of 128 to 512 columns at k of
+// 1024 to 12288, and 128 to 16512 columns at k of 32 to 768, with all
+// epilogues. The estimate picks a form that is slower than the fastest by (mean,
+// most): Qwen3 projections 0.7 %, 17 %; fused QKV 0.8 %, 21 %; other wide weights
+// 0.5 %, 15 %; narrow weights 2.5 %, 69 % (2048 x 256 x 12288 58 us, 34.5 possible);
+// k up to 768 0.9 %, 37 % (3000 x 16512 x 32). At the first three it is never more
+// than 3 % slower than the 256 x 256 blocks alone. (Constants fitted to 296
+// launches of the Qwen3 projections only gave 1.9, 2.1, 2.7 and 4.4 % on
+// average; every k of up to 128 took 128 x 128 blocks: 96 x 128 x 64 5.9 us,
+// now 3.3, 4.7 with the weight stream before these blocks.)
+float mid_cost(const MidShape& s, uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, bool fused_qkv) {
+  const float rounds = (float)(n / (32 * s.tn)) * ((m + 32 * s.tm - 1) / (32 * s.tm)) / 256.f;
   const float block_kb = 2.048f * (s.tn + s.tm) * (k / 32);  // operand kilobytes of a block
-  const float all = blocks * block_kb / 18400.f;
-  const float cu = ceilf(blocks / 256.f) * block_kb / s.cu_gbs;
-  return s.launch_us + blocks / 256.f * s.round_us + fmaxf(all, cu);
+  const float all = rounds * 256.f * block_kb / 17800.f;
+  const float cu = ceilf(rounds) * block_kb / s.cu_gbs;
+  const float more = (fused_qkv ? kMidQkvUs : epilogue == FH_EPI_SWIGLU ? kMidSwigluUs : 0.f) * (s.tn * s.tm / 4.f);
+  return fmaxf(s.least_us + rounds * (s.least_round_us + more),
+               s.launch_us + rounds * (s.round_us + more) + fmaxf(all, cu));
 }
 
-bool mid_pick(uint32_t m, uint32_t n, uint32_t k, bool whole_heads, MidShape* pick, float* cost) {
+bool mid_pick(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, bool fused_qkv, MidShape* pick, float* cost) {
   bool found = false;
   for (const MidShape& s : kMidShapes) {
-    if (n % (32 * s.tn) != 0 || (whole_heads && s.tn != 4)) continue;
-    const float c = mid_cost(s, m, n, k);
+    if (n % (32 * s.tn) != 0 || (fused_qkv && s.tn != 4)) continue;
+    const float c = mid_cost(s, m, n, k, epilogue, fused_qkv);
     if (!found || c < *cost) {
       *pick = s;
       *cost = c;
@@ -335,19 +349,18 @@ hipError_t launch_mid_shape(MidShape v, const uint16_t* xt, const uint16_t* w, u
 
 }  // namespace
 
-float gemm_mid_cost(uint32_t m, uint32_t n, uint32_t k, bool whole_heads) {
+float gemm_mid_cost(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, bool fused_qkv) {
   MidShape v{};
   float cost = 0.f;
-  return m > kMaxRows && n % 32 == 0 && k % 32 == 0 && k > 0 &&
-                 mid_pick(m, n, k, whole_heads, &v, &cost)
+  return m > kMaxRows && n % 32 == 0 && k % 32 == 0 && k > 0 && mid_pick(m, n, k, epilogue, fused_qkv, &v, &cost)
              ? cost
              : -1.f;
 }
 
-uint32_t gemm_mid_block(uint32_t m, uint32_t n, uint32_t k, bool whole_heads) {
+uint32_t gemm_mid_block(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, bool fused_qkv) {
   MidShape v{};
   float cost = 0.f;
-  return mid_pick(m, n, k, whole_heads, &v, &cost) ? (32 * v.tm) << 16 | 32 * v.tn : 0u;
+  return mid_pick(m, n, k, epilogue, fused_qkv, &v, &cost) ? (32 * v.tm) << 16 | 32 * v.tn : 0u;
 }
 
 hipError_t launch_gemm_mid(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_t m, uint32_t n, uint32_t k,
@@ -355,7 +368,7 @@ hipError_t launch_gemm_mid(const uint16_t* x_tiled, const uint16_t* w_tiled, uin
                            hipStream_t s) {
   MidShape v{};
   float cost = 0.f;
-  if (m <= kMaxRows || n % 32 != 0 || k % 32 != 0 || k == 0 || !mid_pick(m, n, k, false, &v, &cost))
+  if (m <= kMaxRows || n % 32 != 0 || k % 32 != 0 || k == 0 || !mid_pick(m, n, k, epilogue, false, &v, &cost))
     return hipErrorInvalidValue;
   const QkvRopeArgs none{};
 #define FH_MID_EPI(E) \
@@ -374,7 +387,7 @@ hipError_t launch_gemm_mid_qkv_rope(const uint16_t* x_tiled, const uint16_t* w_t
                                     uint32_t k, const QkvRopeArgs& qa, hipStream_t s) {
   MidShape v{};
   float cost = 0.f;
-  if (m <= kMaxRows || n != (qa.qh + 2 * qa.kvh) * 128 || k % 32 != 0 || k == 0 || !mid_pick(m, n, k, true, &v, &cost))
+  if (m <= kMaxRows || n != (qa.qh + 2 * qa.kvh) * 128 || k % 32 != 0 || k == 0 || !mid_pick(m, n, k, FH_EPI_BF16, true, &v, &cost))
     return hipErrorInvalidValue;
   return launch_mid_shape<kMidEpiQkvRope>(v, x_tiled, w_tiled, m, n, k, nullptr, nullptr, 0u, qa, nullptr, s);
 }

@@ -162,16 +162,16 @@ hipError_t launch_gemm_large(const uint16_t* x_tiled, const uint16_t* w_tiled, u
 uint32_t gemm_block(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, bool fused_qkv);
 // Mid-sized batches (k_gemm_mid.hip): m > kMaxRows, n % 32 == 0, the same
 // operands as launch_gemm_large. gemm_mid_cost estimates the launch's
-// microseconds (whole_heads: the QKV form), negative where it has no form.
-float gemm_mid_cost(uint32_t m, uint32_t n, uint32_t k, bool whole_heads);
-uint32_t gemm_mid_block(uint32_t m, uint32_t n, uint32_t k, bool whole_heads);
+// microseconds (fused_qkv: the QKV form, any epilogue), negative where it has no form.
+float gemm_mid_cost(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, bool fused_qkv);
+uint32_t gemm_mid_block(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, bool fused_qkv);
 hipError_t launch_gemm_mid(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_t m, uint32_t n, uint32_t k,
                            uint32_t epilogue, const uint16_t* residual, void* out, uint32_t ldo, uint32_t* err,
                            hipStream_t s);
 hipError_t launch_gemm_mid_qkv_rope(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_t m, uint32_t n,
                                     uint32_t k, const QkvRopeArgs& qa, hipStream_t s);
 // Chunks of 256-row x 128-column blocks (k_gemm_band.hip): n % 128 == 0.
-float gemm_band_cost(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue);
+float gemm_band_cost(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, bool fused_qkv);
 hipError_t launch_gemm_band(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_t m, uint32_t n, uint32_t k,
                             uint32_t epilogue, const uint16_t* residual, void* out, uint32_t ldo, uint32_t* err,
                             hipStream_t s);

@@ -179,6 +179,25 @@ def test_narrow_projections_take_blocks_that_split_k():
     assert block(300, 384, 1024, fused_qkv=1) == block(256, 256, 1024, fused_qkv=1) == (0, 0)  # not fused there
 
 
+def test_projections_of_a_short_k_take_small_blocks():
+    # With one to four k-blocks a launch is its prologue, reduction and
+    # epilogue, which the smallest blocks spread over the most CUs.
+    for k in (32, 64, 128):
+        for n in (128, 256, 384, 512, 768, 1152):
+            for m in (33, 64, 96, 160, 256, 257, 400, 600):
+                for epilogue in (_lib.EPI_BF16, _lib.EPI_RESIDUAL, _lib.EPI_SWIGLU, _lib.EPI_F32):
+                    rows, cols = block(m, n, k, epilogue)
+                    assert 0 < rows * cols <= 64 * 64, (m, n, k, epilogue)
+
+
+def test_projections_that_256_x_128_blocks_fit_badly_take_others():
+    # 288 such blocks with the work of 240: some CU gets a full block and a last one (7 % slower than 256 x 256 blocks).
+    for m in (520, 600, 640):
+        assert block(m, 12288, 2048, _lib.EPI_SWIGLU) != (256, 128)
+    # Gate/up of 8B at 3000 rows: 2256 of them in nine rounds, 5 % slower than five rounds of 256 x 256 blocks.
+    assert block(3000, 24576, 4096, _lib.EPI_SWIGLU) == (256, 256)
+
+
 def attention_form(runs, query_heads, kv_heads):
     v = ferric_amd.load().fh_prefill_attention_form(u32([p for p, _ in runs]), u32([n for _, n in runs]), len(runs),
                                                     query_heads, kv_heads)
