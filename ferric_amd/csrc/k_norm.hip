@@ -566,8 +566,11 @@ constexpr uint32_t kWaveNormRows = 256;
 // Row counts up to which the RMSNorm of many rows runs one wave per row (5000
 // rows of width 4096: 20.8 us against 23.6 with 16-row tiles; 8000: 43 against 30).
 constexpr uint32_t kWaveRowsMax = 5120;
-// Row counts up to which the QK-norm of bf16 rows runs one wave per (row, head).
-constexpr uint32_t kWaveQkRows = 64;
+// (row, head)s up to which the QK-norm of bf16 rows runs one wave for each: the
+// 64-per-workgroup kernel takes 5.4 us however few they are, the waves 3.3 us up
+// to 800, 4.0 at 1560 (65 rows of 8 + 2 x 8 heads), 4.6 at 2080 (65 of 16 + 2 x
+// 8), 5.4 at 3840 to 4096, 6.1 at 4480 (80 of 40 + 2 x 8).
+constexpr uint32_t kWaveQkHeads = 4096;
 
 hipError_t launch_qknorm_rope_kv(const uint16_t* qkv, const float* qkv_part, uint32_t splits, const uint16_t* q_norm,
                                  const uint16_t* k_norm, const float* cos_t, const float* sin_t,
@@ -575,13 +578,13 @@ hipError_t launch_qknorm_rope_kv(const uint16_t* qkv, const float* qkv_part, uin
                                  uint16_t* k_cache, uint16_t* v_cache, uint32_t rows, uint32_t qh, uint32_t kvh,
                                  uint32_t stride, uint32_t pages, uint32_t context, float eps, uint32_t* err,
                                  hipStream_t s) {
-  // bf16 rows: a few rows one wave per (row, head) as in decode; beyond that
+  // bf16 rows: a few (row, head)s one wave each as in decode; beyond that
   // 64 (row, head)s per workgroup (8B shape, 256 rows: 11.1 -> 5.5 us).
   // (Its 16-byte accesses need aligned operands; others keep the waves.)
   const uintptr_t bits = (uintptr_t)qkv | (uintptr_t)q_norm | (uintptr_t)k_norm | (uintptr_t)cos_t | (uintptr_t)sin_t |
                          (uintptr_t)q_out | (uintptr_t)k_cache | (uintptr_t)v_cache;
-  if (!qkv_part && rows > kWaveQkRows && (bits & 15u) == 0) {
-    const uint64_t heads = (uint64_t)rows * (qh + 2 * kvh);
+  const uint64_t heads = (uint64_t)rows * (qh + 2 * kvh);
+  if (!qkv_part && heads > kWaveQkHeads && (bits & 15u) == 0) {
     const QkvRopeArgs a{q_norm, k_norm, cos_t, sin_t, positions, table, q_out, k_cache, v_cache,
                         qh,     kvh,    stride, pages, context, eps,   err};
     hipLaunchKernelGGL(qknorm_rope_kv_rows_kernel, dim3((unsigned)((heads + kRowsHeads - 1) / kRowsHeads)), dim3(256), 0, s,

@@ -893,6 +893,13 @@ def test_qknorm_rope_kv_of_many_rows_bit_exact(qh, kvh, rows):
     test_qknorm_rope_kv_bit_exact(qh, kvh, 0, rows)
 
 
+# On either side of 4096 (row, head)s, the line between one wave for each and 64
+# per workgroup, below and above 256 rows.
+@pytest.mark.parametrize("qh,kvh,rows", [(32, 8, 85), (32, 8, 86), (8, 1, 409), (8, 1, 410), (1, 1, 300)])
+def test_qknorm_rope_kv_on_either_side_of_the_wave_line(qh, kvh, rows):
+    test_qknorm_rope_kv_bit_exact(qh, kvh, 0, rows)
+
+
 # The two partition sizes on either side of their rule (16 pages up to 1024
 # partitions of a (row, query head) and 256 workgroups at the context capacity,
 # and for up to 64 pairs): the last launch of 16-page partitions, the first of
