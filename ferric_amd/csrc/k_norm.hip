@@ -528,16 +528,16 @@ __global__ __launch_bounds__(kNormThreads) void tile_activation_kernel(const uin
   }
 }
 
-// Eight elements per thread in 16-byte loads and stores (12.3 M elements: 22.3 ->
-// 14.5 us, 5.1 TB/s; 98 M: 174 -> 106 us), then the elements past the last whole eight. aligned: all three pointers are 16-byte aligned;
-// else every element on its own.
+// kWide: eight elements per thread in 16-byte loads and stores, then the
+// elements past the last whole eight; else every element on its own
+// (launch_swiglu's line between them).
+template <bool kWide>
 __global__ __launch_bounds__(kNormThreads) void swiglu_kernel(const uint16_t* __restrict__ gate,
                                                               const uint16_t* __restrict__ up,
-                                                              uint16_t* __restrict__ out, uint64_t n,
-                                                              uint32_t aligned, uint32_t* err) {
+                                                              uint16_t* __restrict__ out, uint64_t n, uint32_t* err) {
   bool bad = false;
   const uint64_t first = (uint64_t)blockIdx.x * kNormThreads + threadIdx.x, step = (uint64_t)gridDim.x * kNormThreads;
-  const uint64_t eights = aligned ? n / 8 : 0;
+  const uint64_t eights = kWide ? n / 8 : 0;
   for (uint64_t i = first; i < eights; i += step) {
     const uint4 g = reinterpret_cast<const uint4*>(gate)[i], u = reinterpret_cast<const uint4*>(up)[i];
     const uint32_t gs[4] = {g.x, g.y, g.z, g.w}, us[4] = {u.x, u.y, u.z, u.w};
@@ -669,12 +669,18 @@ hipError_t launch_tile_activation(const uint16_t* x, uint16_t* x_tiled, uint32_t
 
 hipError_t launch_swiglu(const uint16_t* gate, const uint16_t* up, uint16_t* out, uint64_t n, uint32_t* err,
                          hipStream_t s) {
-  const bool aligned = (((uintptr_t)gate | (uintptr_t)up | (uintptr_t)out) & 15u) == 0;
-  const uint64_t per = aligned ? 8 * kNormThreads : kNormThreads;
+  // Eight elements per thread from 2^20 elements on where all three operands are
+  // 16-byte aligned: 12.3 M elements 22.3 -> 14.5 us (5.1 TB/s), 98 M 174 -> 106,
+  // 3.1 M 6.3 -> 5.7, 2^20 3.55 -> 3.5. Fewer elements are a chain of a load, the
+  // exponentials and a store, eight times as long: 12288 2.5 -> 2.8, 400000 2.7 -> 3.0.
+  const bool wide = n >= 1u << 20 && (((uintptr_t)gate | (uintptr_t)up | (uintptr_t)out) & 15u) == 0;
+  const uint64_t per = wide ? 8 * kNormThreads : kNormThreads;
   uint64_t g = (n + per - 1) / per;
   if (g > 65536) g = 65536;
-  hipLaunchKernelGGL(swiglu_kernel, dim3((unsigned)g), dim3(kNormThreads), 0, s, gate, up, out, n, aligned ? 1u : 0u,
-                     err);
+  if (wide)
+    hipLaunchKernelGGL(swiglu_kernel<true>, dim3((unsigned)g), dim3(kNormThreads), 0, s, gate, up, out, n, err);
+  else
+    hipLaunchKernelGGL(swiglu_kernel<false>, dim3((unsigned)g), dim3(kNormThreads), 0, s, gate, up, out, n, err);
   return hipGetLastError();
 }
 

@@ -948,6 +948,13 @@ def test_swiglu_remainders_and_alignment(n, offset):
     assert np.all(got[:offset] == 0x1234) and np.all(got[offset + n:] == 0x1234)
 
 
+# The same on either side of 2^20 elements, the line between one element and eight per thread.
+@pytest.mark.parametrize("n,offset", [((1 << 20) - 1, 0), (1 << 20, 0), ((1 << 20) + 7, 0), ((1 << 20) + 9, 1),
+                                      ((1 << 20) + 4103, 8)])
+def test_swiglu_on_either_side_of_the_wide_line(n, offset):
+    test_swiglu_remainders_and_alignment(n, offset)
+
+
 def test_swiglu_standalone():
     r = rng(5)
     n = 1 << 15
