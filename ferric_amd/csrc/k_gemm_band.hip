@@ -334,7 +334,10 @@ hipError_t launch_band(const uint16_t* xt, const uint16_t* w, uint32_t m, uint32
   return hipGetLastError();
 }
 
-bool band_ok(uint32_t m, uint32_t n, uint32_t k) { return m > kMaxRows && n % kBandCols == 0 && k % 32 == 0 && k > 0; }
+// (k < 2^24: a block's weight tiles are within the 32-bit offsets of its loads.)
+bool band_ok(uint32_t m, uint32_t n, uint32_t k) {
+  return m > kMaxRows && n % kBandCols == 0 && k % 32 == 0 && k > 0 && k < 1u << 24;
+}
 
 }  // namespace
 

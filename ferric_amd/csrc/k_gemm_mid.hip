@@ -52,11 +52,16 @@ __device__ __forceinline__ void mid_for(F&& f) {
   }
 }
 
+// From this k on the 8 tiles that a 128-row block has per k-block span 4 GiB.
+constexpr uint32_t kMidFarK = 1u << 24;
+
 // The QKV projection with QK-norm, RoPE and the KV append in its epilogue
 // (TN = 4: a workgroup's columns are one head).
 constexpr int kMidEpiQkvRope = 16;
 
-template <int TN, int TM, int WAVES, int D, int OCC, int EPI>
+// kFar: 64-bit operand addresses (global loads) for a k whose weight rows the
+// buffer loads' 32-bit offsets do not reach (kMidFarK).
+template <int TN, int TM, int WAVES, int D, int OCC, int EPI, bool kFar>
 __global__ __launch_bounds__(WAVES * 64, OCC) void gemm_mid_kernel(const uint16_t* __restrict__ xt,
                                                                    const uint16_t* __restrict__ w, uint32_t m,
                                                                    uint32_t mtiles, uint32_t kb_count,
@@ -104,18 +109,27 @@ __global__ __launch_bounds__(WAVES * 64, OCC) void gemm_mid_kernel(const uint16_
 
   if (kb_n > 0) {
     // Buffer descriptors: the block's weight rows from k-block `wave` on
-    // (32-bit offsets: k < 2^24), and one k-block of its activation rows.
+    // (32-bit offsets: k < kMidFarK), and one k-block of its activation rows.
     const uint64_t w0 = ((uint64_t)gx * 2 * TN * kb_count + wave) * 512, x0 = ((uint64_t)wave * mtiles + gy * 2 * TM) * 512;
     auto wrs = __builtin_amdgcn_make_buffer_rsrc((void*)(w + w0), 0, (2u * TN * kb_count - wave) * 1024u, 0x00020000);
     const uint32_t in_tile = (lane & 15) + 16 * (lane >> 5), second = (lane >> 4) & 1;
     const uint32_t wofs = (second * kb_count * 64 + in_tile) * 16, xofs = (second * 64 + in_tile) * 16;
     const uint32_t wpair = kb_count * 2048u;
+    const u32x4* wfar = reinterpret_cast<const u32x4*>(w + w0) + (uint64_t)second * kb_count * 64 + in_tile;
+    const u32x4* xfar = reinterpret_cast<const u32x4*>(xt + x0) + second * 64 + in_tile;
     // Stage: the operands of half a k-block.
     u32x4 wr[D][TN], xr[D][TM];
     const uint32_t halves = 2 * kb_n;
     auto load = [&](auto slot_c, uint32_t hk) {
       constexpr int S = decltype(slot_c)::value;
       const uint32_t q = min(hk, halves - 1), kk = (q >> 1) * WAVES, half = (q & 1u) * 512;
+      if constexpr (kFar) {
+#pragma unroll
+        for (int i = 0; i < TN; ++i) wr[S][i] = wfar[((uint64_t)kk + 2ull * i * kb_count) * 64 + half / 16];
+#pragma unroll
+        for (int j = 0; j < TM; ++j) xr[S][j] = xfar[(uint64_t)kk * mtiles * 64 + half / 16 + j * 128];
+        return;
+      }
       const uint32_t ws = kk * 1024 + half;
       auto xrs = __builtin_amdgcn_make_buffer_rsrc((void*)(xt + x0 + (uint64_t)kk * mtiles * 512), 0, 2 * TM * 1024u, 0x00020000);
 #pragma unroll
@@ -299,7 +313,7 @@ float mid_cost(const MidShape& s, uint32_t m, uint32_t n, uint32_t k, uint32_t e
 bool mid_pick(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, bool fused_qkv, MidShape* pick, float* cost) {
   bool found = false;
   for (const MidShape& s : kMidShapes) {
-    if (n % (32 * s.tn) != 0 || (fused_qkv && s.tn != 4)) continue;
+    if (n % (32 * s.tn) != 0 || (fused_qkv && s.tn != 4) || (k >= kMidFarK && s.tn * s.tm != 1)) continue;
     const float c = mid_cost(s, m, n, k, epilogue, fused_qkv);
     if (!found || c < *cost) {
       *pick = s;
@@ -310,11 +324,11 @@ bool mid_pick(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, bool fused_
   return found;
 }
 
-template <int TN, int TM, int WAVES, int D, int OCC, int EPI>
+template <int TN, int TM, int WAVES, int D, int OCC, int EPI, bool kFar = false>
 void launch_mid_variant(const uint16_t* xt, const uint16_t* w, uint32_t m, uint32_t n, uint32_t k,
                         const uint16_t* residual, void* out, uint32_t ldo, const QkvRopeArgs& qa, uint32_t* err,
                         hipStream_t s) {
-  hipLaunchKernelGGL((gemm_mid_kernel<TN, TM, WAVES, D, OCC, EPI>), dim3(n / (32 * TN), (m + 32 * TM - 1) / (32 * TM)),
+  hipLaunchKernelGGL((gemm_mid_kernel<TN, TM, WAVES, D, OCC, EPI, kFar>), dim3(n / (32 * TN), (m + 32 * TM - 1) / (32 * TM)),
                      dim3(WAVES * 64), 0, s, xt, w, m, act_mtiles(m), k / 32, residual, out, ldo, qa, err);
 }
 
@@ -327,7 +341,10 @@ hipError_t launch_mid_shape(MidShape v, const uint16_t* xt, const uint16_t* w, u
                             hipStream_t s) {
 #define FH_MID(TN_, TM_, WAVES_, D_, OCC_) \
   launch_mid_variant<TN_, TM_, WAVES_, D_, OCC_, EPI>(xt, w, m, n, k, residual, out, ldo, qa, err, s)
-  if (v.tn == 4 && v.tm == 4) {
+  if (k >= kMidFarK) {
+    if constexpr (EPI == kMidEpiQkvRope) return hipErrorInvalidValue;
+    else launch_mid_variant<1, 1, 8, 12, 2, EPI, true>(xt, w, m, n, k, residual, out, ldo, qa, err, s);
+  } else if (v.tn == 4 && v.tm == 4) {
     FH_MID(4, 4, 4, 4, 1);
   } else if (v.tn == 4) {
     FH_MID(4, 2, 4, 4, 2);

@@ -198,6 +198,15 @@ def test_projections_that_256_x_128_blocks_fit_badly_take_others():
     assert block(3000, 24576, 4096, _lib.EPI_SWIGLU) == (256, 256)
 
 
+def test_projections_of_a_very_long_k_take_64_bit_addresses():
+    # From k = 2^24 on the operands of a block of 128 columns are beyond 32-bit byte offsets.
+    for epilogue in (_lib.EPI_BF16, _lib.EPI_RESIDUAL, _lib.EPI_SWIGLU, _lib.EPI_F32):
+        for n in (128, 384, 4096):
+            for m in (33, 200, 300, 2000):
+                for k in (1 << 24, (1 << 24) + 32, 1 << 27):
+                    assert block(m, n, k, epilogue) in ((32, 32), (256, 256)), (m, n, k, epilogue)
+
+
 def attention_form(runs, query_heads, kv_heads):
     v = ferric_amd.load().fh_prefill_attention_form(u32([p for p, _ in runs]), u32([n for _, n in runs]), len(runs),
                                                     query_heads, kv_heads)

@@ -335,6 +335,47 @@ def test_gemm_mid_sized_batches(m, n, k, epi):
         assert np.mean(got == ref) > 0.97
 
 
+# A k from which the operands of a block are beyond 32-bit byte offsets. Nonzero
+# columns at both ends and around 2^23 and 2^24; small whole numbers, so every
+# sum and its bf16 rounding are exact.
+@pytest.mark.parametrize("epi", ["f32", "bf16", "residual", "swiglu"])
+def test_gemm_of_a_very_long_k(epi):
+    m, n, k = 33, 128, (1 << 24) + 96
+    cols = np.array([0, 31, 32, 4099, (1 << 23) - 1, 1 << 23, (1 << 24) - 1, 1 << 24, (1 << 24) + 95])
+    idx = np.arange(len(cols))
+    xv = ((np.arange(m)[:, None] + idx) % 7 - 3).astype(np.float64)
+    wv = ((3 * np.arange(n)[:, None] + 2 * idx) % 5 - 2).astype(np.float64)
+    x = torch.zeros(tiled_rows(m) * k, dtype=torch.bfloat16, device="cuda")
+    w = torch.zeros(n * k, dtype=torch.bfloat16, device="cuda")
+    in_block = cols // 32, 16 * ((cols % 32) // 8), cols % 8  # k-block, lanes before, element
+
+    def scatter(t, tile, row, values):
+        at = (tile * 64 + row[:, None] % 16 + in_block[1]) * 8 + in_block[2]
+        t[torch.from_numpy(at.reshape(-1)).cuda()] = torch.from_numpy(values.reshape(-1)).to(torch.bfloat16).cuda()
+
+    rows, wide = np.arange(m), np.arange(n)
+    scatter(x, in_block[0] * (tiled_rows(m) // 16) + rows[:, None] // 16, rows, xv)
+    scatter(w, wide[:, None] // 16 * (k // 32) + in_block[0], wide, wv)
+    ref = xv @ wv.T
+    err = du.empty(1, np.uint32)
+    code = {"bf16": _lib.EPI_BF16, "f32": _lib.EPI_F32, "residual": _lib.EPI_RESIDUAL, "swiglu": _lib.EPI_SWIGLU}[epi]
+    ldo = n // 2 if epi == "swiglu" else n
+    out = torch.zeros(tiled_rows(m) * n, dtype=torch.float32 if epi == "f32" else torch.bfloat16, device="cuda")
+    res = torch.arange(m * n, device="cuda").remainder(16).to(torch.bfloat16)
+    _lib.check(LIB.fh_op_gemm(x.data_ptr(), w.data_ptr(), m, n, k, code, 1, res.data_ptr() if epi == "residual" else None,
+                              out.data_ptr(), ldo, du.ptr(err), du.stream()))
+    assert du.to_host(err, np.uint32)[0] == 0
+    if epi == "swiglu":
+        plain = du.empty(m * ldo, np.uint16)
+        _lib.check(LIB.fh_op_untile_activation(out.data_ptr(), du.ptr(plain), m, ldo, du.stream()))
+        pair = ref.astype(np.float32).reshape(m, n // 32, 2, 16)  # a gate tile, then its up tile
+        gate, up = (orc.f32_to_bf16(np.ascontiguousarray(pair[:, :, i]).reshape(-1)) for i in (0, 1))
+        assert du.bf16_ulp_diff(du.to_host(plain, np.uint16), orc.swiglu(gate, up)) <= 1  # exp's last ulp
+        return
+    got = out[: m * n].double().cpu().numpy().reshape(m, n)
+    assert np.array_equal(got, ref + res.double().cpu().numpy().reshape(m, n) if epi == "residual" else ref)
+
+
 # FP32 and SwiGLU of 33 to 256 rows, on both sides of the lines between the
 # weight stream (more than 128 slices of 128 columns, up to 224 rows) and the
 # blocks. Bounds as above.
