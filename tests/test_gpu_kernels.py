@@ -260,7 +260,7 @@ def test_gemm_residual_and_swiglu_epilogues(m):
         assert np.mean(got == ref) > 0.97
 
 
-@pytest.mark.parametrize("m", [3, 40, 300])  # decode kernel, 32-row chunks, 256 x 256 blocks
+@pytest.mark.parametrize("m", [3, 40, 300])  # decode kernel, 32 x 32 blocks
 def test_gemm_swiglu_epilogue_reports_nonfinite(m):
     # A NaN in one activation row makes that row's gate and up NaN: the fused
     # SwiGLU epilogue (decode and prefill kernels) raises the error word where
@@ -271,9 +271,7 @@ def test_gemm_swiglu_epilogue_reports_nonfinite(m):
 @pytest.mark.parametrize("m", [33, 130, 257])
 @pytest.mark.parametrize("n,k", [(128, 64), (256, 1024), (384, 4096)])
 def test_gemm_large_m_bf16_and_f32_epilogues(m, n, k):
-    # 33-256 rows: the panel kernel (FP32) and the decode kernel over row
-    # chunks (bf16); 257 rows: the compute-bound kernel (128 x 128 blocks,
-    # no split-K).
+    # Narrow weights at the smallest batch of blocks, one row past 128 and 256.
     got, ref = _gemm_case(m, n, k, _lib.EPI_F32, m * 5 + n)
     assert np.max(np.abs(got - ref)) <= F32_BOUND
     got, ref = _gemm_case(m, n, k, _lib.EPI_BF16, m * 5 + n + 1)
@@ -284,10 +282,8 @@ def test_gemm_large_m_bf16_and_f32_epilogues(m, n, k):
 @pytest.mark.parametrize("m,n,k,epi", [(160, 6144, 1024, "bf16"), (160, 6144, 1024, "f32"), (100, 24576, 256, "swiglu"),
                                        (70, 4096, 2048, "residual")])
 def test_gemm_wide_batches(m, n, k, epi):
-    # 33-256 rows: bf16 and residual outputs run the decode kernel over row
-    # chunks (64-row chunks, or 32-row ones where an 8-wave launch of 64-row
-    # chunks would need more than one round of the CUs: n = 6144 at 160
-    # rows); FP32 and the fused gate/up run the panel kernel.
+    # 33-256 rows of the models' weights: blocks, and the panel kernel for the
+    # wide fused gate/up.
     code = {"bf16": _lib.EPI_BF16, "f32": _lib.EPI_F32, "swiglu": _lib.EPI_SWIGLU, "residual": _lib.EPI_RESIDUAL}[epi]
     got, ref = _gemm_case(m, n, k, code, 31 * m + n + k)
     if epi == "f32":
@@ -308,22 +304,19 @@ def test_gemm_large_m_residual_and_swiglu_epilogues(m):
         assert np.mean(got == ref) > 0.97
 
 
-# The block shapes of mid-sized batches (32 tn weight rows x 32 tm activation
-# rows, waves splitting k) and the 256-row x 128-column blocks, at their edges:
-# fewer k-blocks than waves and k-blocks not a multiple of them, row blocks
-# with one valid row, waves whose rows are all padding, weights not a multiple
-# of 256 rows. Same bounds as the other epilogues above: FP32 reassociation
-# (F32_BOUND), one bf16 rounding of such a sum, SwiGLU of two of them.
+# Batches of some hundred rows, in whatever blocks the rule takes for them
+# (test_gemm_blocks below holds each block to its edges). Same bounds as the
+# other epilogues above: FP32 reassociation (F32_BOUND), one bf16 rounding of
+# such a sum, SwiGLU of two of them.
 @pytest.mark.parametrize("m,n,k,epi", [
-    (33, 128, 64, "bf16"), (33, 128, 32, "f32"),  # 4 x 4 tiles, 2 and 1 k-blocks for 4 waves
-    (777, 4096, 544, "residual"),                 # 4 x 4, 17 k-blocks, 9 rows in the last block
-    (600, 4096, 4096, "residual"), (450, 6144, 2048, "swiglu"), (640, 4096, 2048, "f32"),  # 4 x 4
-    (257, 6144, 4096, "bf16"), (513, 24576, 96, "swiglu"), (777, 4096, 1056, "f32"),       # 4 x 2
-    (289, 4096, 2048, "bf16"), (300, 4096, 4128, "f32"),                                   # 2 x 4
-    (65, 4096, 256, "residual"), (129, 2048, 1056, "bf16"), (300, 8192, 128, "swiglu"),    # 2 x 2
-    (257, 1024, 2048, "bf16"), (509, 1024, 3072, "residual"), (97, 1024, 96, "f32"),       # 1 x 2, 2 x 2
-    (40, 4096, 4096, "residual"), (48, 1024, 2080, "bf16"), (300, 384, 4096, "f32"),       # 1 x 1
-    (521, 8192, 2048, "residual"), (705, 6144, 4096, "bf16"), (600, 8192, 4096, "swiglu"), (513, 12800, 2080, "f32"),  # 256 x 128
+    (33, 128, 64, "bf16"), (33, 128, 32, "f32"), (777, 4096, 544, "residual"),
+    (600, 4096, 4096, "residual"), (450, 6144, 2048, "swiglu"), (640, 4096, 2048, "f32"),
+    (257, 6144, 4096, "bf16"), (513, 24576, 96, "swiglu"), (777, 4096, 1056, "f32"),
+    (289, 4096, 2048, "bf16"), (300, 4096, 4128, "f32"),
+    (65, 4096, 256, "residual"), (129, 2048, 1056, "bf16"), (300, 8192, 128, "swiglu"),
+    (257, 1024, 2048, "bf16"), (509, 1024, 3072, "residual"), (97, 1024, 96, "f32"),
+    (40, 4096, 4096, "residual"), (48, 1024, 2080, "bf16"), (300, 384, 4096, "f32"),
+    (521, 8192, 2048, "residual"), (705, 6144, 4096, "bf16"), (600, 8192, 4096, "swiglu"), (513, 12800, 2080, "f32"),
 ])
 def test_gemm_mid_sized_batches(m, n, k, epi):
     code = {"bf16": _lib.EPI_BF16, "f32": _lib.EPI_F32, "swiglu": _lib.EPI_SWIGLU, "residual": _lib.EPI_RESIDUAL}[epi]
@@ -333,6 +326,35 @@ def test_gemm_mid_sized_batches(m, n, k, epi):
     else:
         assert du.bf16_close(got, ref, ulps=3 if epi == "swiglu" else 1)
         assert np.mean(got == ref) > 0.97
+
+
+# Every block (rows x columns) with every epilogue, at its edges: one k-block,
+# fewer than the waves that split k and not a multiple of them or of the rings'
+# slots, last row blocks of one or a few valid rows, waves whose rows are all
+# padding. The block is asked of the rule, so that a change of its estimates
+# cannot leave one without a test. Bounds as above.
+@pytest.mark.parametrize("rows,cols,m,n,k,epi", [
+    (32, 32, 33, 128, 32, "bf16"), (32, 32, 640, 384, 4128, "f32"), (32, 32, 129, 2560, 96, "residual"),
+    (32, 32, 65, 128, 32, "swiglu"),
+    (64, 32, 33, 8192, 1056, "bf16"), (64, 32, 97, 2560, 128, "f32"), (64, 32, 509, 1024, 4128, "residual"),
+    (64, 32, 48, 6144, 1024, "swiglu"),
+    (64, 64, 1030, 2560, 2080, "bf16"), (64, 64, 65, 6144, 32, "f32"), (64, 64, 1345, 384, 1056, "residual"),
+    (64, 64, 600, 4096, 224, "swiglu"),
+    (64, 128, 160, 6144, 2080, "bf16"), (64, 128, 257, 6144, 32, "f32"), (64, 128, 509, 4096, 1056, "residual"),
+    (64, 128, 513, 2560, 2080, "swiglu"),
+    (128, 64, 65, 12800, 2080, "bf16"), (128, 64, 777, 2048, 4128, "f32"), (128, 64, 900, 1152, 2048, "residual"),
+    (128, 64, 513, 2048, 4096, "swiglu"),
+    (128, 128, 333, 6144, 2080, "bf16"), (128, 128, 640, 6144, 2080, "f32"), (128, 128, 777, 2560, 4128, "residual"),
+    (128, 128, 333, 6144, 2080, "swiglu"),
+    (256, 128, 513, 8192, 32, "bf16"), (256, 128, 705, 8192, 544, "f32"), (256, 128, 521, 8192, 1056, "residual"),
+    (256, 128, 450, 12800, 2080, "swiglu"),
+    (256, 256, 321, 22016, 2080, "bf16"), (256, 256, 385, 22784, 2080, "f32"), (256, 256, 513, 17920, 2080, "residual"),
+    (256, 256, 321, 24576, 1056, "swiglu"), (256, 256, 385, 23296, 32, "swiglu"),
+])
+def test_gemm_blocks(rows, cols, m, n, k, epi):
+    code = {"bf16": _lib.EPI_BF16, "f32": _lib.EPI_F32, "residual": _lib.EPI_RESIDUAL, "swiglu": _lib.EPI_SWIGLU}[epi]
+    assert LIB.fh_gemm_block(m, n, k, code, 0) == rows << 16 | cols
+    test_gemm_mid_sized_batches(m, n, k, epi)
 
 
 # A k from which the operands of a block are beyond 32-bit byte offsets. Nonzero
@@ -625,7 +647,7 @@ def test_sqrt_rn_is_correctly_rounded_for_every_normal_float():
     assert proc.returncode == 0 and "failures 0" in proc.stdout, proc.stdout + proc.stderr
 
 
-# rows = 260: bf16 rows beyond 256 take the lane-per-(row, head) kernel;
+# rows = 260: more than 4096 (row, head)s of bf16 rows take the kernel of many rows;
 # rows = 160 with 5 splits: the wide batches' 256-row partial slabs.
 @pytest.mark.parametrize("qh,kvh,splits,rows", [(32, 8, 0, 9), (16, 8, 0, 9), (32, 8, 1, 9), (32, 8, 3, 9),
                                                 (32, 8, 0, 260), (32, 8, 5, 160)])

@@ -730,21 +730,34 @@ def test_prefill_chunk_of_at_most_32_rows():
 
 def test_prefill_chunk_8b_fused_qkv_epilogue():
     # 8B layer geometry, one layer, 292 rows: above 256 rows the QKV
-    # projection runs the 256 x 256-block kernel with QK-norm, RoPE and the KV
-    # append in its epilogue (32 query + 16 key/value heads, 24 column blocks).
+    # projection runs with QK-norm, RoPE and the KV append in its epilogue (32
+    # query + 16 key/value heads; 64 x 128 blocks).
     cfg = dict(ferric_amd.QWEN3_8B, layers=1)
     limits = PagedLimits(context_tokens=4096, physical_page_count=320, page_table_stride=256)
     _prefill_case(cfg, limits, [150, 140], [100, 3000], 512, 43, "prefill 8b fused qkv")
 
 
-@pytest.mark.parametrize("prompts", [[270, 160], [300, 221, 200], [257], [264]])
-def test_prefill_chunk_8b_fused_qkv_epilogue_of_mid_sized_blocks(prompts):
+@pytest.mark.parametrize("prompts,block", [([270, 160], (128, 128)), ([300, 221, 200], (256, 128)),
+                                           ([257], (64, 128)), ([264], (64, 128))])
+def test_prefill_chunk_8b_fused_qkv_epilogue_of_mid_sized_blocks(prompts, block):
     # 8B layer geometry, one layer: at 431 rows the QKV projection runs 128 x
     # 128 blocks (one head each, the last with 47 valid rows), at 722 rows the
     # 256-row ones, with QK-norm, RoPE and the KV append in their epilogues.
+    assert ferric_amd.load().fh_gemm_block(sum(prompts) + 1, 6144, 4096, 0, 1) == block[0] << 16 | block[1]
     cfg = dict(ferric_amd.QWEN3_8B, layers=1, vocabulary=4096)
     limits = PagedLimits(context_tokens=2048, physical_page_count=200, page_table_stride=128)
     _prefill_case(cfg, limits, prompts, [900], 768, 47, "prefill 8b mid-sized blocks")
+
+
+@pytest.mark.parametrize("rows", [1217, 1281])
+def test_prefill_chunk_fused_qkv_epilogue_of_256_x_256_blocks(rows):
+    # 32 query and 16 KV heads: 32 column blocks of two heads each, the last row
+    # block with one valid row, in its fourth wave (1217) or its first (1281).
+    cfg = dict(ferric_amd.QWEN3_0_6B, layers=1, hidden=512, query_heads=32, kv_heads=16, intermediate=512,
+               vocabulary=4096)
+    assert ferric_amd.load().fh_gemm_block(rows, 8192, 512, 0, 1) == 256 << 16 | 256
+    limits = PagedLimits(context_tokens=2048, physical_page_count=200, page_table_stride=128)
+    _prefill_case(cfg, limits, [700, rows - 701], [90], 1536, 49, f"prefill 256 x 256 blocks {rows}")
 
 
 def test_prefill_qknorm_inside_block_attention_is_bit_identical():
@@ -915,9 +928,9 @@ def test_prefill_ignores_unwritten_slots_of_the_last_page():
         pair.close()
 
 
-# Chunks of more than 256 rows: the attention of long blocks. Query heads per
-# KV head 1, 2, 4 and 8, and the three splits of the 4 waves over vectors and
-# keys (32-, 64- and 128-vector blocks as the chunk grows); prompts whose
+# Chunks of more than 256 rows: the attention of long blocks, with 1, 2, 4 and 8
+# query heads per KV head (the splits of the 4 waves over vectors and keys are
+# the next test's); prompts whose
 # lengths leave blocks of one row, pages and key tiles partly filled, decode
 # rows at context lengths around tile and page-table-chunk edges beside them,
 # and rows interleaved by sequence (one-row blocks).
@@ -949,6 +962,28 @@ def test_prefill_attention_of_long_blocks(qh, kvh, prompts, decode, interleave):
         pair.check_kv()
     finally:
         pair.close()
+
+
+# Each split of the 4 waves over vectors and keys (form 1, 2 and 4: blocks of
+# 128, 64 and 32 vectors) with 1, 2, 4 and 8 query heads per KV head, over
+# several key tiles, beside decode rows at context lengths around tile edges.
+# The form is asked of the rule.
+@pytest.mark.parametrize("qh,kvh,form,prompts,decode", [
+    (32, 32, 1, [150, 129, 161, 128, 147], [63, 64, 65, 127, 129]),
+    (32, 16, 1, [150, 129, 161, 128, 147, 150], [63, 64, 65, 127, 129]),
+    (32, 8, 1, [150, 129, 161, 128, 147, 150], [63, 64, 65, 127, 129]),
+    (32, 4, 1, [150, 129, 161, 128, 147, 150, 155, 157], [63, 64, 65, 127, 129]),
+    (8, 8, 2, [150, 167], [63, 64, 65, 127, 129]), (16, 8, 2, [150, 167], [63, 64, 65, 127, 129]),
+    (32, 8, 2, [150, 167], [63, 64, 65, 127, 129]), (32, 4, 2, [150, 167], [63, 64, 65, 127, 129]),
+    (8, 8, 4, [513], []), (16, 8, 4, [513], []), (8, 2, 4, [401], [63, 127, 128, 129, 1025]),
+    (16, 2, 4, [401], [63, 127, 128, 129, 1025]),
+])
+def test_prefill_attention_forms(qh, kvh, form, prompts, decode):
+    runs = [(0, n) for n in prompts] + [(p, 1) for p in decode]
+    got = ferric_amd.load().fh_prefill_attention_form(*[(ctypes.c_uint32 * len(runs))(*v) for v in zip(*runs)],
+                                                      len(runs), qh, kvh)
+    assert got == (128 // form // (qh // kvh)) << 16 | form
+    test_prefill_attention_of_long_blocks(qh, kvh, prompts, decode, False)
 
 
 # Chunks of more than 256 rows made of many short runs of rows: the short blocks
@@ -1170,7 +1205,7 @@ def _golden_row_spread(case_name="qwen3-8b-b32"):
 
 def test_prefill_8b_full_depth_two_prompts_match_oracle():
     # The prefill path at full depth: Qwen3-8B, all 36 layers, two 160-token
-    # prompts as one 320-row chunk (above 256 rows: the 256 x 256-block
+    # prompts as one 320-row chunk (above 256 rows: block
     # projections with QK-norm, RoPE and the KV append in the QKV epilogue,
     # and the block attention), every bar of the module docstring applied,
     # then one decode step on the prefilled cache.
