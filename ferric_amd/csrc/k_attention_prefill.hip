@@ -35,7 +35,7 @@
 // exponentials, the split of P), two waves per SIMD: the matrix cores are 57 %
 // busy at the 1.8 GHz the power limit leaves. us per layer, 16-row blocks with
 // 16-key tiles (k_attention_block.hip) -> this kernel: one 8000-token 8B prompt
-// 2010 -> 775, 32 prompts of 256 tokens 94 -> 64, one of 777 tokens 42 -> 23
+// 2010 -> 711, 32 prompts of 256 tokens 94 -> 63, one of 777 tokens 42 -> 22
 // (29 without the waves along the keys), a 509-token 0.6B prompt 21 -> 13 (18).
 #include <cmath>
 #include <type_traits>
@@ -356,10 +356,10 @@ struct PrefillForm {
   uint32_t form, tile, slots;
   float launch_us, chain_us, group_us, tile_us, round_us;
 };
-constexpr PrefillForm kPrefillForms[] = {{0, 64, 0, 9.0f, 0.f, 0.f, 1.75f, 0.f},
-                                         {1, 64, 512, 8.5f, 1.8f, 0.58f, 1.38f, 2.28f},
-                                         {2, 64, 512, 8.1f, 1.16f, 1.71f, 0.87f, 1.49f},
-                                         {4, 128, 256, 9.6f, 1.56f, 3.36f, 1.74f, 1.84f}};
+constexpr PrefillForm kPrefillForms[] = {{0, 64, 0, 8.97f, 0.f, 0.f, 1.75f, 0.f},
+                                         {1, 64, 512, 8.53f, 1.8f, 0.58f, 1.38f, 2.28f},
+                                         {2, 64, 512, 8.06f, 1.16f, 1.71f, 0.87f, 1.49f},
+                                         {4, 128, 256, 9.63f, 1.56f, 3.36f, 1.74f, 1.84f}};
 
 }  // namespace
 

@@ -285,12 +285,17 @@ LargeKernel pick_kernel(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, b
 // weight through the panel kernel: where its 128-column slices fill more than
 // half of the CUs, up to 224 rows. Fewer slices leave too many CUs idle, and
 // with more rows the panel's LDS traffic exceeds its weight stream. Panel
-// against the blocks (us, cold weights): 152 slices (19456 x 2560) 64 rows 24
-// / 26, 160 rows 35 / 38; 128 slices (16384 x 4096) 40 rows 33 / 29, 160 rows
-// 48 / 43; 48 slices (6144 x 1024) 48 rows 10.8 / 7.5, 160 rows 17.6 / 9.5; 32
-// slices (4096 x 4096) 30 / 12.5, 44 / 18.7; 192 slices (24576 x 4096) 200
-// rows 67 / 71, 240 rows 75 / 69; 1187 slices (151936 x 4096) 160 rows 283 /
-// 317, 240 rows 400 / 357.
+// against the fastest block (us, cold weights): 152 slices (19456 x 2560) 64 rows
+// 25 / 27, 160 rows 36 / 39; 128 slices (16384 x 4096) 40 rows 33 / 29, 160 rows
+// 48 / 43; 48 slices (6144 x 1024) 48 rows 10.8 / 6.5, 160 rows 17.6 / 9.5; 32
+// slices (4096 x 4096) 30 / 12.5, 44 / 18.7; 192 slices (24576 x 4096) 64 rows
+// 37 / 42, 160 rows 53 / 63, 224 rows 69 / 71, 240 rows 75 / 69; 1187 slices
+// (151936 x 4096) 64 rows 230 / 250, 160 rows 284 / 313, 240 rows 400 / 357. The
+// line is not the faster side everywhere: the panel's time steps at 97 and 161
+// rows (gate/up at 100 to 128 rows 56 / 53, the head of 4096 at 192 to 224 rows
+// 334 / 315 to 384 / 356), and a head of 1024 columns is up to 9 % faster in
+// blocks below 65 rows (48 rows 70 / 66) and up to 21 % above 160 (208 rows 131 /
+// 108). Both sides ran the panel before the blocks.
 bool panel_streams(uint32_t m, uint32_t n) { return m <= 224 && n > 128 * kPanelCols; }
 
 }  // namespace

@@ -13,15 +13,17 @@
 // reassociation of the serial order, as in the other projection kernels,
 // fixed by the launch shape.
 //
-// What bounds it: the operands, read from L2 (64 (TN + TM) KiB per k-block of
-// 32 and workgroup / 32): about 14.6 TB/s over all CUs on every block shape,
-// with and without the MFMAs and at 3 to 7 stages in flight, so the largest
-// block that still fills the CUs is the fastest (launch_gemm_mid picks it).
+// What bounds it: the operands, read from L2 (2 (TN + TM) KiB per k-block and
+// workgroup). Launches of 512 and more blocks on the models' weights read them
+// at 15 to 17 TB/s over all CUs in the median of each shape (128 x 128 blocks:
+// 11.6, with 8 us of reduction and epilogue), 24 at most, with and without the
+// MFMAs and at 3 to 7 stages in flight. So large blocks read less and small ones
+// fill the CUs; gemm_mid_cost weighs the two.
 // Measured against the 256 x 256-block kernel (us per launch, cold weights):
-//   777 rows: O 4096 x 4096 87 -> 39, down 4096 x 12288 225 -> 98, QKV 6144 x 4096 88 -> 63
-//   509 rows: O 1024 x 2048 47 -> 7.2, down 1024 x 3072 64 -> 9.5, gate/up 6144 x 1024 35 -> 12
-//   300 rows: O 4096 x 4096 85 -> 25
-//   48 rows: down 4096 x 12288 55 (the weight-streaming kernel over row chunks) -> 32
+//   777 rows: O 4096 x 4096 87 -> 38, down 4096 x 12288 225 -> 101
+//   512 rows: O 1024 x 2048 48 -> 7.4, down 1024 x 3072 64 -> 10.0, gate/up 6144 x 1024 30 -> 12.2
+//   288 rows: O 4096 x 4096 87 -> 28
+//   48 rows: down 4096 x 12288 56 (the weight-streaming kernel over row chunks) -> 32
 //
 // A 32x32x16 operand (lane l: row l % 32, columns 8 (l / 32) .. + 7) is half
 // a k-block of two adjacent 16-row tiles: in-tile lanes l % 16 + 16 (l / 32)
@@ -289,7 +291,7 @@ constexpr float kMidSwigluUs = 0.43f, kMidQkvUs = 0.47f;
 // rate, plus the shape's overheads; and no less than the launch takes at a k
 // of a few k-blocks. Its constants and those of the other two kernels'
 // estimates (gemm_band_cost, block_cost) are fitted together to the times of
-// every form at 3221 launches: 33 to 8192 rows of the Qwen3 projections, their
+// every form at 3261 launches: 33 to 8192 rows of the Qwen3 projections, their
 // fused QKV form, other wide weights and weights of 128 to 512 columns at k of
 // 1024 to 12288, and 128 to 16512 columns at k of 32 to 768, with all
 // epilogues. The estimate picks a form that is slower than the fastest by (mean,
@@ -299,7 +301,7 @@ constexpr float kMidSwigluUs = 0.43f, kMidQkvUs = 0.47f;
 // than 3 % slower than the 256 x 256 blocks alone. (Constants fitted to 296
 // launches of the Qwen3 projections only gave 1.9, 2.1, 2.7 and 4.4 % on
 // average; every k of up to 128 took 128 x 128 blocks: 96 x 128 x 64 5.9 us,
-// now 3.3, 4.7 with the weight stream before these blocks.)
+// now 2.9, 4.8 with the weight stream before these blocks.)
 float mid_cost(const MidShape& s, uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, bool fused_qkv) {
   const float rounds = (float)(n / (32 * s.tn)) * ((m + 32 * s.tm - 1) / (32 * s.tm)) / 256.f;
   const float block_kb = 2.048f * (s.tn + s.tm) * (k / 32);  // operand kilobytes of a block

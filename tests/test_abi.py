@@ -230,6 +230,39 @@ def test_prefill_attention_form_follows_the_runs_of_a_chunk():
     assert attention_form([(0, 300)], 24, 8) == attention_form([(0, 300)], 32, 0) == (0, 0)  # heads not supported
 
 
+def measured(name):
+    """Rows of a table of measured times, without its comment and heading lines."""
+    with open(ROOT / "profiles" / name) as f:
+        return [line.rstrip("\n").split(",") for line in f.readlines()[2:]]
+
+
+def test_projection_estimates_against_the_times_they_are_fitted_to():
+    blocks = [(128, 128), (64, 128), (128, 64), (64, 64), (64, 32), (32, 32), (256, 128), (256, 256)]
+    codes = {"bf16": 0, "residual": 1, "swiglu": 2, "f32": 3, "qkv": 0}
+    worse, against_256 = [], []
+    for m, n, k, epilogue, *us in measured("projection_blocks_us.csv"):
+        taken = block(int(m), int(n), int(k), codes[epilogue], epilogue == "qkv")
+        if taken == (0, 0):
+            continue  # the weight stream
+        times = dict(zip(blocks, (float(t) if t else np.inf for t in us)))
+        worse.append(times[taken] / min(times.values()))
+        if int(k) >= 1024:
+            against_256.append(times[taken] / times[256, 256])
+    assert len(worse) > 3000 and np.mean(worse) <= 1.011 and max(worse) <= 1.7
+    assert max(against_256) <= 1.03
+
+
+def test_prefill_attention_estimates_against_the_times_they_are_fitted_to():
+    worse, against_short = [], []
+    for heads, kv, runs, *us in measured("prefill_attention_forms_us.csv"):
+        rows = [r.replace("@", "x").split("x") for r in runs.split(" ")]
+        _, form = attention_form([(int(p), int(n)) for c, n, p in rows for _ in range(int(c))], int(heads), int(kv))
+        times = dict(zip((0, 1, 2, 4), map(float, us)))
+        worse.append(times[form] / min(times.values()))
+        against_short.append(times[form] / times[0])
+    assert len(worse) == 840 and np.mean(worse) <= 1.005 and max(worse) <= 1.21 and max(against_short) <= 1.15
+
+
 def test_ops_reject_bad_shapes_before_any_launch():
     lib = ferric_amd.load()
     p = ctypes.c_void_p(16)  # never dereferenced: validation fails first
