@@ -343,20 +343,23 @@ bool band_ok(uint32_t m, uint32_t n, uint32_t k) {
 
 // Estimated microseconds of a launch (fitted with mid_cost, k_gemm_mid.hip):
 // rounds of the 256 CUs in units of a full block, at least one; a last block of
-// at most 64 rows takes two thirds of one, a longer one a quarter per 64 rows.
+// at most 64 rows takes 0.59 of one, a longer one a quarter per 64 rows.
 // Blocks that outnumber the CUs' rounds with less than their work leave some CU
 // a full block and a last one: 600 x 12288 x 2048 SwiGLU is 288 blocks with the
 // work of 240, 54 us (50 in 256 x 256 blocks), not the 37 of one round.
 float gemm_band_cost(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, bool fused_qkv) {
   if (!band_ok(m, n, k)) return -1.f;
   const uint32_t tail = m % kLargeBlockRows;
-  const float part = tail == 0 ? 0.f : tail <= 64 ? 0.66f : (tail + 63) / 64 * 0.25f;
+  const float part = tail == 0 ? 0.f : tail <= 64 ? 0.59f : (tail + 63) / 64 * 0.25f;
   const float bands = (float)(n / kBandCols);
   float rounds = ceilf(bands * (m / kLargeBlockRows + part) / 256.f);
   if (bands * ((m + kLargeBlockRows - 1) / kLargeBlockRows) > 256.f * rounds) rounds += part;
-  const float around =
-      fused_qkv ? 7.03f : epilogue == FH_EPI_SWIGLU ? 5.84f : epilogue == FH_EPI_RESIDUAL ? 2.01f : 1.3f;
-  return 4.55f + rounds * (around + (k / 32) * 0.412f);
+  const float around = fused_qkv                       ? 6.66f
+                       : epilogue == FH_EPI_SWIGLU   ? 3.47f
+                       : epilogue == FH_EPI_RESIDUAL ? 1.91f
+                       : epilogue == FH_EPI_F32      ? 1.6f
+                                                     : 1.79f;
+  return 4.86f + rounds * (around + (k / 32) * 0.41f);
 }
 
 hipError_t launch_gemm_band(const uint16_t* x_tiled, const uint16_t* w_tiled, uint32_t m, uint32_t n, uint32_t k,

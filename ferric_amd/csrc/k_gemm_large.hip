@@ -264,9 +264,9 @@ __global__ __launch_bounds__(512) void gemm_large_xd_kernel(const uint16_t* __re
 // longer the more CUs run, and what a block costs around its k loop.
 float block_cost(uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, bool fused_qkv) {
   const uint32_t blocks = n / (16 * kBigTiles) * ((m + 255) / 256);
-  const float kb_us = blocks < 100 ? 0.514f : blocks < 256 ? 0.703f : 0.689f;
+  const float kb_us = blocks < 100 ? 0.477f : blocks < 256 ? 0.607f : 0.688f;
   const float around =
-      fused_qkv ? 12.93f : epilogue == FH_EPI_SWIGLU ? 13.97f : epilogue == FH_EPI_RESIDUAL ? 16.37f : 13.52f;
+      fused_qkv ? 11.86f : epilogue == FH_EPI_SWIGLU ? 10.83f : epilogue == FH_EPI_RESIDUAL ? 25.58f : 15.26f;
   return ((blocks + 255) / 256) * (around + (k / 32) * kb_us);
 }
 

@@ -279,15 +279,15 @@ struct MidShape {
   uint32_t tn, tm;
   float cu_gbs, launch_us, round_us, least_us, least_round_us;
 };
-constexpr MidShape kMidShapes[] = {{4, 4, 69.0f, 0.66f, 10.82f, 8.11f, 0.01f}, {4, 2, 73.0f, 3.59f, 0.46f, 2.20f, 1.92f},
-                                    {2, 4, 77.3f, 3.32f, 1.55f, 4.84f, 0.67f}, {2, 2, 75.2f, 2.21f, 0.04f, 2.95f, 0.76f},
-                                    {1, 2, 65.0f, 2.07f, 0.39f, 2.70f, 0.62f}, {1, 1, 66.8f, 2.19f, 0.34f, 1.61f, 0.85f}};
+constexpr MidShape kMidShapes[] = {{4, 4, 69.0f, 0.55f, 6.84f, 11.22f, 3.58f}, {4, 2, 73.1f, 1.92f, 0.62f, 6.69f, 1.91f},
+                                    {2, 4, 83.1f, 2.59f, 1.45f, 4.82f, 1.09f}, {2, 2, 75.9f, 1.47f, 0.02f, 4.00f, 0.80f},
+                                    {1, 2, 83.1f, 2.45f, 0.26f, 3.72f, 0.64f}, {1, 1, 64.0f, 3.08f, 0.19f, 2.94f, 0.84f}};
 // Microseconds that the SwiGLU and the QK-norm epilogues take longer, per 256
 // blocks of 4 32 x 32 outputs.
-constexpr float kMidSwigluUs = 0.43f, kMidQkvUs = 0.47f;
+constexpr float kMidSwigluUs = 0.14f, kMidQkvUs = 0.40f;
 
 // Estimated microseconds of one launch: the operand bytes of all blocks at
-// 17.8 TB/s, but no less than those of the blocks one CU runs at its own
+// 18.2 TB/s, but no less than those of the blocks one CU runs at its own
 // rate, plus the shape's overheads; and no less than the launch takes at a k
 // of a few k-blocks. Its constants and those of the other two kernels'
 // estimates (gemm_band_cost, block_cost) are fitted together to the times of
@@ -295,17 +295,19 @@ constexpr float kMidSwigluUs = 0.43f, kMidQkvUs = 0.47f;
 // fused QKV form, other wide weights and weights of 128 to 512 columns at k of
 // 1024 to 12288, and 128 to 16512 columns at k of 32 to 768, with all
 // epilogues. The estimate picks a form that is slower than the fastest by (mean,
-// most): Qwen3 projections 0.7 %, 17 %; fused QKV 0.8 %, 21 %; other wide weights
-// 0.5 %, 15 %; narrow weights 2.5 %, 69 % (2048 x 256 x 12288 58 us, 34.5 possible);
-// k up to 768 0.9 %, 37 % (3000 x 16512 x 32). At the first three it is never more
-// than 3 % slower than the 256 x 256 blocks alone. (Constants fitted to 296
-// launches of the Qwen3 projections only gave 1.9, 2.1, 2.7 and 4.4 % on
-// average; every k of up to 128 took 128 x 128 blocks: 96 x 128 x 64 5.9 us,
-// now 2.9, 4.8 with the weight stream before these blocks.)
+// most): Qwen3 projections 1.8 %, 25 % (64 x 4096 x 1024 6.0 us, 4.8 possible); fused
+// QKV 0.8 %, 21 %; other wide weights 1.9 %, 27 %; narrow weights 3.9 %, 69 % (2048 x
+// 256 x 12288 58 us, 34.5 possible); k up to 768 3.6 %, 55 %. At k of 1024 and more
+// it is never more than 3 % slower than the 256 x 256 blocks alone. (Constants
+// fitted to 296 launches of the Qwen3 projections only, without the least time
+// and the epilogues' own, took 128 x 128 blocks for every k of up to 128: 96 x
+// 128 x 64 5.9 us, now 2.9, 4.8 with the weight stream before these blocks. Where
+// their choice was no slower than before these blocks, the fit keeps it for the
+// Qwen3 projections of up to 256 rows.)
 float mid_cost(const MidShape& s, uint32_t m, uint32_t n, uint32_t k, uint32_t epilogue, bool fused_qkv) {
   const float rounds = (float)(n / (32 * s.tn)) * ((m + 32 * s.tm - 1) / (32 * s.tm)) / 256.f;
   const float block_kb = 2.048f * (s.tn + s.tm) * (k / 32);  // operand kilobytes of a block
-  const float all = rounds * 256.f * block_kb / 17800.f;
+  const float all = rounds * 256.f * block_kb / 18200.f;
   const float cu = ceilf(rounds) * block_kb / s.cu_gbs;
   const float more = (fused_qkv ? kMidQkvUs : epilogue == FH_EPI_SWIGLU ? kMidSwigluUs : 0.f) * (s.tn * s.tm / 4.f);
   return fmaxf(s.least_us + rounds * (s.least_round_us + more),

@@ -248,7 +248,7 @@ def test_projection_estimates_against_the_times_they_are_fitted_to():
         worse.append(times[taken] / min(times.values()))
         if int(k) >= 1024:
             against_256.append(times[taken] / times[256, 256])
-    assert len(worse) > 3000 and np.mean(worse) <= 1.011 and max(worse) <= 1.7
+    assert len(worse) > 3000 and np.mean(worse) <= 1.033 and max(worse) <= 1.7
     assert max(against_256) <= 1.03
 
 

@@ -336,19 +336,19 @@ def test_gemm_mid_sized_batches(m, n, k, epi):
 @pytest.mark.parametrize("rows,cols,m,n,k,epi", [
     (32, 32, 33, 128, 32, "bf16"), (32, 32, 640, 384, 4128, "f32"), (32, 32, 129, 2560, 96, "residual"),
     (32, 32, 65, 128, 32, "swiglu"),
-    (64, 32, 33, 8192, 1056, "bf16"), (64, 32, 97, 2560, 128, "f32"), (64, 32, 509, 1024, 4128, "residual"),
-    (64, 32, 48, 6144, 1024, "swiglu"),
-    (64, 64, 1030, 2560, 2080, "bf16"), (64, 64, 65, 6144, 32, "f32"), (64, 64, 1345, 384, 1056, "residual"),
+    (64, 32, 65, 128, 1056, "bf16"), (64, 32, 129, 128, 512, "f32"), (64, 32, 509, 1024, 4128, "residual"),
+    (64, 32, 40, 128, 1056, "swiglu"),
+    (64, 64, 129, 4096, 2080, "bf16"), (64, 64, 65, 6144, 32, "f32"), (64, 64, 1345, 384, 1056, "residual"),
     (64, 64, 600, 4096, 224, "swiglu"),
-    (64, 128, 160, 6144, 2080, "bf16"), (64, 128, 257, 6144, 32, "f32"), (64, 128, 509, 4096, 1056, "residual"),
+    (64, 128, 160, 6144, 2080, "bf16"), (64, 128, 129, 6144, 1056, "f32"), (64, 128, 509, 4096, 1056, "residual"),
     (64, 128, 513, 2560, 2080, "swiglu"),
-    (128, 64, 65, 12800, 2080, "bf16"), (128, 64, 777, 2048, 4128, "f32"), (128, 64, 900, 1152, 2048, "residual"),
+    (128, 64, 777, 1280, 2080, "bf16"), (128, 64, 777, 2048, 4128, "f32"), (128, 64, 900, 1152, 2048, "residual"),
     (128, 64, 513, 2048, 4096, "swiglu"),
     (128, 128, 333, 6144, 2080, "bf16"), (128, 128, 640, 6144, 2080, "f32"), (128, 128, 777, 2560, 4128, "residual"),
     (128, 128, 333, 6144, 2080, "swiglu"),
-    (256, 128, 513, 8192, 32, "bf16"), (256, 128, 705, 8192, 544, "f32"), (256, 128, 521, 8192, 1056, "residual"),
+    (256, 128, 513, 8192, 32, "bf16"), (256, 128, 777, 6144, 1056, "f32"), (256, 128, 333, 16128, 1056, "residual"),
     (256, 128, 450, 12800, 2080, "swiglu"),
-    (256, 256, 321, 22016, 2080, "bf16"), (256, 256, 385, 22784, 2080, "f32"), (256, 256, 513, 17920, 2080, "residual"),
+    (256, 256, 321, 22016, 2080, "bf16"), (256, 256, 385, 22784, 2080, "f32"), (256, 256, 513, 14592, 4128, "residual"),
     (256, 256, 321, 24576, 1056, "swiglu"), (256, 256, 385, 23296, 32, "swiglu"),
 ])
 def test_gemm_blocks(rows, cols, m, n, k, epi):
