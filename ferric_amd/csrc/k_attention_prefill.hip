@@ -356,21 +356,22 @@ struct PrefillForm {
   uint32_t form, tile, slots;
   float launch_us, chain_us, group_us, tile_us, round_us;
 };
-constexpr PrefillForm kPrefillForms[] = {{0, 64, 0, 8.97f, 0.f, 0.f, 1.75f, 0.f},
-                                         {1, 64, 512, 8.53f, 1.8f, 0.58f, 1.38f, 2.28f},
-                                         {2, 64, 512, 8.06f, 1.16f, 1.71f, 0.87f, 1.49f},
-                                         {4, 128, 256, 9.63f, 1.56f, 3.36f, 1.74f, 1.84f}};
+constexpr PrefillForm kPrefillForms[] = {{0, 64, 0, 9.05f, 0.f, 0.f, 1.76f, 0.f},
+                                         {1, 64, 512, 8.35f, 1.82f, 0.67f, 1.43f, 2.59f},
+                                         {2, 64, 512, 8.24f, 1.24f, 1.91f, 0.87f, 1.62f},
+                                         {4, 128, 256, 9.29f, 1.74f, 4.42f, 1.56f, 1.96f}};
 
 }  // namespace
 
 // The form with the lowest estimate: the longest workgroup's chain, the work
 // of all of them, or rounds of average ones, whichever is longest. Its
-// constants are fitted to the times of all forms over 840 chunks of 257 to
-// 8000 rows (1 to 2000 sequences of 1 to 4000 rows at contexts of 0 to 7000
+// constants are fitted to the times of all forms over 1368 chunks of 257 to
+// 8000 rows (1 to 2000 sequences of 1 to 5000 rows at contexts of 0 to 7000
 // tokens, alone and mixed; 1, 2, 4 and 8 query heads per KV head): it picks a
-// form 0.4 % slower than the fastest on average, 21 % at most, and never one
-// more than 15 % slower than the short blocks. Waves along the keys by the
-// chunk's rows alone, as before, were 28 % slower than the fastest on average:
+// form 0.4 % slower than the fastest on average, 17 % at most (32 sequences of
+// 24 rows on 3000 tokens, 84 us in short blocks, 99 taken), and never one more
+// than 7 % slower than waves along the keys by the chunk's rows alone, as
+// before. Those were 22 % slower than the fastest on average:
 // a chunk of many short runs got long blocks that held a row or two. us per
 // layer by the rows alone / now / short blocks: 0.6B 300 sequences of 1 row 67 /
 // 14 / 14, 8B 300 x 1 68 / 17 / 17, 20 x 16 rows on 7000 tokens 288 / 198 / 191,
@@ -393,7 +394,7 @@ uint32_t attention_prefill_form(const uint32_t* position, const uint32_t* rows, 
       }
     const float n = (float)(groups * kvh), all = (float)(tiles * kvh), average = all / n;
     // Short blocks: 4, 2 or 1 page phases (launch_attention_blocks).
-    const float chain = f.form ? f.chain_us : n <= 256.f ? 1.6f : n <= 512.f ? 2.74f : 3.6f;
+    const float chain = f.form ? f.chain_us : n <= 256.f ? 1.62f : n <= 512.f ? 2.81f : 3.69f;
     float us = fmaxf(chain * longest, (f.group_us * n + f.tile_us * all) / 256.f);
     if (f.slots) us = fmaxf(us, average * (chain + (ceilf(n / f.slots) - 1.f) * f.round_us));
     us += f.launch_us;

@@ -260,7 +260,7 @@ def test_prefill_attention_estimates_against_the_times_they_are_fitted_to():
         times = dict(zip((0, 1, 2, 4), map(float, us)))
         worse.append(times[form] / min(times.values()))
         against_short.append(times[form] / times[0])
-    assert len(worse) == 840 and np.mean(worse) <= 1.005 and max(worse) <= 1.21 and max(against_short) <= 1.15
+    assert len(worse) == 1368 and np.mean(worse) <= 1.005 and max(worse) <= 1.18 and max(against_short) <= 1.18
 
 
 def test_ops_reject_bad_shapes_before_any_launch():
