@@ -35,7 +35,7 @@
 // exponentials, the split of P), two waves per SIMD: the matrix cores are 57 %
 // busy at the 1.8 GHz the power limit leaves. us per layer, 16-row blocks with
 // 16-key tiles (k_attention_block.hip) -> this kernel: one 8000-token 8B prompt
-// 2010 -> 711, 32 prompts of 256 tokens 94 -> 63, one of 777 tokens 42 -> 22
+// 2010 -> 689, 32 prompts of 256 tokens 94 -> 63, one of 777 tokens 42 -> 22
 // (29 without the waves along the keys), a 509-token 0.6B prompt 21 -> 13 (18).
 #include <cmath>
 #include <type_traits>
